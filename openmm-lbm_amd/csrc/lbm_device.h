@@ -333,14 +333,102 @@ __device__ __forceinline__ uint4x philox(uint32_t c0, uint32_t c1, uint32_t c2, 
  * (r cos 2 pi u2, r sin 2 pi u2).  The angle needs no more than 16 bits, so three Philox blocks
  * (12 words: 8 radii, 4 words of two angles each) give 16 normals.
  */
+/*
+ * The FP64 functions of the transform, for its own arguments only (the general ones of the math library also reduce
+ * any angle and handle every special value, and made the FP64 pass issue-bound).  256^3 FP64 with fluctuations: the
+ * fused pass 1.328 -> 0.950 ms (0.936 ms without noise); 128^3 170.7 -> 120.8 us.
+ */
+
+/* 1/d for a normal d: the hardware's estimate and two Newton steps. */
+__device__ __forceinline__ double reciprocalF64(double d) {
+    double r = __builtin_amdgcn_rcp(d);
+    r = fma(fma(-d, r, 1.0), r, r);
+    return fma(fma(-d, r, 1.0), r, r);
+}
+
+/* sqrt(x) for x = 0 or a normal x: the hardware's 1/sqrt(x), refined with g -> sqrt(x) and h -> 1/(2 sqrt(x)) together
+   (Goldschmidt's iteration), then one correction by the residual x - g^2. */
+__device__ __forceinline__ double sqrtF64(double x) {
+    double y = __builtin_amdgcn_rsq(x);
+    double g = x*y, h = 0.5*y;
+    double r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    g = fma(fma(-g, g, x), h, g);
+    return x == 0.0 ? 0.0 : g;
+}
+
+/*
+ * -ln(n 2^-32) for a whole number n in [1, 2^32].  n 2^-32 = m 2^e with m in [sqrt(1/2), sqrt(2)), f = m - 1 (exact) and
+ * s = f/(2 + f): ln m = 2 atanh(s) = f - s (f - R), R = 2 (s^2/3 + s^4/5 + ...); |s| < 0.172, so the terms to s^20 leave
+ * 2e-18.  ln 2 is split into a part of 32 bits, whose product with e is exact, and the rest.
+ */
+__device__ __forceinline__ double minusLog32(double n) {
+    double m = __builtin_amdgcn_frexp_mant(n);              // [1/2, 1)
+    int e = __builtin_amdgcn_frexp_exp(n) - 32;
+    const bool low = m < 0.70710678118654752;
+    m = low ? m + m : m;
+    const double k = (double) (low ? e - 1 : e);
+    const double f = m - 1.0, d = m + 1.0;
+    const double inv = reciprocalF64(d);
+    double s = f*inv;
+    s = fma(fma(-s, d, f), inv, s);
+    const double z = s*s;
+    double R = 2.0/21.0;
+    R = fma(R, z, 2.0/19.0);
+    R = fma(R, z, 2.0/17.0);
+    R = fma(R, z, 2.0/15.0);
+    R = fma(R, z, 2.0/13.0);
+    R = fma(R, z, 2.0/11.0);
+    R = fma(R, z, 2.0/9.0);
+    R = fma(R, z, 2.0/7.0);
+    R = fma(R, z, 2.0/5.0);
+    R = fma(R, z, 2.0/3.0);
+    R *= z;
+    constexpr double LN2_HI = 2977044471.0/4294967296.0;    // ln 2 rounded to 2^-32
+    constexpr double LN2_LO = 1.9082149292705877e-10;
+    return -fma(k, LN2_HI, f - fma(s, f - R, -k*LN2_LO));
+}
+
+/* cos and sin of 2 pi b 2^-16: the whole number b gives the quadrant and the rest x, |x| <= pi/4, exactly, and the
+   Taylor series to x^18 and x^17 leave 3e-20. */
+__device__ __forceinline__ void cosSinTurn16(uint32_t b, double& c, double& s) {
+    const uint32_t quadrant = (b + 8192u) >> 14;
+    const double x = (double) ((int) b - (int) (quadrant << 14))*9.5873799242852576857e-05;      // 2 pi 2^-16
+    const double z = x*x;
+    double p = -1.0/6402373705728000.0;
+    p = fma(p, z, 1.0/20922789888000.0);
+    p = fma(p, z, -1.0/87178291200.0);
+    p = fma(p, z, 1.0/479001600.0);
+    p = fma(p, z, -1.0/3628800.0);
+    p = fma(p, z, 1.0/40320.0);
+    p = fma(p, z, -1.0/720.0);
+    p = fma(p, z, 1.0/24.0);
+    p = fma(p, z, -0.5);
+    const double cx = fma(p, z, 1.0);
+    double q = 1.0/355687428096000.0;
+    q = fma(q, z, -1.0/1307674368000.0);
+    q = fma(q, z, 1.0/6227020800.0);
+    q = fma(q, z, -1.0/39916800.0);
+    q = fma(q, z, 1.0/362880.0);
+    q = fma(q, z, -1.0/5040.0);
+    q = fma(q, z, 1.0/120.0);
+    q = fma(q, z, -1.0/6.0);
+    const double sx = fma(q*z, x, x);
+    c = (quadrant & 1u) ? sx : cx;
+    s = (quadrant & 1u) ? cx : sx;
+    c = ((quadrant + 1u) & 2u) ? -c : c;
+    s = (quadrant & 2u) ? -s : s;
+}
+
 template <typename R>
 __device__ __forceinline__ void boxMullerPair(uint32_t a, uint32_t b, R* out) {
     if constexpr (std::is_same<R, double>::value) {
-        const double twoPi = 6.283185307179586476925287;
-        double r = sqrt(-2.0*log(((double) a + 1.0)*2.3283064365386963e-10));
-        double angle = twoPi*((double) b*1.52587890625e-05);
-        out[0] = r*cos(angle);
-        out[1] = r*sin(angle);
+        const double r = sqrtF64(2.0*minusLog32((double) a + 1.0));
+        double c, s;
+        cosSinTurn16(b, c, s);
+        out[0] = r*c;
+        out[1] = r*s;
     }
     else {
         // Hardware transcendentals: v_log_f32 is log2 (so -2 ln u1 = -2 ln 2 log2 u1), v_sin_f32/v_cos_f32
