@@ -130,6 +130,7 @@ struct lbm_context {
     double wallOverrideValue[3] = {0, 0, 0};
     // Particles.
     int numParticles = 0, numSystem = 0, numSlots = 0;
+    bool identityParticles = false;       // coupled particle i is particle i of the System, and all are coupled
     bool dense = false;                   // denseCoupling(): index order, component-plane reactions
     bool wide = false;                    // 64-bit element indices in the fused pass (populations above 4 GiB)
     bool coupleXcd = true;                // LBM_AMD_COUPLE_XCD: the coupling's particles in XCD-contiguous runs
@@ -475,11 +476,15 @@ void advanceFluid(lbm_context* c, const double* dPos, const double* dVel, const 
     }
 }
 
-void beginStepDevice(lbm_context* c, int64_t step, const double* dPos, double* dVel) {
+void beginState(lbm_context* c, int64_t step) {
     c->stepIndex = step;
     c->stepPending = true;
     c->wallStepDone = false;
     c->wallOverride = false;
+}
+
+void beginStepDevice(lbm_context* c, int64_t step, const double* dPos, double* dVel) {
+    beginState(c, step);
     if (c->mask != nullptr && c->numParticles > 0) {
         // The reflection also clears the step's other wall partial sums.
         ParticleArgs a = particleArgs(c, step, true);
@@ -655,6 +660,9 @@ void create(const lbm_params* params, const int* solid, int numSolid, const int*
                 throw Error(LBM_ERROR_INVALID, "LBMForce: a coupled particle index is out of range");
             m[i] = masses[i]/c->cellMass();
         }
+        c->identityParticles = numParts == numSys;
+        for (int i = 0; i < numParts && c->identityParticles; i++)
+            c->identityParticles = parts[i] == i;
         c->particles = deviceAlloc<int>(numParts);
         c->mass = deviceAlloc<double>(numParts);
         upload(c->particles, c->hostParticles, c->stream);
@@ -800,6 +808,26 @@ int fail(const Error& e) {
 }
 
 }  // namespace
+
+bool lbm_internal_reflection(lbm_context* c, int64_t step, int n, StepReflection& out) {
+    out = StepReflection();
+    if (c->mask != nullptr && c->numParticles > 0) {
+        if (!c->identityParticles || c->numParticles != n)
+            return false;
+        out.args = particleArgs(c, step, true);
+        out.mass = c->mass;
+        out.mask = c->mask;
+        out.partials = c->wallPartials;
+        out.count = c->wallPartialCount;
+        out.ownOffset = c->wallReflectOffset;
+        return true;
+    }
+    return c->wallPartialCount == 0;
+}
+
+void lbm_internal_begin_reflected(lbm_context* c, int64_t step) {
+    beginState(c, step);
+}
 
 #define LBM_TRY(...) \
     try { __VA_ARGS__; g_lastError.clear(); return LBM_OK; } \

@@ -279,6 +279,18 @@ void centredCouple(CentredState* state, int storage, const void* src, const uint
         const double* ucm, const ParticleArgs& a, const double g[3], double* particleForce,
         unsigned long long* reactionFixed, uint32_t* touched, double* partials, hipStream_t stream);
 
+/*
+ * The reflection at solid nodes that begins a step, for a caller that runs it in a kernel of its own (the device-resident
+ * particle host merges it with its integrator).
+ */
+struct StepReflection {
+    ParticleArgs args;
+    const double* mass = nullptr;
+    const uint32_t* mask = nullptr;
+    double* partials = nullptr;     // the step's wall partial sums: the kernel clears those outside its own slots
+    int count = 0, ownOffset = 0;
+};
+
 /* Nodes per axis of an interpolation stencil (LBMStencils.h:42-104). */
 __host__ __device__ inline int stencilWidth(int stencil) {
     switch (stencil) {
@@ -290,3 +302,11 @@ __host__ __device__ inline int stencilWidth(int stencil) {
 }
 
 }  // namespace lbm
+
+/*
+ * For the particle host (lbm_harness.hip).  lbm_internal_reflection: whether lbm_begin_step_device(step) does nothing on
+ * the device but the reflection, of the coupled particles 0 .. n - 1 in their order, or nothing at all (out.mask null);
+ * lbm_internal_begin_reflected then stands in for it, once the caller's kernel is on the stream.
+ */
+bool lbm_internal_reflection(lbm_context* c, int64_t step, int n, lbm::StepReflection& out);
+void lbm_internal_begin_reflected(lbm_context* c, int64_t step);

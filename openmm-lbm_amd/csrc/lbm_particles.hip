@@ -30,48 +30,17 @@ __global__ void __launch_bounds__(BLOCK) reflectParticles(const double* __restri
         const int* __restrict__ particles, const double* __restrict__ mass, const uint32_t* __restrict__ mask,
         ParticleArgs a, double* __restrict__ allPartials, int count, int ownOffset) {
     double* partials = allPartials + 3*(size_t) ownOffset;
-    for (int j = blockIdx.x*BLOCK + threadIdx.x; j < 3*count; j += gridDim.x*BLOCK)
-        if (j < 3*ownOffset || j >= 3*(ownOffset + (int) gridDim.x))
-            allPartials[j] = 0.0;
+    clearOtherPartials(allPartials, count, ownOffset);
     double acc[3] = {0, 0, 0};
     int i = blockIdx.x*BLOCK + threadIdx.x;
     if (i < a.numParticles) {
         int part = particles[i];
         const double* x = positions + 3*(size_t) part;
         double* v = velocities + 3*(size_t) part;
-        int size[3] = {(int) a.g.nx, (int) a.g.ny, (int) a.g.nz};
-        int near[3], idx[3][2];
-        double wt[3][2];
-        for (int k = 0; k < 3; k++) {
-            double s = wrapCoordinate(x[k], a.dx, size[k]);
-            near[k] = nearestIndex(s, size[k]);
-            double lower = floor(s);
-            idx[k][0] = ((int) lower) % size[k];
-            idx[k][1] = (idx[k][0] + 1) % size[k];
-            wt[k][1] = s - lower;
-            wt[k][0] = 1.0 - wt[k][1];
-        }
-        uint32_t nearNode = (uint32_t) (near[0] + (int) a.g.nx*(near[1] + (int) a.g.ny*near[2]));
-        if (isSolid(mask, nearNode)) {
-            double solid[2][2][2];
-            for (int p = 0; p < 2; p++)
-                for (int q = 0; q < 2; q++)
-                    for (int r = 0; r < 2; r++)
-                        solid[p][q][r] = isSolid(mask, (uint32_t) (idx[0][p] + (int) a.g.nx*(idx[1][q] + (int) a.g.ny*idx[2][r]))) ? 1.0 : 0.0;
-            double n[3] = {0, 0, 0};
-            for (int p = 0; p < 2; p++)
-                for (int q = 0; q < 2; q++) {
-                    n[0] += wt[1][p]*wt[2][q]*(solid[1][p][q] - solid[0][p][q]);
-                    n[1] += wt[0][p]*wt[2][q]*(solid[p][1][q] - solid[p][0][q]);
-                    n[2] += wt[0][p]*wt[1][q]*(solid[p][q][1] - solid[p][q][0]);
-                }
-            if (v[0]*n[0] + v[1]*n[1] + v[2]*n[2] > 0) {
-                for (int k = 0; k < 3; k++) {
-                    acc[k] = v[k]*(2.0*mass[i]*a.cellMass);
-                    v[k] = -v[k];
-                }
-            }
-        }
+        double vi[3] = {v[0], v[1], v[2]};
+        if (reflectParticle(x, vi, mass[i], mask, a, acc))
+            for (int k = 0; k < 3; k++)
+                v[k] = vi[k];
     }
     storeWallPartial<BLOCK>(acc, partials);
 }

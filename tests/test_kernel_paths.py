@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 from lbm_amd import LBMForce
+from lbm_amd.harness import DeviceParticles
 import oracle_lib
 from parity import Setup
 
@@ -28,3 +29,37 @@ def test_fp64_normals_match_the_oracle(seed):
     a, b = gpu.getFluidState(), ref.getFluidState()
     assert np.abs(b).max() > 0
     assert np.abs(a - b).max() <= 1e-14*np.abs(b).max()
+
+
+@pytest.mark.parametrize("beads,walls,bonds", [(1, True, False), (256, True, True), (257, True, True), (300, False, True)])
+def test_merged_launch_between_steps_is_bit_identical(beads, walls, bonds):
+    """Twelve steps in one call (update, reflection and other forces of the steps between in one launch) against twelve
+    calls of one step (a launch each); beads beside the walls, so that some are reflected."""
+    rng = np.random.default_rng(beads)
+    s = Setup((16, 12, 20), tau=0.7)
+    s.add_particles(rng.uniform([0, 0, 0.2], [16, 12, 18.8], size=(beads, 3)), velocities=rng.normal(scale=3.0, size=(beads, 3)))
+
+    def conf(f):
+        if walls:
+            f.setSolidNodes([i for k in (0, 19) for i in range(k*192, (k + 1)*192)])
+            f.setWallScheme(LBMForce.BounceBack)
+        f.setFriction(10.0)
+        f.setTemperature(300.0)
+        f.setFluidFluctuations(True)
+        f.setRandomNumberSeed(9)
+        f.setInterpolationStencil(LBMForce.Trilinear)
+    s.configure.append(conf)
+    results = []
+    for calls, steps in ((1, 12), (12, 1)):
+        ctx = s.build()
+        dp = DeviceParticles(ctx)
+        if bonds:
+            dp.setBonds(np.stack([np.arange(beads - 1), np.arange(1, beads)], axis=1), 100.0, 0.5)
+        for _ in range(calls):
+            dp.step(steps)
+        pos, vel = dp.pull()
+        results.append((pos, vel, ctx.getFluidState(), ctx.getWallForce()))
+    for a, b in zip(*results):
+        assert np.array_equal(a, b)
+    if walls and beads > 1:
+        assert np.abs(results[0][3]).max() > 0
