@@ -270,8 +270,7 @@ void createBatch(lbm_batch* b, int R, const lbm_params* params, const int* numPa
         d.step.step = 0;
         d.step.mu = 3.0*p.fluid_kT*p.dt*p.dt/(cellMass*p.dx*p.dx);
         d.step.roundSeed = 0;
-        int w = stencilWidth(p.interpolation_stencil);
-        d.step.reactionPlanes = denseCoupling((uint64_t) numParticles[r], w*w*w, (uint64_t) g.n) ? 1 : 0;
+        d.step.reactionPlanes = 0;         // the coupling's staged atomics want a node's accumulators side by side
         ParticleArgs& a = d.part;
         a.g = g;
         a.numParticles = numParticles[r];

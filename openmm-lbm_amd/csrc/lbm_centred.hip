@@ -210,6 +210,7 @@ struct CgArgs {
     double* partials;        // [RED_BLOCKS][8]
     double* scalars;
     int slots;               // w^3
+    const int* order;        // the particles in processing order (their slots are kept in that order), or nullptr
     // Sparse particles (split = 1): a product spreads only the slots at nodes that several slots share (spreadsAt); a
     // slot alone at its node contributes (w/rho) w x of its own particle directly.  seen/shared: node bits set by
     // cgMarkShared and cleared by cgForces.
@@ -223,18 +224,34 @@ __device__ __forceinline__ bool spreadsAt(const CgArgs& c, uint32_t node) {
     return !c.split || ((c.shared[node >> 5] >> (node & 31)) & 1u);
 }
 
+/*
+ * The work-group's place in the processing order: each XCD takes a contiguous run of the particles, sorted by node, so
+ * that the node sums that neighbouring stencils share are read through one L2.  For dense particles only (56,320 Keys
+ * particles in 120^3: a gather 58.6 -> 39.1 us; 20,000 in 256^3 share few nodes and keep the index order).
+ */
+__device__ __forceinline__ uint32_t placeOf(const CgArgs& c) {
+    return c.order != nullptr ? xcdContiguousTile(blockIdx.x, gridDim.x) : blockIdx.x;
+}
+
+/* The particle at place `rank` of the processing order. */
+__device__ __forceinline__ int particleAt(const CgArgs& c, int rank) {
+    return c.order != nullptr ? c.order[rank] : rank;
+}
+
 /* One group of LANES lanes per particle, one lane per stencil slot: the slot's node, weight and w/rho, the particle's
    right-hand side, diagonal and F = rhs/diagonal. */
 template <typename S, int LANES>
 __global__ void __launch_bounds__(BLOCK) cgSetup(const S* __restrict__ src, const uint32_t* __restrict__ mask,
         const double* __restrict__ positions, const double* __restrict__ velocities,
         const double* __restrict__ otherForces, const int* __restrict__ particles, const double* __restrict__ mass,
-        const double* __restrict__ ucm, ParticleArgs a, double gx, double gy, double gz, CgArgs c) {
+        const double* __restrict__ ucm, ParticleArgs a, double gx, double gy, double gz, CgArgs c,
+        const double4* __restrict__ field) {
     constexpr int GROUPS = BLOCK/LANES;
     const double h = 0.5, aa = a.gamma*h;
     int lane = threadIdx.x % LANES;
-    int i = blockIdx.x*GROUPS + threadIdx.x/LANES;
-    bool active = i < a.numParticles;
+    const int rank = (int) placeOf(c)*GROUPS + threadIdx.x/LANES;
+    bool active = rank < a.numParticles;
+    const int i = active ? particleAt(c, rank) : 0;
     int part = active ? particles[i] : 0;
     const double* x = positions + 3*(size_t) part;
     // The stencil of the lanes (groupStencil): each lane evaluates its own slot's kernel weight per axis.
@@ -257,8 +274,16 @@ __global__ void __launch_bounds__(BLOCK) cgSetup(const S* __restrict__ src, cons
         bool solid = solidAt(mask, node);
         double winv = 0.0;
         if (!solid) {
-            double j[3];
-            double rho = nodeMoments(src, a.g, node, ucm, a.removal, j);
+            double j[3], rho;
+            if (field != nullptr) {
+                const double4 m = field[node];
+                j[0] = m.x;
+                j[1] = m.y;
+                j[2] = m.z;
+                rho = m.w;
+            }
+            else
+                rho = nodeMoments(src, a.g, node, ucm, a.removal, j);
             if (rho > 0) {
                 ux = (j[0] + h*(rho*gx))*(weight/rho);
                 uy = (j[1] + h*(rho*gy))*(weight/rho);
@@ -267,19 +292,16 @@ __global__ void __launch_bounds__(BLOCK) cgSetup(const S* __restrict__ src, cons
                 winv = weight/rho;
             }
         }
-        size_t sl = (size_t) i*c.slots + lane;
+        size_t sl = (size_t) rank*c.slots + lane;
         c.slotNode[sl] = node;
         c.slotW[sl] = weight;
         c.slotWInvRho[sl] = winv;
         c.slotSolid[sl] = solid ? 1 : 0;
     }
-#pragma unroll
-    for (int off = 1; off < LANES; off <<= 1) {
-        ux += __shfl_xor(ux, off, LANES);
-        uy += __shfl_xor(uy, off, LANES);
-        uz += __shfl_xor(uz, off, LANES);
-        self += __shfl_xor(self, off, LANES);
-    }
+    ux = groupSum<LANES>(ux);
+    uy = groupSum<LANES>(uy);
+    uz = groupSum<LANES>(uz);
+    self = groupSum<LANES>(self);
     if (active && lane == 0) {
         double m = mass[i];
         double known[3], random[3];
@@ -361,10 +383,13 @@ __device__ __forceinline__ void combinePartials(const double* __restrict__ parti
         }
 }
 
-/* spread[node] += w x (fixed point), one thread per particle slot.  The fixed-point scale, 2^(52 - e) with
+/* spread[node] += w x (fixed point), one thread per particle slot and component: consecutive lanes add to consecutive
+   words, 12 for a Keys row, so a wavefront's atomics, which run at the memory side and are bound by the requests, reach it
+   as a third of those that three strided adds per slot made (56,320 Keys particles in 120^3: 255 -> 105 us).  The fixed-point scale, 2^(52 - e) with
    2^e >= max |x| (1 if x is zero), is formed by the first wavefront of every work-group from the largest |x| of the
    blocks in c.partials (one fixed combination, so every work-group has the same value); work-group 0 keeps it and its
    inverse in the scalars for the gather.  The solve's first product (first = 1) records which slots spread. */
+template <int SLOTS>
 __global__ void __launch_bounds__(BLOCK) cgSpread(const double* __restrict__ x, int n, CgArgs c,
         const double* done, int first) {
     if (done != nullptr && *done != 0.0)
@@ -383,27 +408,28 @@ __global__ void __launch_bounds__(BLOCK) cgSpread(const double* __restrict__ x, 
         }
     }
     __syncthreads();
-    size_t t = (size_t) blockIdx.x*BLOCK + threadIdx.x;
-    if (t >= (size_t) n*c.slots)
+    const uint64_t item = (uint64_t) placeOf(c)*BLOCK + threadIdx.x;
+    const uint64_t t = item/3;
+    const int k = (int) (item - 3*t);
+    const uint64_t rank = t/SLOTS;
+    if (rank >= (uint64_t) n)
         return;
     double w = c.slotW[t];
     uint32_t node = c.slotNode[t];
     bool spreads;
     if (first) {
         spreads = w != 0.0 && spreadsAt(c, node);
-        c.slotSpreads[t] = spreads ? 1 : 0;
+        if (k == 0)
+            c.slotSpreads[t] = spreads ? 1 : 0;
     }
     else
         spreads = c.slotSpreads[t] != 0;
     if (!spreads)
         return;
-    size_t i = t/c.slots;
-    const double scale = sharedScale;
-    for (int k = 0; k < 3; k++) {
-        long long v = llrint(w*x[3*i + k]*scale);
-        if (v != 0)
-            atomicAdd(c.spread + 3*(size_t) node + k, (unsigned long long) v);
-    }
+    const size_t i = (size_t) particleAt(c, (int) rank);
+    long long v = llrint(w*x[3*i + k]*sharedScale);
+    if (v != 0)
+        atomicAdd(c.spread + 3*(size_t) node + k, (unsigned long long) v);
 }
 
 /* Ax = x (1 + a)/m + a sum_slots (w/rho) spread[node], one group of LANES lanes per particle. */
@@ -414,11 +440,12 @@ __global__ void __launch_bounds__(BLOCK) cgGather(const double* __restrict__ x, 
         return;
     constexpr int GROUPS = BLOCK/LANES;
     int lane = threadIdx.x % LANES;
-    int i = blockIdx.x*GROUPS + threadIdx.x/LANES;
-    bool active = i < n;
+    const int rank = (int) placeOf(c)*GROUPS + threadIdx.x/LANES;
+    bool active = rank < n;
+    const int i = active ? particleAt(c, rank) : 0;
     double s[3] = {0, 0, 0};
     if (active && lane < c.slots) {
-        size_t sl = (size_t) i*c.slots + lane;
+        size_t sl = (size_t) rank*c.slots + lane;
         double winv = c.slotWInvRho[sl];
         const bool spreads = c.slotSpreads[sl] != 0;
         const uint32_t node = c.slotNode[sl];
@@ -440,10 +467,8 @@ __global__ void __launch_bounds__(BLOCK) cgGather(const double* __restrict__ x, 
             }
         }
     }
-#pragma unroll
-    for (int off = 1; off < LANES; off <<= 1)
-        for (int k = 0; k < 3; k++)
-            s[k] += __shfl_xor(s[k], off, LANES);
+    for (int k = 0; k < 3; k++)
+        s[k] = groupSum<LANES>(s[k]);
     if (active && lane == 0)
         for (int k = 0; k < 3; k++)
             Ax[3*(size_t) i + k] = x[3*(size_t) i + k]*((1.0 + aa)/mass[i]) + s[k]*aa;
@@ -602,17 +627,20 @@ __global__ void __launch_bounds__(BLOCK) cgForces(int n, ParticleArgs a, CgArgs 
         unsigned long long* __restrict__ reactionFixed, uint32_t* __restrict__ touched, double* __restrict__ partials) {
     constexpr int GROUPS = BLOCK/LANES;
     int lane = threadIdx.x % LANES;
-    int i = blockIdx.x*GROUPS + threadIdx.x/LANES;
+    const int rank = (int) placeOf(c)*GROUPS + threadIdx.x/LANES;
     double wallAcc[3] = {0, 0, 0};
     uint32_t node = 0;
     bool flagged = false;
-    if (i < n) {
+    __shared__ StagedReactions<BLOCK> staged;
+    staged.clear();
+    if (rank < n) {
+        const int i = particleAt(c, rank);
         double F[3] = {c.F[3*(size_t) i], c.F[3*(size_t) i + 1], c.F[3*(size_t) i + 2]};
         if (lane == 0)
             for (int k = 0; k < 3; k++)
                 particleForce[3*(size_t) i + k] = F[k]*a.forceScale;
         if (a.isStep && lane < c.slots) {
-            size_t sl = (size_t) i*c.slots + lane;
+            size_t sl = (size_t) rank*c.slots + lane;
             double w = c.slotW[sl];
             node = c.slotNode[sl];
             if (w != 0.0) {
@@ -621,14 +649,17 @@ __global__ void __launch_bounds__(BLOCK) cgForces(int n, ParticleArgs a, CgArgs 
                 // With the split, a fluid slot that spreads nothing is alone at its node: a store, not an atomic.
                 if (c.split && !solid && c.slotSpreads[sl] == 0 && c.slotWInvRho[sl] != 0.0)
                     flagged = storeReaction(node, r, a, reactionFixed);
+                else if (solid)
+                    for (int k = 0; k < 3; k++)
+                        wallAcc[k] = r[k];               // lattice momentum; the host converts the wall partials
                 else
-                    flagged = addReaction(node, solid, r, a, reactionFixed, wallAcc);
+                    flagged = staged.put(node, r, a);
             }
         }
         // Both arrays of node sums and the node bits of the split, cleared for the next solve (every word that a
         // spread or cgMarkShared set belongs to one of these slots; nothing reads them after the solve).
         if (lane < c.slots) {
-            size_t sl = (size_t) i*c.slots + lane;
+            size_t sl = (size_t) rank*c.slots + lane;
             uint32_t at = c.slotNode[sl];
             if (c.slotSpreads[sl] != 0)
                 for (int k = 0; k < 3; k++) {
@@ -642,6 +673,8 @@ __global__ void __launch_bounds__(BLOCK) cgForces(int n, ParticleArgs a, CgArgs 
         }
     }
     // The slots of a particle are its lanes, x fastest, as in the explicit coupling: one OR per run of a row's lanes.
+    if (a.isStep)
+        staged.add(a, reactionFixed);
     if (a.isStep)
         markTouched<LANES == 64 ? 4 : LANES == 32 ? 3 : 2>(touched, node, flagged, lane);
     blockPartials(wallAcc, partials);
@@ -773,8 +806,12 @@ void multiply(CentredState* st, const double* x, double* Ax, const double* mass,
     c.spread = st->sums[sums];
     c.spreadOther = st->sums[1 - sums];
     int n = st->n;
-    size_t slotItems = (size_t) n*c.slots;
-    cgSpread<<<blocksOf(slotItems, BLOCK), BLOCK, 0, stream>>>(x, n, c, done, first ? 1 : 0);
+    const unsigned spreadGroups = blocksOf(3*(size_t) n*c.slots, BLOCK);
+    switch (st->lanes) {
+    case 8: cgSpread<8><<<spreadGroups, BLOCK, 0, stream>>>(x, n, c, done, first ? 1 : 0); break;
+    case 32: cgSpread<27><<<spreadGroups, BLOCK, 0, stream>>>(x, n, c, done, first ? 1 : 0); break;
+    default: cgSpread<64><<<spreadGroups, BLOCK, 0, stream>>>(x, n, c, done, first ? 1 : 0); break;
+    }
     switch (st->lanes) {
     case 8: cgGather<8><<<blocksOf(n, BLOCK/8), BLOCK, 0, stream>>>(x, Ax, mass, n, aa, c, done); break;
     case 32: cgGather<32><<<blocksOf(n, BLOCK/32), BLOCK, 0, stream>>>(x, Ax, mass, n, aa, c, done); break;
@@ -792,7 +829,7 @@ bool converged(CentredState* st, hipStream_t stream) {
 template <typename S>
 void centredCoupleT(CentredState* st, const S* src, const uint32_t* mask, const double* positions,
         const double* velocities, const double* otherForces, const int* particles, const double* mass,
-        const double* ucm, const ParticleArgs& a, const double g[3], double* particleForce,
+        const double* ucm, const ParticleArgs& a, const double g[3], const double4* field, const int* order, double* particleForce,
         unsigned long long* reactionFixed, uint32_t* touched, double* partials, hipStream_t stream) {
     int n = a.numParticles;
     if (n == 0)
@@ -808,20 +845,21 @@ void centredCoupleT(CentredState* st, const S* src, const uint32_t* mask, const 
         return;
     }
     CgArgs& c = st->cg;
+    c.order = order;
     double aa = 0.5*a.gamma;
     unsigned groups = blocksOf(n, BLOCK/st->lanes);
     switch (st->lanes) {
     case 8:
         cgSetup<S, 8><<<groups, BLOCK, 0, stream>>>(src, mask, positions, velocities, otherForces, particles, mass, ucm, a,
-                g[0], g[1], g[2], c);
+                g[0], g[1], g[2], c, field);
         break;
     case 32:
         cgSetup<S, 32><<<groups, BLOCK, 0, stream>>>(src, mask, positions, velocities, otherForces, particles, mass, ucm, a,
-                g[0], g[1], g[2], c);
+                g[0], g[1], g[2], c, field);
         break;
     default:
         cgSetup<S, 64><<<groups, BLOCK, 0, stream>>>(src, mask, positions, velocities, otherForces, particles, mass, ucm, a,
-                g[0], g[1], g[2], c);
+                g[0], g[1], g[2], c, field);
         break;
     }
     if (c.split)
@@ -882,24 +920,24 @@ void centredCoupleT(CentredState* st, const S* src, const uint32_t* mask, const 
 
 void centredCouple(CentredState* st, int storage, const void* src, const uint32_t* mask, const double* positions,
         const double* velocities, const double* otherForces, const int* particles, const double* mass,
-        const double* ucm, const ParticleArgs& a, const double g[3], double* particleForce,
+        const double* ucm, const ParticleArgs& a, const double g[3], const double4* field, const int* order, double* particleForce,
         unsigned long long* reactionFixed, uint32_t* touched, double* partials, hipStream_t stream) {
     switch (storage) {
     case LBM_STORAGE_FP16:
         centredCoupleT<__half>(st, (const __half*) src, mask, positions, velocities, otherForces, particles, mass, ucm, a,
-                g, particleForce, reactionFixed, touched, partials, stream);
+                g, field, order, particleForce, reactionFixed, touched, partials, stream);
         break;
     case LBM_STORAGE_BF16:
         centredCoupleT<__hip_bfloat16>(st, (const __hip_bfloat16*) src, mask, positions, velocities, otherForces,
-                particles, mass, ucm, a, g, particleForce, reactionFixed, touched, partials, stream);
+                particles, mass, ucm, a, g, field, order, particleForce, reactionFixed, touched, partials, stream);
         break;
     case LBM_STORAGE_FP64:
         centredCoupleT<double>(st, (const double*) src, mask, positions, velocities, otherForces, particles, mass, ucm, a,
-                g, particleForce, reactionFixed, touched, partials, stream);
+                g, field, order, particleForce, reactionFixed, touched, partials, stream);
         break;
     default:
         centredCoupleT<float>(st, (const float*) src, mask, positions, velocities, otherForces, particles, mass, ucm, a,
-                g, particleForce, reactionFixed, touched, partials, stream);
+                g, field, order, particleForce, reactionFixed, touched, partials, stream);
         break;
     }
 }

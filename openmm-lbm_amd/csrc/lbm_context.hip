@@ -308,7 +308,7 @@ StepArgs stepArgs(lbm_context* c, int64_t step) {
     a.step = step;
     a.mu = 3.0*c->p.fluid_kT*c->p.dt*c->p.dt/(c->cellMass()*c->p.dx*c->p.dx);
     a.roundSeed = (uint32_t) (c->seed*0x9E3779B9u) ^ (uint32_t) (step*0x85EBCA6Bll) ^ (uint32_t) ((uint64_t) step >> 32);
-    a.reactionPlanes = c->dense ? 1 : 0;
+    a.reactionPlanes = c->binned ? 1 : 0;
     return a;
 }
 
@@ -330,7 +330,7 @@ ParticleArgs particleArgs(lbm_context* c, int64_t step, bool isStep) {
     a.seed = c->seed;
     a.step = step;
     a.hasSolids = c->mask != nullptr;
-    a.reactionPlanes = c->dense ? 1 : 0;
+    a.reactionPlanes = c->binned ? 1 : 0;
     a.xcdOrder = c->coupleXcd ? 1 : 0;
     a.overflow = c->overflow;
     return a;
@@ -346,10 +346,21 @@ void couple(lbm_context* c, const double* dPos, const double* dVel, const double
     if (a.removal)
         reduceMoments(c);
     double* partials = isStep && c->mask != nullptr ? c->wallPartials + 3*(size_t) c->wallCoupleOffset : nullptr;
+    const int* order = nullptr;
+    try {
+        if (c->order != nullptr && c->closure == nullptr)
+            order = coupleOrderAt(c->order, step, dPos, c->particles, a, c->stream);
+    }
+    catch (const std::runtime_error& e) {
+        throw Error(LBM_ERROR_RUNTIME, e.what());
+    }
     if (c->centred != nullptr) {
         // Centred drag: the other forces (dForces, before the coupling adds to them) enter the particle velocities.
+        if (c->momentField != nullptr)
+            launchMomentField(c->p.storage, c->popA, c->mask, a, c->ucm, c->momentField, dPos, c->particles, nullptr,
+                    c->stream);
         centredCouple(c->centred, c->p.storage, c->popA, c->mask, dPos, dVel, dForces, c->particles, c->mass, c->ucm, a,
-                c->p.body_acceleration, c->particleForce, c->reactionFixed, c->touched, partials, c->stream);
+                c->p.body_acceleration, c->momentField, order, c->particleForce, c->reactionFixed, c->touched, partials, c->stream);
         return;
     }
     if (c->closure != nullptr) {
@@ -367,14 +378,6 @@ void couple(lbm_context* c, const double* dPos, const double* dVel, const double
         launchClosureFallback(c->p.storage, c->popA, c->mask, dPos, dVel, c->particles, c->mass, c->ucm, a,
                 c->closureOod, c->particleForce, c->reactionFixed, c->touched, partials, c->stream);
         return;
-    }
-    const int* order = nullptr;
-    try {
-        if (c->order != nullptr)
-            order = coupleOrderAt(c->order, step, dPos, c->particles, a, c->stream);
-    }
-    catch (const std::runtime_error& e) {
-        throw Error(LBM_ERROR_RUNTIME, e.what());
     }
     const SpreadBins* bins = nullptr;
     if (c->binned && isStep) {
@@ -681,7 +684,7 @@ void create(const lbm_params* params, const int* solid, int numSolid, const int*
         try {
             if (p.drag_scheme == LBM_DRAG_CENTERED)
                 c->centred = centredCreate(numParts, p.interpolation_stencil, (uint32_t) n);
-            else if (!c->dense)
+            if (p.drag_scheme == LBM_DRAG_CENTERED ? c->dense && p.interpolation_stencil != LBM_STENCIL_NEAREST : !c->dense)
                 // Sparse particles gain DRAM locality from the node order; dense ones would contend for the same
                 // accumulators when neighbours are processed together (measured: 100,000 chain beads with Keys on
                 // 128^3 couple 6% slower in node order), so they keep the index order.
@@ -702,7 +705,7 @@ void create(const lbm_params* params, const int* solid, int numSolid, const int*
         // The moment field: by default for dense particles with the explicit drag; LBM_AMD_FIELD=0 or 1 forces it.
         const char* fieldEnv = getenv("LBM_AMD_FIELD");
         bool field = fieldEnv ? fieldEnv[0] == '1' : c->dense;
-        if (p.drag_scheme == LBM_DRAG_EXPLICIT && field)
+        if (field && (p.drag_scheme == LBM_DRAG_EXPLICIT || p.interpolation_stencil != LBM_STENCIL_NEAREST))
             c->momentField = deviceAlloc<double4>(n);
         // The stencils formed once per particle for the groups of the explicit stencil coupling, by default for dense
         // particles (100,000 Keys beads on 128^3: the coupling kernel 148 -> 110 us, the setup 11 us; for 20,000 sparse

@@ -127,11 +127,11 @@ __device__ __forceinline__ bool reactionInRange(double r, unsigned int* overflow
 }
 
 /*
- * Index of component c of a node's three reaction accumulators.  Sparse particles use node-major [node][3]: a stencil
- * row's reactions share cache lines, which the lattice pass reads and clears (13 us less per step on 20,000 Keys beads
- * on 256^3).  Dense particles (the stencils covering more than a quarter of the lattice) use component planes [3][node]:
- * neighbouring stencils then spread their concurrent atomics over three times as many lines (node-major costs 100,000
- * chain beads on 128^3 23% more).
+ * Index of component c of a node's three reaction accumulators.  Where atomics spread the reactions the layout is
+ * node-major [node][3]: a stencil row's reactions are consecutive words, which the staged atomics (StagedReactions) and
+ * the lattice pass's reads want.  Where one thread writes each node (spreadTiles) it is component planes [3][node], whose
+ * stores and reads are contiguous (the lattice pass of crowded beads in 120^3 reads planes in 71 us, node-major in 81 us;
+ * the atomics gain more than that from the other layout).
  */
 __host__ __device__ inline size_t reactionIndex(uint32_t node, int c, uint32_t n, int planes) {
     return planes ? (size_t) c*n + node : 3*(size_t) node + c;
@@ -270,13 +270,14 @@ void launchParticleNodes(const double* positions, const int* particles, const Pa
 
 /* The centred drag (lbm_centred.hip): its buffers for numParticles coupled particles, and one coupling.  otherForces
    (kJ/mol/nm, all System particles, may be null) are the forces on the particles before the coupling; g is the body
-   acceleration in lattice units.  Throws std::runtime_error. */
+   acceleration in lattice units; field: the moments of the nodes (launchMomentField) for the stencils of dense particles,
+   or nullptr; order: the particles in the order to process their stencils (coupleOrderAt), or nullptr.  Throws std::runtime_error. */
 struct CentredState;
 CentredState* centredCreate(int numParticles, int stencil, uint32_t numNodes);
 void centredDestroy(CentredState* state);
 void centredCouple(CentredState* state, int storage, const void* src, const uint32_t* mask, const double* positions,
         const double* velocities, const double* otherForces, const int* particles, const double* mass,
-        const double* ucm, const ParticleArgs& a, const double g[3], double* particleForce,
+        const double* ucm, const ParticleArgs& a, const double g[3], const double4* field, const int* order, double* particleForce,
         unsigned long long* reactionFixed, uint32_t* touched, double* partials, hipStream_t stream);
 
 /*

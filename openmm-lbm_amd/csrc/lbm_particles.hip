@@ -218,7 +218,7 @@ __global__ void __launch_bounds__(BLOCK) coupleParticles(const S* __restrict__ s
     // Sparse beads with FP16/BF16 populations: each XCD takes a contiguous run of the work-groups, so that beads near
     // in the processing order (sorted by node) share an L2 for the 128 B lines, 64 nodes wide, that they read
     // (coupled step of 256^3 with 20,000 Keys beads 0.401 -> 0.397 ms; no gain with FP32's 32-node lines).
-    const uint32_t group = isReduced<S>() && !BINNED && a.xcdOrder ? xcdContiguousTile(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t group = (isReduced<S>() || BINNED) && a.xcdOrder ? xcdContiguousTile(blockIdx.x, gridDim.x) : blockIdx.x;
     int rank = (int) group*GROUPS + threadIdx.x/LANES;    // position in the processing order
     bool active = rank < a.numParticles;
     int i = active && order != nullptr ? order[rank] : rank;
@@ -250,10 +250,12 @@ __global__ void __launch_bounds__(BLOCK) coupleParticles(const S* __restrict__ s
         finishGroupBinned<LANES>(sl, u, velocities + 3*(size_t) part, positions + 3*(size_t) part, (uint32_t) i, m, active,
                 lane, a, particleForce + 3*(size_t) (active ? i : 0), reactionFixed, touched, wallAcc, myNoise,
                 systemForces != nullptr ? systemForces + 3*(size_t) part : nullptr, bins, pre);
-    else
-        finishGroup<LANES>(sl, u, velocities + 3*(size_t) part, (uint32_t) i, m, active, lane, a,
+    else {
+        __shared__ StagedReactions<BLOCK> staged;
+        finishGroup<LANES, BLOCK>(sl, u, velocities + 3*(size_t) part, (uint32_t) i, m, active, lane, a,
                 particleForce + 3*(size_t) (active ? i : 0), reactionFixed, touched, wallAcc, myNoise,
-                systemForces != nullptr ? systemForces + 3*(size_t) part : nullptr);
+                systemForces != nullptr ? systemForces + 3*(size_t) part : nullptr, &staged);
+    }
     if (partials != nullptr)
         storeWallPartial<BLOCK>(wallAcc, partials);
 }
@@ -535,8 +537,10 @@ __global__ void __launch_bounds__(THREADS) coupleBatch(const ReplicaDesc* __rest
         myNoise = noise[threadIdx.x/LANES];
     }
     double wallAcc[3] = {0, 0, 0};
-    finishGroup<LANES>(sl, u, velocities + 3*(size_t) pp, (uint32_t) (pp - d->particleBegin), active ? mass[pp] : 0.0, active,
-            lane, a, forces + 3*(size_t) pp, d->reactionFixed, d->touched, wallAcc, myNoise);
+    __shared__ StagedReactions<THREADS> staged;
+    finishGroup<LANES, THREADS>(sl, u, velocities + 3*(size_t) pp, (uint32_t) (pp - d->particleBegin),
+            active ? mass[pp] : 0.0, active, lane, a, forces + 3*(size_t) pp, d->reactionFixed, d->touched, wallAcc, myNoise,
+            nullptr, &staged);
 }
 
 /* Leapfrog Verlet of the batch (the coupling force is the only force).  The step counter is advanced by advanceStep,
