@@ -310,13 +310,18 @@ struct uint4x {
     uint32_t x, y, z, w;
 };
 
+/* a ^ b ^ c in one instruction (left to itself the compiler makes two of it). */
+__device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+    return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+}
+
 __device__ __forceinline__ uint4x philox(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0, uint32_t k1) {
 #pragma unroll
     for (int round = 0; round < 10; round++) {
         uint64_t p0 = (uint64_t) PHILOX_M0*c0;
         uint64_t p1 = (uint64_t) PHILOX_M1*c2;
-        uint32_t n0 = (uint32_t) (p1 >> 32) ^ c1 ^ k0;
-        uint32_t n2 = (uint32_t) (p0 >> 32) ^ c3 ^ k1;
+        uint32_t n0 = xor3((uint32_t) (p1 >> 32), c1, k0);
+        uint32_t n2 = xor3((uint32_t) (p0 >> 32), c3, k1);
         c1 = (uint32_t) p1;
         c3 = (uint32_t) p0;
         c0 = n0;
@@ -552,23 +557,33 @@ __device__ __forceinline__ typename StorageTraits<S>::Real loadPopStream(const S
         return __builtin_nontemporal_load(asGlobal(p));
 }
 
+/* The random bits of population q's stochastic rounding, from the node's hash.  v_cvt_sr_f16_f32 takes bits 31-19 of its
+   word (v_cvt_sr_bf16_f32 31-16), so FP16 needs no folding of the high bits into the low ones. */
 template <typename S>
-__device__ __forceinline__ void storePopStream(S* p, typename StorageTraits<S>::Real v, uint32_t rnd) {
+__device__ __forceinline__ uint32_t roundingBits(uint32_t hash, int q) {
+    const uint32_t r = (hash ^ (uint32_t) (q*0x9E3779B9u))*0x85EBCA6Bu;
+    return std::is_same<S, __half>::value ? r : r ^ (r >> 13);
+}
+
+template <typename S>
+__device__ __forceinline__ void storePopStream(__attribute__((address_space(1))) S* p, typename StorageTraits<S>::Real v,
+        uint32_t rnd) {
+    using Bits = __attribute__((address_space(1))) uint16_t;
     if constexpr (std::is_same<S, __half>::value) {
         typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-        half2v h = {0, 0};
+        half2v h = __builtin_bit_cast(half2v, v);      // the half that is not stored: anything, here v's own register
         h = __builtin_amdgcn_cvt_sr_f16_f32(h, v, rnd, false);
-        __builtin_nontemporal_store(__builtin_bit_cast(uint16_t, h[0]), asGlobal(reinterpret_cast<uint16_t*>(p)));
+        __builtin_nontemporal_store(__builtin_bit_cast(uint16_t, h[0]), (Bits*) p);
     }
     else if constexpr (std::is_same<S, __hip_bfloat16>::value) {
         typedef __bf16 bf2v __attribute__((ext_vector_type(2)));
-        bf2v h = {0, 0};
+        bf2v h = __builtin_bit_cast(bf2v, v);
         h = __builtin_amdgcn_cvt_sr_bf16_f32(h, v, rnd, false);
-        __builtin_nontemporal_store(__builtin_bit_cast(uint16_t, h[0]), asGlobal(reinterpret_cast<uint16_t*>(p)));
+        __builtin_nontemporal_store(__builtin_bit_cast(uint16_t, h[0]), (Bits*) p);
     }
     else {
         (void) rnd;
-        __builtin_nontemporal_store(v, asGlobal(p));
+        __builtin_nontemporal_store(v, p);
     }
 }
 

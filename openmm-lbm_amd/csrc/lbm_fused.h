@@ -104,20 +104,29 @@ __device__ __forceinline__ void collideNode(const typename StorageTraits<S>::Rea
     uint32_t rnd = 0;
     if constexpr (isReduced<S>())
         rnd = mixBits(node ^ a.roundSeed);
+    auto* base = asGlobal(dst);
+    [[maybe_unused]] uint32_t offset = (uint32_t) e*(uint32_t) sizeof(S);
 #pragma unroll
     for (int q = 0; q < NQ; q++) {
         uint32_t r = 0;
-        if constexpr (isReduced<S>()) {
-            r = (rnd ^ (uint32_t) (q*0x9E3779B9u))*0x85EBCA6Bu;
-            r ^= r >> 13;
-        }
+        if constexpr (isReduced<S>())
+            r = roundingBits<S>(rnd, q);
         R v = (R) out[q];
         if constexpr (FLUCT)
             v += noise[q];
         if constexpr (WIDE)
-            storePopStream(dst + (uint64_t) q*a.g.qstride + e, v, r);
-        else
-            storePopStream(atByte(dst + (size_t) q*a.g.qstride, e*(uint32_t) sizeof(S)), v, r);
+            storePopStream<S>(base + (uint64_t) q*a.g.qstride + e, v, r);
+        else {
+            // With FP16/BF16 storage and fluctuations the pass is bound by the issue of its instructions (a wavefront's 767
+            // vector ones, 684 with this, Philox's three-input xors and no idle halves in the roundings: 256^3 FP16
+            // 287 -> 256 us, 128^3 39.6 -> 37.4 us; FP32 734 -> 673, 433 -> 432 us, bound by memory).
+            // The node's byte offset, opaque from one population to the next: each store then takes it beside a scalar
+            // base.  Seen as one value, it made the compiler step a 64-bit vector address instead.
+            asm("" : "+v"(offset));
+            using Byte = __attribute__((address_space(1))) char;
+            using Pop = __attribute__((address_space(1))) S;
+            storePopStream<S>((Pop*) ((Byte*) (base + (size_t) q*a.g.qstride) + offset), v, r);
+        }
     }
 }
 
