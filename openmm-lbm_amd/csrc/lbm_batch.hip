@@ -44,16 +44,6 @@ T* alloc(size_t count, const char* what) {
     return (T*) p;
 }
 
-FastDiv fastDivOf(uint32_t d) {
-    FastDiv f;
-    f.d = d;
-    f.l = 0;
-    while ((1ull << f.l) < d)
-        f.l++;
-    f.m = d <= 1 ? 0 : (uint32_t) (((1ull << 32)*((1ull << f.l) - d))/d + 1);
-    return f;
-}
-
 }  // namespace
 
 struct lbm_batch {
@@ -115,8 +105,7 @@ void buildTiles(lbm_batch* b, int threads) {
     std::vector<uint16_t> tiles;
     for (int r = 0; r < b->numReplicas; r++) {
         b->desc[r].tileBegin = (uint32_t) tiles.size();
-        uint32_t n = b->desc[r].step.g.n;
-        uint32_t count = (n + threads - 1)/threads;
+        uint32_t count = (uint32_t) ((fusedThreads(b->desc[r].step.g) + threads - 1)/threads);
         tiles.insert(tiles.end(), count, (uint16_t) r);
     }
     if (b->tileReplica)
@@ -252,10 +241,8 @@ void createBatch(lbm_batch* b, int R, const lbm_params* params, const int* numPa
         g.nz = p.nz;
         g.nxy = (uint32_t) (p.nx*p.ny);
         g.n = (uint32_t) ((int64_t) p.nx*p.ny*p.nz);
-        g.divx = fastDivOf(p.nx);
-        g.divxy = fastDivOf(g.nxy);
         g.rowShift = 0;
-        g.qstride = g.nx;
+        const uint64_t popCount = layoutRows(g, sizeof(float));
         g.openX = g.openY = g.openZ = 0;
         double cellMass = p.density*p.dx*p.dx*p.dx;
         uint32_t seed = (uint32_t) p.random_number_seed;
@@ -291,16 +278,18 @@ void createBatch(lbm_batch* b, int R, const lbm_params* params, const int* numPa
         d.dt = p.dt;
         d.particleBegin = particleBegin;
         size_t n = g.n;
-        d.popA = alloc<float>(NQ*n, "populations");
-        d.popB = alloc<float>(NQ*n, "populations");
+        d.popA = alloc<float>(popCount, "populations");
+        d.popB = alloc<float>(popCount, "populations");
         d.reactionFixed = alloc<unsigned long long>(3*n, "reactions");
-        d.touched = alloc<uint32_t>((n + 31)/32, "touched mask");
-        b->buffers.insert(b->buffers.end(), {d.popA, d.popB, d.reactionFixed, d.touched});
+        d.touchedA = alloc<uint32_t>((n + 31)/32, "touched mask");
+        d.touchedB = alloc<uint32_t>((n + 31)/32, "touched mask");
+        b->buffers.insert(b->buffers.end(), {d.popA, d.popB, d.reactionFixed, d.touchedA, d.touchedB});
         hipCheck(hipMemsetAsync(d.reactionFixed, 0, 3*n*sizeof(unsigned long long), b->stream), "memset");
-        hipCheck(hipMemsetAsync(d.touched, 0, ((n + 31)/32)*sizeof(uint32_t), b->stream), "memset");
+        hipCheck(hipMemsetAsync(d.touchedA, 0, ((n + 31)/32)*sizeof(uint32_t), b->stream), "memset");
+        hipCheck(hipMemsetAsync(d.touchedB, 0, ((n + 31)/32)*sizeof(uint32_t), b->stream), "memset");
         launchInitEquilibrium(LBM_STORAGE_FP32, d.popA, nullptr, g, p.initial_velocity[0], p.initial_velocity[1],
                 p.initial_velocity[2], b->stream);
-        hipCheck(hipMemcpyAsync(d.popB, d.popA, NQ*n*sizeof(float), hipMemcpyDeviceToDevice, b->stream), "copy");
+        hipCheck(hipMemcpyAsync(d.popB, d.popA, popCount*sizeof(float), hipMemcpyDeviceToDevice, b->stream), "copy");
         for (int i = 0; i < numParticles[r]; i++) {
             double m = masses[particleBegin + i];
             if (!(m > 0))

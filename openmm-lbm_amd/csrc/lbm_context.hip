@@ -51,16 +51,6 @@ struct Error : public std::runtime_error {
         } \
     } while (0)
 
-static FastDiv makeFastDiv(uint32_t d) {
-    FastDiv f;
-    f.d = d;
-    f.l = 0;
-    while ((1ull << f.l) < d)
-        f.l++;
-    f.m = d <= 1 ? 0 : (uint32_t) (((1ull << 32)*((1ull << f.l) - d))/d + 1);
-    return f;
-}
-
 template <typename T>
 static T* deviceAlloc(size_t count) {
     if (count == 0)
@@ -141,7 +131,10 @@ struct lbm_context {
     double* particleForce = nullptr;
     std::vector<double> hostForce;
     unsigned long long* reactionFixed = nullptr;   // [node][3] fixed-point accumulators of the particle reactions
-    uint32_t* touched = nullptr;                   // one bit per node: accumulators holding a reaction
+    // One bit per node, accumulators holding a reaction: the mask that the next lattice step's coupling sets (clear before
+    // it) and the other, which that step's fused pass clears; they swap with each step.
+    uint32_t* touched = nullptr;
+    uint32_t* nextTouched = nullptr;
     double* stagePos = nullptr;
     double* stageVel = nullptr;
     // Learned closure (include/lbm_amd_closure.h): the network and its per-particle buffers.
@@ -414,7 +407,8 @@ void advanceFluid(lbm_context* c, const double* dPos, const double* dVel, const 
         HIP_CHECK(hipEventRecord(ev.first, c->stream));
     }
     launchFused(c->p.storage, c->fusedPath, c->mask != nullptr, particles, c->fluct(), c->popA, c->popB, c->mask,
-            c->reactionFixed, c->touched, c->ucm, a, c->stream);
+            c->reactionFixed, c->touched, c->nextTouched, c->ucm, a, c->stream);
+    std::swap(c->touched, c->nextTouched);
     if (c->profile) {
         HIP_CHECK(hipEventRecord(ev.second, c->stream));
         c->events.push_back(ev);
@@ -532,7 +526,7 @@ void destroy(lbm_context* c) {
                        c->overflow, c->binCounts[0], c->binCounts[1], c->binSpilled, c->bins.beads, c->bins.anchor, c->bins.force,
                        c->bins.slotWeight, c->momentField, c->axisStencils,
                        c->ucm, c->wallPartials, c->particles, c->mass, c->particleForce, c->reactionFixed,
-                       c->touched, c->stagePos, c->stageVel, c->closureX, c->closureNode, c->closureU, c->closureDu,
+                       c->touched, c->nextTouched, c->stagePos, c->stageVel, c->closureX, c->closureNode, c->closureU, c->closureDu,
                        c->closureOod, c->closureFrame, c->closureCounters, c->closureField, c->stageForce};
     for (void* b : buffers)
         if (b)
@@ -568,8 +562,6 @@ void create(const lbm_params* params, const int* solid, int numSolid, const int*
     c->g.nz = p.nz;
     c->g.nxy = (uint32_t) (p.nx*p.ny);
     c->g.n = (uint32_t) n;
-    c->g.divx = makeFastDiv(p.nx);
-    c->g.divxy = makeFastDiv(c->g.nxy);
     c->g.openX = c->openAxis(0);
     c->g.openY = c->openAxis(1);
     c->g.openZ = c->openAxis(2);
@@ -582,13 +574,13 @@ void create(const lbm_params* params, const int* solid, int numSolid, const int*
     c->g.rowShift = rowBlock == 4 ? 2u : rowBlock == 2 ? 1u : 0u;
     while (c->g.rowShift > 0 && p.ny % (1 << c->g.rowShift) != 0)
         c->g.rowShift--;
-    c->g.qstride = (uint32_t) p.nx << c->g.rowShift;
     if (n > (1ull << 30))
         throw Error(LBM_ERROR_INVALID, "LBMForce: the lattice is too large for one GPU: at most 2^30 nodes");
+    const uint64_t popBytes = layoutRows(c->g, c->elem)*c->elem;
     // The fused pass addresses populations by 32-bit byte offsets while an array of them fits in 4 GiB (up to 56.5 M
     // nodes with FP32 storage), and by 64-bit indices beyond.  LBM_AMD_WIDE_ADDRESSING=1 takes the 64-bit path always.
     const char* wideEnv = getenv("LBM_AMD_WIDE_ADDRESSING");
-    c->wide = NQ*n*c->elem > (1ull << 32) || (wideEnv && wideEnv[0] == '1');
+    c->wide = popBytes > (1ull << 32) || (wideEnv && wideEnv[0] == '1');
     // The LDS-staged pass (fusedRows) where the row length allows it; LBM_AMD_FUSED_ROWS=0 or 1 forces the choice
     // (where it fits).
     const char* rowsEnv = getenv("LBM_AMD_FUSED_ROWS");
@@ -598,8 +590,8 @@ void create(const lbm_params* params, const int* solid, int numSolid, const int*
     if (c->seed == 0)
         c->seed = (uint32_t) std::chrono::high_resolution_clock::now().time_since_epoch().count() | 1u;
     HIP_CHECK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-    c->popA = deviceAlloc<char>(NQ*n*c->elem);
-    c->popB = deviceAlloc<char>(NQ*n*c->elem);
+    c->popA = deviceAlloc<char>(popBytes);
+    c->popB = deviceAlloc<char>(popBytes);
     // Solid nodes.
     c->numFluid = (double) n;
     if (numSolid > 0) {
@@ -677,6 +669,8 @@ void create(const lbm_params* params, const int* solid, int numSolid, const int*
         HIP_CHECK(hipMemsetAsync(c->reactionFixed, 0, 3*n*sizeof(unsigned long long), c->stream));
         c->touched = deviceAlloc<uint32_t>((n + 31)/32);
         HIP_CHECK(hipMemsetAsync(c->touched, 0, ((n + 31)/32)*sizeof(uint32_t), c->stream));
+        c->nextTouched = deviceAlloc<uint32_t>((n + 31)/32);
+        HIP_CHECK(hipMemsetAsync(c->nextTouched, 0, ((n + 31)/32)*sizeof(uint32_t), c->stream));
         c->stagePos = deviceAlloc<double>(3*(size_t) std::max(numSys, 1));
         c->stageVel = deviceAlloc<double>(3*(size_t) std::max(numSys, 1));
         if (p.drag_scheme == LBM_DRAG_CENTERED)
@@ -741,7 +735,7 @@ void create(const lbm_params* params, const int* solid, int numSolid, const int*
     // The fluid at equilibrium with the initial velocity; solid nodes hold no fluid.
     launchInitEquilibrium(p.storage, c->popA, c->mask, c->g, p.initial_velocity[0], p.initial_velocity[1],
             p.initial_velocity[2], c->stream);
-    HIP_CHECK(hipMemcpyAsync(c->popB, c->popA, NQ*n*c->elem, hipMemcpyDeviceToDevice, c->stream));
+    HIP_CHECK(hipMemcpyAsync(c->popB, c->popA, popBytes, hipMemcpyDeviceToDevice, c->stream));
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipStreamSynchronize(c->stream));
 }

@@ -609,7 +609,11 @@ struct Geometry {
     FastDiv divx, divxy;
     int openX, openY, openZ;
     uint32_t rowShift = 0;      // log2 of the rows per block of the population layout (elementOf)
-    uint32_t qstride = 0;       // elements between populations of one node: nx << rowShift
+    uint32_t qstride = 0;       // elements between populations of one node: the row stride << rowShift
+    // The fused pass's threads: each row in chunks of 2^chunkShift nodes, chunksPerRow of them (chunkedNode).
+    uint32_t chunkShift = 5, chunksPerRow = 0;
+    FastDiv divChunks, divy;
+    int padded = 0;             // rows hold whole chunks: the lanes past a row's end store too
 };
 
 /*
@@ -648,9 +652,25 @@ __device__ __forceinline__ void nodeCoords(const Geometry& g, uint32_t node, uin
     i = rem - j*g.nx;
 }
 
+/*
+ * The node of thread t of the fused pass: each row (j, k) is taken in chunks of 2^chunkShift nodes from its start, by
+ * consecutive threads, so that a chunk's loads and stores never run across a row's end.  Returns false past the last row.
+ * i may lie past the row's end (the row's last chunk).
+ */
+__device__ __forceinline__ bool chunkedNode(const Geometry& g, uint32_t t, uint32_t& i, uint32_t& j, uint32_t& k) {
+    const uint32_t chunk = t >> g.chunkShift;
+    const uint32_t row = fastDiv(chunk, g.divChunks);
+    if (row >= g.ny*g.nz)
+        return false;
+    i = ((chunk - row*g.chunksPerRow) << g.chunkShift) + (t & ((1u << g.chunkShift) - 1u));
+    k = fastDiv(row, g.divy);
+    j = row - k*g.ny;
+    return true;
+}
+
 template <typename I>
 __device__ __forceinline__ NeighboursOf<I> elementNeighbours(const Geometry& g, uint32_t i, uint32_t j, uint32_t k) {
-    const I slab = (I) NQ*(I) g.nxy, all = (I) NQ*(I) g.n;
+    const I slab = (I) NQ*(I) (g.qstride >> g.rowShift)*(I) g.ny, all = slab*(I) g.nz;
     const uint32_t r = j + g.ny*k;
     const I here = rowElement<I>(g, r);
     NeighboursOf<I> nb;

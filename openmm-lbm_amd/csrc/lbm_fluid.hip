@@ -25,12 +25,10 @@ namespace lbm {
 /* ------------------------------------------------------------------------------------------ */
 template <typename S, bool SOLIDS, bool REACTION, bool FLUCT, int THREADS, bool WIDE>
 __global__ void __launch_bounds__(THREADS) fusedStep(const S* __restrict__ src, S* __restrict__ dst,
-        const uint32_t* __restrict__ mask, unsigned long long* __restrict__ reactionFixed, uint32_t* __restrict__ touched,
-        const double* __restrict__ ucm, StepArgs a) {
-    uint32_t node = blockIdx.x*THREADS + threadIdx.x;
-    if (node >= a.g.n)
-        return;
-    fusedNode<S, SOLIDS, REACTION, FLUCT, WIDE>(src, dst, mask, reactionFixed, touched, ucm, a, node);
+        const uint32_t* __restrict__ mask, unsigned long long* __restrict__ reactionFixed,
+        const uint32_t* __restrict__ touched, uint32_t* __restrict__ nextTouched, const double* __restrict__ ucm, StepArgs a) {
+    fusedNode<S, SOLIDS, REACTION, FLUCT, WIDE>(src, dst, mask, reactionFixed, touched, nextTouched, ucm, a,
+            blockIdx.x*THREADS + threadIdx.x);
 }
 
 /* The storage value v as the load type (FP32 for FP16/BF16). */
@@ -70,8 +68,8 @@ __device__ __forceinline__ int directionOf(uint64_t packed, int q) {
 template <typename S, bool SOLIDS, bool REACTION, bool FLUCT, int SEG>
 __global__ void __launch_bounds__(ROW_THREADS) __attribute__((amdgpu_waves_per_eu(sizeof(S) == 8 ? 1 : 8)))
 fusedRows(const S* __restrict__ src, S* __restrict__ dst,
-        const uint32_t* __restrict__ mask, unsigned long long* __restrict__ reactionFixed, uint32_t* __restrict__ touched,
-        const double* __restrict__ ucm, StepArgs a) {
+        const uint32_t* __restrict__ mask, unsigned long long* __restrict__ reactionFixed,
+        const uint32_t* __restrict__ touched, uint32_t* __restrict__ nextTouched, const double* __restrict__ ucm, StepArgs a) {
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     constexpr int T = ROW_THREADS;
     constexpr int V = 16/(int) sizeof(S);
@@ -120,7 +118,7 @@ fusedRows(const S* __restrict__ src, S* __restrict__ dst,
     const uint32_t node = base + threadIdx.x;
     if (node >= a.g.n)
         return;
-    const uint32_t touchedWord = takeTouchedWord<REACTION>(touched, node);
+    const uint32_t touchedWord = takeTouchedWord<REACTION>(touched, nextTouched, node);
     if constexpr (SOLIDS)
         if (isSolid(mask, node))
             return;
@@ -148,15 +146,13 @@ __global__ void __launch_bounds__(THREADS) fusedBatch(const ReplicaDesc* __restr
     // its reads' overfetch at tile borders shared in one L2 (runs of 128: 0.468 ms; of 256 or one run per XCD: none).
     const uint32_t tile = xcdOrder ? xcdChunkedTile(blockIdx.x, gridDim.x) : blockIdx.x;
     const ReplicaDesc* d = table + tileReplica[tile];
-    uint32_t node = (tile - d->tileBegin)*THREADS + threadIdx.x;
     StepArgs a = d->step;
-    if (node >= a.g.n)
-        return;
     a.step = *stepCounter;
     a.roundSeed = 0;
     const float* src = (a.step & 1) ? d->popB : d->popA;
     float* dst = (a.step & 1) ? d->popA : d->popB;
-    fusedNode<float, false, true, FLUCT>(src, dst, nullptr, d->reactionFixed, d->touched, nullptr, a, node);
+    fusedNode<float, false, true, FLUCT>(src, dst, nullptr, d->reactionFixed, (a.step & 1) ? d->touchedB : d->touchedA,
+            (a.step & 1) ? d->touchedA : d->touchedB, nullptr, a, (tile - d->tileBegin)*THREADS + threadIdx.x);
 }
 
 void launchFusedBatch(int threads, bool fluct, const ReplicaDesc* table, const uint16_t* tileReplica, uint32_t numTiles,
@@ -649,6 +645,43 @@ static inline unsigned gridFor(uint64_t n) {
     return (unsigned) ((n + BLOCK - 1)/BLOCK);
 }
 
+static FastDiv makeFastDiv(uint32_t d) {
+    FastDiv f;
+    f.d = d;
+    f.l = 0;
+    while ((1ull << f.l) < d)
+        f.l++;
+    f.m = d <= 1 ? 0 : (uint32_t) (((1ull << 32)*((1ull << f.l) - d))/d + 1);
+    return f;
+}
+
+uint64_t layoutRows(Geometry& g, size_t elementSize) {
+    g.divx = makeFastDiv(g.nx);
+    g.divxy = makeFastDiv(g.nxy);
+    g.divy = makeFastDiv(g.ny);
+    // Chunks of 32 nodes, or of 16 with FP64 storage: a 128 B line (64 B with FP16 or BF16: chunks of 64 gain nothing
+    // there and idle more lanes), from the row's start and into rows padded to whole chunks, so that every line is
+    // written whole by one half-wavefront.  Where nx is no multiple of the chunk, consecutive threads on consecutive nodes
+    // wrote lines in pieces from wavefronts on different XCDs.  The pass without noise, that order against this one: FP32
+    // 150^3 151 -> 98.8 us, 120^3 67.0 -> 51.9, 200^3 295 -> 238, 75^3 23.1 -> 20.3; FP16 150^3 74.0 -> 56.6, 101^3
+    // 27.6 -> 21.0; FP64 150^3 247 -> 195, 101^3 79.4 -> 65.6 (chunks of 32: 69.1).  Chunks without the padding: FP32
+    // 150^3 145 us; padding without the chunks: 156.  FP32 takes chunks of 16 (64 B) where those of 32 would pad a row by
+    // more than a quarter (48^3: 10.9 us with 32, 9.8 with 16; 80^3 and 112^3, padded by less: 20.9 and 45.7 with 32, 20.8
+    // and 47.4 with 16).
+    const uint32_t by32 = (g.nx + 31u)/32u*32u;
+    g.chunkShift = elementSize == 8 || (elementSize == 4 && (by32 - g.nx)*4u > g.nx) ? 4 : 5;
+    g.chunksPerRow = ((g.nx - 1u) >> g.chunkShift) + 1u;
+    g.divChunks = makeFastDiv(g.chunksPerRow);
+    const uint64_t rows = (uint64_t) g.ny*g.nz;
+    const uint32_t whole = g.chunksPerRow << g.chunkShift;
+    // No padding where rows are grouped in blocks, or where it would take an array that fits beyond the 4 GiB of the
+    // 32-bit offsets.
+    g.padded = whole != g.nx && g.rowShift == 0 && (NQ*rows*whole*elementSize <= (1ull << 32) ||
+            NQ*rows*g.nx*elementSize > (1ull << 32)) ? 1 : 0;
+    g.qstride = (g.padded ? whole : g.nx) << g.rowShift;
+    return NQ*rows*(g.qstride >> g.rowShift);
+}
+
 #define LBM_DISPATCH_STORAGE(storage, S, ...) \
     switch (storage) { \
     case LBM_STORAGE_FP16: { using S = __half; __VA_ARGS__; break; } \
@@ -659,45 +692,45 @@ static inline unsigned gridFor(uint64_t n) {
 
 template <typename S, bool SOL, bool REA, bool WIDE>
 static void launchFusedT(bool fluct, const void* src, void* dst, const uint32_t* mask, unsigned long long* reactionFixed,
-        uint32_t* touched, const double* ucm, const StepArgs& a, hipStream_t stream) {
+        const uint32_t* touched, uint32_t* nextTouched, const double* ucm, const StepArgs& a, hipStream_t stream) {
     // FP16/BF16 storage: 256-thread work-groups (2% faster on config3 than 512; 512 is best for FP32).
     constexpr int T = sizeof(S) == 2 ? FUSED_THREADS_REDUCED : FUSED_THREADS;
-    unsigned grid = (unsigned) ((a.g.n + T - 1)/T);
+    unsigned grid = (unsigned) ((fusedThreads(a.g) + T - 1)/T);
     if (fluct)
         fusedStep<S, SOL, REA, true, T, WIDE><<<grid, T, 0, stream>>>((const S*) src, (S*) dst, mask, reactionFixed,
-                touched, ucm, a);
+                touched, nextTouched, ucm, a);
     else
         fusedStep<S, SOL, REA, false, T, WIDE><<<grid, T, 0, stream>>>((const S*) src, (S*) dst, mask, reactionFixed,
-                touched, ucm, a);
+                touched, nextTouched, ucm, a);
 }
 
 template <typename S, bool SOL, bool REA, int SEG>
 static void launchRowsT(bool fluct, const void* src, void* dst, const uint32_t* mask, unsigned long long* reactionFixed,
-        uint32_t* touched, const double* ucm, const StepArgs& a, hipStream_t stream) {
+        const uint32_t* touched, uint32_t* nextTouched, const double* ucm, const StepArgs& a, hipStream_t stream) {
     unsigned grid = (unsigned) ((a.g.n + ROW_THREADS - 1)/ROW_THREADS);
     if (fluct)
         fusedRows<S, SOL, REA, true, SEG><<<grid, ROW_THREADS, 0, stream>>>((const S*) src, (S*) dst, mask,
-                reactionFixed, touched, ucm, a);
+                reactionFixed, touched, nextTouched, ucm, a);
     else
         fusedRows<S, SOL, REA, false, SEG><<<grid, ROW_THREADS, 0, stream>>>((const S*) src, (S*) dst, mask,
-                reactionFixed, touched, ucm, a);
+                reactionFixed, touched, nextTouched, ucm, a);
 }
 
 template <typename S, bool SOL, bool REA>
 static void launchPathT(int path, bool fluct, const void* src, void* dst, const uint32_t* mask,
-        unsigned long long* reactionFixed, uint32_t* touched, const double* ucm, const StepArgs& a, hipStream_t stream) {
+        unsigned long long* reactionFixed, const uint32_t* touched, uint32_t* nextTouched, const double* ucm, const StepArgs& a, hipStream_t stream) {
     switch (path) {
     case FUSED_WIDE:
-        launchFusedT<S, SOL, REA, true>(fluct, src, dst, mask, reactionFixed, touched, ucm, a, stream);
+        launchFusedT<S, SOL, REA, true>(fluct, src, dst, mask, reactionFixed, touched, nextTouched, ucm, a, stream);
         break;
     case FUSED_ROWS:
         if (a.g.nx == 128)
-            launchRowsT<S, SOL, REA, 128>(fluct, src, dst, mask, reactionFixed, touched, ucm, a, stream);
+            launchRowsT<S, SOL, REA, 128>(fluct, src, dst, mask, reactionFixed, touched, nextTouched, ucm, a, stream);
         else
-            launchRowsT<S, SOL, REA, ROW_THREADS>(fluct, src, dst, mask, reactionFixed, touched, ucm, a, stream);
+            launchRowsT<S, SOL, REA, ROW_THREADS>(fluct, src, dst, mask, reactionFixed, touched, nextTouched, ucm, a, stream);
         break;
     default:
-        launchFusedT<S, SOL, REA, false>(fluct, src, dst, mask, reactionFixed, touched, ucm, a, stream);
+        launchFusedT<S, SOL, REA, false>(fluct, src, dst, mask, reactionFixed, touched, nextTouched, ucm, a, stream);
     }
 }
 
@@ -706,16 +739,16 @@ bool fusedRowsFit(uint32_t nx, bool wide, uint32_t rowShift) {
 }
 
 void launchFused(int storage, int path, bool solids, bool reaction, bool fluct, const void* src, void* dst,
-        const uint32_t* mask, unsigned long long* reactionFixed, uint32_t* touched, const double* ucm, const StepArgs& a,
+        const uint32_t* mask, unsigned long long* reactionFixed, const uint32_t* touched, uint32_t* nextTouched, const double* ucm, const StepArgs& a,
         hipStream_t stream) {
     LBM_DISPATCH_STORAGE(storage, S, {
         if (solids) {
-            if (reaction) launchPathT<S, true, true>(path, fluct, src, dst, mask, reactionFixed, touched, ucm, a, stream);
-            else launchPathT<S, true, false>(path, fluct, src, dst, mask, reactionFixed, touched, ucm, a, stream);
+            if (reaction) launchPathT<S, true, true>(path, fluct, src, dst, mask, reactionFixed, touched, nextTouched, ucm, a, stream);
+            else launchPathT<S, true, false>(path, fluct, src, dst, mask, reactionFixed, touched, nextTouched, ucm, a, stream);
         }
         else {
-            if (reaction) launchPathT<S, false, true>(path, fluct, src, dst, mask, reactionFixed, touched, ucm, a, stream);
-            else launchPathT<S, false, false>(path, fluct, src, dst, mask, reactionFixed, touched, ucm, a, stream);
+            if (reaction) launchPathT<S, false, true>(path, fluct, src, dst, mask, reactionFixed, touched, nextTouched, ucm, a, stream);
+            else launchPathT<S, false, false>(path, fluct, src, dst, mask, reactionFixed, touched, nextTouched, ucm, a, stream);
         }
     })
 }

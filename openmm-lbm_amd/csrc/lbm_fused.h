@@ -11,16 +11,17 @@
 namespace lbm {
 
 /*
- * The touched-mask word of a node's wavefront (32 nodes): every lane reads it, then its first lane (always inside the
- * lattice, since words are 32-aligned) clears it for the next step.
+ * The touched-mask word of a node, read from the step's mask; the word's first node clears it in the next step's mask (the
+ * two masks alternate, so that no thread can clear a word that another has yet to read).
  */
 template <bool REACTION>
-__device__ __forceinline__ uint32_t takeTouchedWord(uint32_t* __restrict__ touched, uint32_t node) {
+__device__ __forceinline__ uint32_t takeTouchedWord(const uint32_t* __restrict__ touched, uint32_t* __restrict__ nextTouched,
+        uint32_t node) {
     uint32_t touchedWord = 0;
     if constexpr (REACTION) {
         touchedWord = *asGlobal(touched + (node >> 5));
-        if ((node & 31) == 0 && touchedWord != 0)
-            *asGlobal(touched + (node >> 5)) = 0;
+        if ((node & 31) == 0)
+            *asGlobal(nextTouched + (node >> 5)) = 0;
     }
     return touchedWord;
 }
@@ -131,23 +132,33 @@ __device__ __forceinline__ void collideNode(const typename StorageTraits<S>::Rea
 }
 
 /*
- * One node: pull C_q(x - c_q) from src and collide (collideNode).  Returns without writing for solid nodes.
+ * Thread t of the pass: one node (chunkedNode), pull C_q(x - c_q) from src and collide (collideNode).  Writes nothing for
+ * solid nodes.  A lane past the end of a padded row repeats the row's last node into the padding, so that the row's last
+ * lines are written whole.
  */
 template <typename S, bool SOLIDS, bool REACTION, bool FLUCT, bool WIDE = false>
 __device__ __forceinline__ void fusedNode(const S* __restrict__ src, S* __restrict__ dst, const uint32_t* __restrict__ mask,
-        unsigned long long* __restrict__ reactionFixed, uint32_t* __restrict__ touched, const double* __restrict__ ucm,
-        const StepArgs& a, uint32_t node) {
-    uint32_t touchedWord = takeTouchedWord<REACTION>(touched, node);
+        unsigned long long* __restrict__ reactionFixed, const uint32_t* __restrict__ touched,
+        uint32_t* __restrict__ nextTouched, const double* __restrict__ ucm, const StepArgs& a, uint32_t t) {
+    uint32_t i, j, k;
+    if (!chunkedNode(a.g, t, i, j, k))
+        return;
+    const uint32_t past = i < a.g.nx ? 0u : i - (a.g.nx - 1u);
+    if (past != 0u && !a.g.padded)
+        return;
+    i -= past;
+    const uint32_t node = (k*a.g.ny + j)*a.g.nx + i;
+    uint32_t touchedWord = 0;
+    if (past == 0u)
+        touchedWord = takeTouchedWord<REACTION>(touched, nextTouched, node);
     if constexpr (SOLIDS)
         if (isSolid(mask, node))
             return;
-    uint32_t i, j, k;
-    nodeCoords(a.g, node, i, j, k);
     using Offset = typename std::conditional<WIDE, long long, int>::type;
     const ElementIndex<WIDE> e = elementOf<ElementIndex<WIDE>>(a.g, i, j, k);
     typename StorageTraits<S>::Real fr[NQ];
     pullNodeStream<S, WIDE>(src, a.g.qstride, e, elementNeighbours<Offset>(a.g, i, j, k), fr);
-    collideNode<S, REACTION, FLUCT, WIDE>(fr, dst, reactionFixed, touchedWord, ucm, a, node, e);
+    collideNode<S, REACTION, FLUCT, WIDE>(fr, dst, reactionFixed, touchedWord, ucm, a, node, e + past);
 }
 
 }  // namespace lbm

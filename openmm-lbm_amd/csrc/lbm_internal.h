@@ -153,7 +153,8 @@ struct ReplicaDesc {
     float* popA;
     float* popB;
     unsigned long long* reactionFixed;
-    uint32_t* touched;
+    uint32_t* touchedA;          // the touched masks of even and odd steps
+    uint32_t* touchedB;
     double dt;                   // ps
     uint32_t tileBegin;          // first work-group of this replica in the fused grid
     int particleBegin;           // first particle of this replica in the batch arrays
@@ -200,8 +201,15 @@ void launchVerletBatch(const ReplicaDesc* table, const uint16_t* particleReplica
 enum FusedPath { FUSED_DIRECT = 0, FUSED_WIDE = 1, FUSED_ROWS = 2 };
 bool fusedRowsFit(uint32_t nx, bool wide, uint32_t rowShift);
 void launchFused(int storage, int path, bool solids, bool reaction, bool fluct, const void* src, void* dst,
-        const uint32_t* mask, unsigned long long* reactionFixed, uint32_t* touched, const double* ucm, const StepArgs& a,
-        hipStream_t stream);
+        const uint32_t* mask, unsigned long long* reactionFixed, const uint32_t* touched, uint32_t* nextTouched,
+        const double* ucm, const StepArgs& a, hipStream_t stream);
+/* Threads of the fused pass (chunkedNode). */
+inline uint64_t fusedThreads(const Geometry& g) {
+    return ((uint64_t) g.ny*g.nz*g.chunksPerRow) << g.chunkShift;
+}
+/* The rows' chunks and the population layout (divisions, chunkShift, qstride, padded) of a lattice whose sizes and
+   rowShift are set; returns the elements of one population array. */
+uint64_t layoutRows(Geometry& g, size_t elementSize);
 void launchMomentReduce(int storage, bool solids, const void* src, const uint32_t* mask, const Geometry& g,
         double* partials, hipStream_t stream);
 void launchFinishReduce(const double* partials, double numFluid, double* totals, double* ucm, hipStream_t stream);

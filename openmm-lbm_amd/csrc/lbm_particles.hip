@@ -539,8 +539,8 @@ __global__ void __launch_bounds__(THREADS) coupleBatch(const ReplicaDesc* __rest
     double wallAcc[3] = {0, 0, 0};
     __shared__ StagedReactions<THREADS> staged;
     finishGroup<LANES, THREADS>(sl, u, velocities + 3*(size_t) pp, (uint32_t) (pp - d->particleBegin),
-            active ? mass[pp] : 0.0, active, lane, a, forces + 3*(size_t) pp, d->reactionFixed, d->touched, wallAcc, myNoise,
-            nullptr, &staged);
+            active ? mass[pp] : 0.0, active, lane, a, forces + 3*(size_t) pp, d->reactionFixed,
+            (a.step & 1) ? d->touchedB : d->touchedA, wallAcc, myNoise, nullptr, &staged);
 }
 
 /* Leapfrog Verlet of the batch (the coupling force is the only force).  The step counter is advanced by advanceStep,

@@ -6,7 +6,7 @@ import pytest
 from lbm_amd import LBMForce
 from lbm_amd.harness import DeviceParticles
 import oracle_lib
-from parity import Setup
+from parity import Setup, lockstep
 
 pytestmark = pytest.mark.gpu
 
@@ -63,3 +63,26 @@ def test_merged_launch_between_steps_is_bit_identical(beads, walls, bonds):
         assert np.array_equal(a, b)
     if walls and beads > 1:
         assert np.abs(results[0][3]).max() > 0
+
+
+@pytest.mark.parametrize("storage,tolerance", [(LBMForce.FP32, 1e-5), (LBMForce.FP64, 1e-11)], ids=["fp32", "fp64"])
+@pytest.mark.parametrize("nx", [1, 15, 16, 17, 31, 32, 33, 48, 65])
+def test_row_chunks_match_the_oracle(nx, storage, tolerance):
+    """Rows that end at, before and past the chunks of 16 and 32 nodes that the lattice pass takes, with an irregular
+    solid block and reactions on nodes of every touched-mask word (tolerances of the parity tests)."""
+    rng = np.random.default_rng(nx)
+    ny, nz = 5, 6
+    s = Setup((nx, ny, nz), tau=0.7)
+    s.add_particles(rng.uniform(0, [nx, ny, nz], size=(40, 3)), velocities=rng.normal(scale=0.5, size=(40, 3)))
+
+    def conf(f):
+        if nx > 2:
+            f.setSolidNodes([i + nx*(2 + ny*3) for i in range(nx//2)] + [nx - 1])
+            f.setWallScheme(LBMForce.BounceBack)
+        f.setBodyAcceleration((0.1, 0.05, -0.02))
+        f.setFriction(10.0)
+        f.setTemperature(0.0)
+        f.setInterpolationStencil(LBMForce.Trilinear)
+    s.configure.append(conf)
+    worst, _, _ = lockstep(s, 12, check_every=4, storage=storage)
+    assert max(worst.values()) <= tolerance, worst
