@@ -12,10 +12,10 @@
  * kernel.  Backward, dH^T = W dZ^T has the same property.  Per tile of 16 particles: 24 + 16 + 4 MFMAs forward,
  * 4 + 16 more backward.
  *
- * Training (lbm_mlp_train): per minibatch, mlpTrainForward (forward, error, backward through the activations; writes
- * the FP16 activations and errors row by row), mlpWeightGrad (dW = P^T Q over chunks of 256 particles, one 16 x 16 tile
- * of one matrix per wave, partial sums per chunk), mlpUpdate (the chunks summed in a fixed order, Adam on the FP32
- * master parameters, new FP16 operands).  Every sum has a fixed order: training is reproducible run to run.
+ * Training (lbm_mlp_train): per minibatch, mlpTrainForward (forward, error, backward through the activations; writes the
+ * FP16 activations and errors transposed, 256 particles to a chunk) and mlpGradUpdate (dW = P^T Q, one 16 x 16 tile of one
+ * matrix per work-group and one chunk per wave; the chunks summed in a fixed order, Adam on the FP32 master parameters, new
+ * FP16 operands).  Every sum has a fixed order: training is reproducible run to run.
  */
 #include "lbm_mlp.h"
 #include <algorithm>
@@ -40,6 +40,9 @@ typedef float float4_t __attribute__((ext_vector_type(4)));
 constexpr int WAVES = 4;                 // waves per work-group of the network kernels
 constexpr int CHUNK = 256;               // particles per partial sum of the weight gradients
 constexpr int GRAD_JOBS = 24 + 16 + 4;   // 16 x 16 tiles of dW1, dW2, dW3
+constexpr int GRAD_WAVES = 8;            // chunks that a work-group of the weight gradients takes at a time
+// Chunks up to which one work-group per tile takes them all and updates the parameters (minibatches of up to 8,192 rows).
+constexpr int GRAD_ONE_LAUNCH = 32;
 
 __device__ __forceinline__ float4_t mfma16(half4_t a, half4_t b, float4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0);
@@ -154,134 +157,131 @@ __global__ void __launch_bounds__(64*WAVES) mlpInfer(const MlpDevice* __restrict
 }
 
 /*
- * Training, forward and backward through the activations, one wave per tile of 16 rows of the minibatch (rows[b] is the
- * dataset row of minibatch row b; rows at or beyond count are padding and get zero errors).  Per row b it stores
- * H1, H2 (post-activation), dZ1, dZ2 (errors at the pre-activations) and dY = (2/3)(y - t) as FP16; the loss sum
- * goes to lossSum (a diagnostic).
+ * The layer inputs P and errors Q of a minibatch, as the weight gradients read them: per chunk of CHUNK rows, [unit][row] in
+ * FP16, so that the four consecutive rows of an MFMA operand are one 8-byte load.
+ */
+struct TrainActivations {
+    _Float16 *X, *H1, *H2, *dZ1, *dZ2, *dY;
+};
+
+/* Elements (unit 16t + quad + r, this row) of a tile -> out[chunk][unit][row]. */
+__device__ __forceinline__ void storeTransposed(_Float16* out, int units, int b, int t, int quad, half4_t v) {
+    _Float16* p = out + ((size_t) (b/CHUNK)*units + 16*t + quad)*CHUNK + b % CHUNK;
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+        p[r*CHUNK] = v[r];
+}
+
+/* v rounded to FP32 and then to FP16 (a product and its conversion would otherwise be fused, with one rounding, or not, as
+   the compiler sees fit). */
+__device__ __forceinline__ _Float16 toHalf(float v) {
+    asm("" : "+v"(v));
+    return (_Float16) v;
+}
+
+/*
+ * Training, forward and backward through the activations, one work-group of four waves per tile of 16 rows of the
+ * minibatch (rows[b] is the dataset row of minibatch row b; rows at or beyond count are padding and get zero errors): wave
+ * t computes units 16t .. 16t + 15 of every layer, and the waves exchange their tiles, which are the next layer's B
+ * operands as they are, through LDS.  Stores X, H1, H2 (post-activation), dZ1, dZ2 (errors at the pre-activations) and
+ * dY = (2/3)(y - t); the loss sum goes to lossSum (a diagnostic).  A minibatch of 2,048 rows is 128 tiles: bound by the
+ * latency of one tile's chain (64 divisions and exponentials per lane with one wave per tile), 11.5 us with one wave per
+ * tile, 7.3 us with four.
  */
 __global__ void __launch_bounds__(64*WAVES) mlpTrainForward(const MlpDevice* __restrict__ m,
-        const _Float16* __restrict__ X, const float* __restrict__ T, const int* __restrict__ rows, int count, int tiles,
-        _Float16* __restrict__ H1, _Float16* __restrict__ H2, _Float16* __restrict__ dZ1, _Float16* __restrict__ dZ2,
-        _Float16* __restrict__ dY, double* __restrict__ lossSum) {
-    int lane = threadIdx.x & 63;
-    int tile = blockIdx.x*WAVES + (threadIdx.x >> 6);
-    if (tile >= tiles)
-        return;
-    int row = lane & 15, quad = (lane >> 4)*4;
-    ForwardWeights w;
-    loadForward(m, row, quad, w);
-    int b = tile*16 + row;
-    bool valid = b < count;
-    int src = rows[b];
-    half4_t x[6];
+        const _Float16* __restrict__ X, const float* __restrict__ T, const int* __restrict__ rows, int count,
+        TrainActivations act, double* __restrict__ lossSum) {
+    static_assert(WAVES == 4 && MLP_H == 64, "one wave per 16 hidden units");
+    __shared__ half4_t shared[3][WAVES][64];
+    const int lane = threadIdx.x & 63, t = threadIdx.x >> 6;
+    const int row = lane & 15, quad = (lane >> 4)*4;
+    const int b = blockIdx.x*16 + row;
+    const bool valid = b < count;
+    const int src = rows[b];
+    half4_t x[6], w1[6], w2[4], w3[4], w2n[4];
+    float4_t z1, z2, y;
+#pragma unroll
+    for (int s = 0; s < 6; s++) {
+        x[s] = load4(X + (size_t) src*MLP_IN_PAD + 16*s + quad);
+        w1[s] = load4(m->w1t + (16*t + row)*MLP_IN_PAD + 16*s + quad);
+    }
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        w2[s] = load4(m->w2t + (16*t + row)*MLP_H + 16*s + quad);
+        w3[s] = load4(m->w3t + row*MLP_H + 16*s + quad);
+        w2n[s] = load4(m->w2 + (16*t + row)*MLP_H + 16*s + quad);
+    }
+    const half4_t w3n = load4(m->w3 + (16*t + row)*MLP_OUT_PAD + quad);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        z1[r] = m->b1[16*t + quad + r];
+        z2[r] = m->b2[16*t + quad + r];
+        y[r] = m->b3[quad + r];
+    }
+    // Forward (the sums of forwardTile).
+    half4_t h1, h2, dz1, dz2;
 #pragma unroll
     for (int s = 0; s < 6; s++)
-        x[s] = load4(X + (size_t) src*MLP_IN_PAD + 16*s + quad);
-    Activations a;
-    forwardTile(w, x, a);
+        z1 = mfma16(w1[s], x[s], z1);
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+        h1[r] = toHalf(siluf(z1[r]));
+    shared[0][t][lane] = h1;
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+        z2 = mfma16(w2[s], shared[0][s][lane], z2);
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+        h2[r] = toHalf(siluf(z2[r]));
+    shared[1][t][lane] = h2;
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+        y = mfma16(w3[s], shared[1][s][lane], y);
     // Output error (lanes 0-15 hold outputs 0-3 of their row; output 3 and up are padding).
     float4_t dy = {0, 0, 0, 0};
     float e = 0;
     if (quad == 0 && valid)
         for (int r = 0; r < MLP_OUT; r++) {
-            float d = a.y[r] - T[3*(size_t) src + r];
+            float d = y[r] - T[3*(size_t) src + r];
             dy[r] = (2.0f/3.0f)*d;
             e += d*d;
         }
     half4_t dyb;
 #pragma unroll
     for (int r = 0; r < 4; r++)
-        dyb[r] = (_Float16) dy[r];
+        dyb[r] = toHalf(dy[r]);
     // Backward: dH2^T = W3 dY^T, dZ2 = dH2 silu'(Z2), dH1^T = W2 dZ2^T, dZ1 = dH1 silu'(Z1).
-    half4_t dz2[4], dz1[4];
+    float4_t acc = mfma16(w3n, dyb, float4_t{0, 0, 0, 0});
 #pragma unroll
-    for (int t = 0; t < 4; t++) {
-        half4_t w3n = load4(m->w3 + (16*t + row)*MLP_OUT_PAD + quad);
-        float4_t acc = mfma16(w3n, dyb, float4_t{0, 0, 0, 0});
+    for (int r = 0; r < 4; r++)
+        dz2[r] = toHalf(acc[r]*dsiluf(z2[r]));
+    shared[2][t][lane] = dz2;
+    __syncthreads();
+    acc = float4_t{0, 0, 0, 0};
 #pragma unroll
-        for (int r = 0; r < 4; r++)
-            dz2[t][r] = (_Float16) (acc[r]*dsiluf(a.z2[t][r]));
-    }
+    for (int s = 0; s < 4; s++)
+        acc = mfma16(w2n[s], shared[2][s][lane], acc);
 #pragma unroll
-    for (int t = 0; t < 4; t++) {
-        float4_t acc = {0, 0, 0, 0};
+    for (int r = 0; r < 4; r++)
+        dz1[r] = toHalf(acc[r]*dsiluf(z1[r]));
+    storeTransposed(act.H1, MLP_H, b, t, quad, h1);
+    storeTransposed(act.H2, MLP_H, b, t, quad, h2);
+    storeTransposed(act.dZ1, MLP_H, b, t, quad, dz1);
+    storeTransposed(act.dZ2, MLP_H, b, t, quad, dz2);
 #pragma unroll
-        for (int s = 0; s < 4; s++)
-            acc = mfma16(load4(m->w2 + (16*t + row)*MLP_H + 16*s + quad), dz2[s], acc);
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-            dz1[t][r] = (_Float16) (acc[r]*dsiluf(a.z1[t][r]));
-    }
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-        store4(H1 + (size_t) b*MLP_H + 16*t + quad, a.h1[t]);
-        store4(H2 + (size_t) b*MLP_H + 16*t + quad, a.h2[t]);
-        store4(dZ1 + (size_t) b*MLP_H + 16*t + quad, dz1[t]);
-        store4(dZ2 + (size_t) b*MLP_H + 16*t + quad, dz2[t]);
-    }
-    store4(dY + (size_t) b*MLP_OUT_PAD + quad, dyb);
+    for (int s = 0; s < 6; s++)
+        if (s % WAVES == t)
+            storeTransposed(act.X, MLP_IN_PAD, b, s, quad, x[s]);
+    if (t != WAVES - 1)
+        return;
+    storeTransposed(act.dY, MLP_OUT_PAD, b, 0, quad, dyb);
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1)
         e += __shfl_xor(e, off);
     if (lane == 0)
         atomicAdd(lossSum, (double) e/3.0);
-}
-
-/*
- * Weight gradients: wave (chunk, job) computes one 16 x 16 tile of dW = P^T Q over the 256 minibatch rows of its chunk,
- * P the layer input (X through rows, H1, H2) and Q the layer error (dZ1, dZ2, dY), and, for the first row tile, the
- * bias gradient (column sums of Q).  Written to partials[chunk][parameter].
- */
-__global__ void __launch_bounds__(64*WAVES) mlpWeightGrad(const _Float16* __restrict__ X, const int* __restrict__ rows,
-        const _Float16* __restrict__ H1, const _Float16* __restrict__ H2, const _Float16* __restrict__ dZ1,
-        const _Float16* __restrict__ dZ2, const _Float16* __restrict__ dY, int chunks, float* __restrict__ partials) {
-    int lane = threadIdx.x & 63;
-    int wave = blockIdx.x*WAVES + (threadIdx.x >> 6);
-    int chunk = wave/GRAD_JOBS, job = wave % GRAD_JOBS;
-    if (chunk >= chunks)
-        return;
-    int row = lane & 15, quad = (lane >> 4)*4;
-    const _Float16* P;
-    const _Float16* Q;
-    int pw, qw, ti, to, offW, offB, width;
-    bool gather = false;
-    if (job < 24) {
-        P = X; pw = MLP_IN_PAD; Q = dZ1; qw = MLP_H; ti = job/4; to = job % 4;
-        offW = MLP_OFF_W1; offB = MLP_OFF_B1; width = MLP_H; gather = true;
-    }
-    else if (job < 40) {
-        P = H1; pw = MLP_H; Q = dZ2; qw = MLP_H; ti = (job - 24)/4; to = (job - 24) % 4;
-        offW = MLP_OFF_W2; offB = MLP_OFF_B2; width = MLP_H;
-    }
-    else {
-        P = H2; pw = MLP_H; Q = dY; qw = MLP_OUT_PAD; ti = job - 40; to = 0;
-        offW = MLP_OFF_W3; offB = MLP_OFF_B3; width = MLP_OUT_PAD;
-    }
-    float4_t acc = {0, 0, 0, 0};
-    float bsum = 0;
-    for (int k = 0; k < CHUNK/16; k++) {
-        int b0 = chunk*CHUNK + 16*k + quad;
-        half4_t pa, qb;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            int b = b0 + e;
-            int prow = gather ? rows[b] : b;
-            pa[e] = P[(size_t) prow*pw + 16*ti + row];
-            qb[e] = Q[(size_t) b*qw + 16*to + row];
-            bsum += (float) qb[e];
-        }
-        acc = mfma16(pa, qb, acc);
-    }
-    float* out = partials + (size_t) chunk*MLP_PARAMS;
-#pragma unroll
-    for (int r = 0; r < 4; r++)
-        out[offW + (16*ti + quad + r)*width + 16*to + row] = acc[r];
-    if (ti == 0) {
-        bsum += __shfl_xor(bsum, 16);
-        bsum += __shfl_xor(bsum, 32);
-        if (lane < 16)
-            out[offB + 16*to + lane] = bsum;
-    }
 }
 
 /* The FP16 operands and FP32 biases of parameter p. */
@@ -315,29 +315,117 @@ __global__ void mlpPack(const float* __restrict__ master, MlpDevice* __restrict_
         storeOperand(d, p, master[p]);
 }
 
-/* Sum of the chunk partials (fixed order) / count -> gradient; with apply, one Adam step (beta 0.9, 0.999, eps 1e-8;
-   c1, c2 the bias corrections 1/(1 - beta^t)) and the new FP16 operands. */
-__global__ void mlpUpdate(float* __restrict__ master, float* __restrict__ m1, float* __restrict__ m2,
-        const float* __restrict__ partials, int chunks, float invCount, float lr, float c1, float c2,
-        MlpDevice* __restrict__ d, float* __restrict__ gradOut, int apply) {
+/* The gradient g (summed over the chunks) of parameter p / count; with apply, one Adam step (beta 0.9, 0.999, eps 1e-8; c1,
+   c2 the bias corrections 1/(1 - beta^t)) and the new FP16 operands. */
+struct UpdateArgs {
+    float *master, *m1, *m2;
+    float invCount, lr, c1, c2;
+    MlpDevice* dev;
+    float* gradOut;
+    int apply;
+};
+
+__device__ __forceinline__ void updateParameter(const UpdateArgs& u, int p, float g) {
+    g *= u.invCount;
+    if (u.gradOut)
+        u.gradOut[p] = g;
+    if (!u.apply)
+        return;
+    float mm = 0.9f*u.m1[p] + 0.1f*g;
+    float vv = 0.999f*u.m2[p] + 0.001f*g*g;
+    u.m1[p] = mm;
+    u.m2[p] = vv;
+    float w = u.master[p] - u.lr*(mm*u.c1)/(sqrtf(vv*u.c2) + 1e-8f);
+    u.master[p] = w;
+    storeOperand(u.dev, p, w);
+}
+
+/*
+ * Weight gradients and update, one work-group per 16 x 16 tile of dW = P^T Q (P the layer input X, H1, H2; Q the layer error
+ * dZ1, dZ2, dY): wave w forms the tile over the 256 rows of chunk w, w + GRAD_WAVES, ..., and for the first row tile the bias
+ * gradient (column sums of Q); the chunks are summed in their order and the parameters updated (updateParameter), which
+ * nothing else in this launch reads.  All loads of a chunk are in flight at once (their latency is what bounds it): with a
+ * minibatch of 2,048 rows 10.5 us, where partial sums from 8 two-byte gathers per MFMA took 24.1 us and their sum and update
+ * 4.8 us in a launch of its own.  Many chunks (above GRAD_ONE_LAUNCH) take blockIdx.y work-groups per tile, each of which
+ * leaves its chunks' tiles in partials[chunk][parameter] for mlpUpdate.
+ */
+__global__ void __launch_bounds__(64*GRAD_WAVES) mlpGradUpdate(TrainActivations act, int chunks, UpdateArgs u,
+        float* __restrict__ partials) {
+    __shared__ float part[GRAD_WAVES][256 + 16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, job = blockIdx.x;
+    const int row = lane & 15, quad = (lane >> 4)*4;
+    const _Float16 *P, *Q;
+    int pw, qw, ti, to, offW, offB, width;
+    if (job < 24) {
+        P = act.X; pw = MLP_IN_PAD; Q = act.dZ1; qw = MLP_H; ti = job/4; to = job % 4;
+        offW = MLP_OFF_W1; offB = MLP_OFF_B1; width = MLP_H;
+    }
+    else if (job < 40) {
+        P = act.H1; pw = MLP_H; Q = act.dZ2; qw = MLP_H; ti = (job - 24)/4; to = (job - 24) % 4;
+        offW = MLP_OFF_W2; offB = MLP_OFF_B2; width = MLP_H;
+    }
+    else {
+        P = act.H2; pw = MLP_H; Q = act.dY; qw = MLP_OUT_PAD; ti = job - 40; to = 0;
+        offW = MLP_OFF_W3; offB = MLP_OFF_B3; width = MLP_OUT_PAD;
+    }
+    // The sum over the chunks: thread p < 256 of weight (16 ti + p/16, 16 to + p % 16), thread 256 + o of bias 16 to + o.
+    const int p = threadIdx.x;
+    int index = -1;
+    if (p < 256)
+        index = offW + (16*ti + p/16)*width + 16*to + p % 16;
+    else if (p < 256 + 16 && ti == 0)
+        index = offB + 16*to + p - 256;
+    float g = 0;
+    for (int first = (int) blockIdx.y*GRAD_WAVES; first < chunks; first += (int) gridDim.y*GRAD_WAVES) {
+        const int chunk = first + wave;
+        if (chunk < chunks) {
+            const _Float16* pt = P + ((size_t) chunk*pw + 16*ti + row)*CHUNK + quad;
+            const _Float16* qt = Q + ((size_t) chunk*qw + 16*to + row)*CHUNK + quad;
+            half4_t pa[CHUNK/16], qb[CHUNK/16];
+#pragma unroll
+            for (int k = 0; k < CHUNK/16; k++) {
+                pa[k] = load4(pt + 16*k);
+                qb[k] = load4(qt + 16*k);
+            }
+            float4_t acc = {0, 0, 0, 0};
+            float bsum = 0;
+#pragma unroll
+            for (int k = 0; k < CHUNK/16; k++) {
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    bsum += (float) qb[k][e];
+                acc = mfma16(pa[k], qb[k], acc);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                part[wave][16*(quad + r) + row] = acc[r];
+            bsum += __shfl_xor(bsum, 16);
+            bsum += __shfl_xor(bsum, 32);
+            if (lane < 16)
+                part[wave][256 + lane] = bsum;
+        }
+        __syncthreads();
+        if (index >= 0)
+            for (int w = 0; w < GRAD_WAVES && first + w < chunks; w++) {
+                if (partials != nullptr)
+                    partials[(size_t) (first + w)*MLP_PARAMS + index] = part[w][p];
+                g += part[w][p];
+            }
+        __syncthreads();
+    }
+    if (index >= 0 && partials == nullptr)
+        updateParameter(u, index, g);
+}
+
+/* The chunks' partial sums in their order, and the update. */
+__global__ void mlpUpdate(const float* __restrict__ partials, int chunks, UpdateArgs u) {
     int p = blockIdx.x*blockDim.x + threadIdx.x;
     if (p >= MLP_PARAMS)
         return;
     float g = 0;
     for (int c = 0; c < chunks; c++)
         g += partials[(size_t) c*MLP_PARAMS + p];
-    g *= invCount;
-    if (gradOut)
-        gradOut[p] = g;
-    if (!apply)
-        return;
-    float mm = 0.9f*m1[p] + 0.1f*g;
-    float vv = 0.999f*m2[p] + 0.001f*g*g;
-    m1[p] = mm;
-    m2[p] = vv;
-    float w = master[p] - lr*(mm*c1)/(sqrtf(vv*c2) + 1e-8f);
-    master[p] = w;
-    storeOperand(d, p, w);
+    updateParameter(u, p, g);
 }
 
 /* Raw pairs -> normalized FP16 inputs [n][96] and normalized FP32 targets [n][3]. */
@@ -460,25 +548,30 @@ namespace {
 
 /* Minibatch buffers of the training kernels, for up to `rows` rows (a multiple of CHUNK). */
 struct TrainBuffers {
-    int capacity = 0;
-    _Float16 *H1 = nullptr, *H2 = nullptr, *dZ1 = nullptr, *dZ2 = nullptr, *dY = nullptr;
-    float* partials = nullptr;
+    _Float16* halves = nullptr;
+    TrainActivations act{};
+    float* partials = nullptr;        // above GRAD_ONE_LAUNCH chunks
     double* loss = nullptr;
     void allocate(int rows) {
-        capacity = rows;
-        H1 = deviceAlloc<_Float16>((size_t) rows*MLP_H);
-        H2 = deviceAlloc<_Float16>((size_t) rows*MLP_H);
-        dZ1 = deviceAlloc<_Float16>((size_t) rows*MLP_H);
-        dZ2 = deviceAlloc<_Float16>((size_t) rows*MLP_H);
-        dY = deviceAlloc<_Float16>((size_t) rows*MLP_OUT_PAD);
-        partials = deviceAlloc<float>((size_t) (rows/CHUNK)*MLP_PARAMS);
+        const size_t n = (size_t) rows;
+        halves = deviceAlloc<_Float16>(n*(MLP_IN_PAD + 4*MLP_H + MLP_OUT_PAD));
+        act.X = halves;
+        act.H1 = act.X + n*MLP_IN_PAD;
+        act.H2 = act.H1 + n*MLP_H;
+        act.dZ1 = act.H2 + n*MLP_H;
+        act.dZ2 = act.dZ1 + n*MLP_H;
+        act.dY = act.dZ2 + n*MLP_H;
+        if (rows/CHUNK > GRAD_ONE_LAUNCH)
+            partials = deviceAlloc<float>((size_t) (rows/CHUNK)*MLP_PARAMS);
         loss = deviceAlloc<double>(1);
     }
     ~TrainBuffers() {
-        void* all[] = {H1, H2, dZ1, dZ2, dY, partials, loss};
-        for (void* p : all)
-            if (p)
-                (void) hipFree(p);
+        if (halves)
+            (void) hipFree(halves);
+        if (partials)
+            (void) hipFree(partials);
+        if (loss)
+            (void) hipFree(loss);
     }
 };
 
@@ -523,19 +616,19 @@ struct Dataset {
 void minibatch(lbm_mlp* m, const Dataset& data, const int* rows, int count, TrainBuffers& buf, bool apply, float lr,
         float* gradOut) {
     int chunks = (count + CHUNK - 1)/CHUNK;
-    int tiles = chunks*(CHUNK/16);
-    mlpTrainForward<<<blocksFor(tiles, WAVES), 64*WAVES, 0, m->stream>>>(m->dev, data.X, data.T, rows, count, tiles,
-            buf.H1, buf.H2, buf.dZ1, buf.dZ2, buf.dY, buf.loss);
-    mlpWeightGrad<<<blocksFor((int64_t) chunks*GRAD_JOBS, WAVES), 64*WAVES, 0, m->stream>>>(data.X, rows, buf.H1, buf.H2,
-            buf.dZ1, buf.dZ2, buf.dY, chunks, buf.partials);
+    mlpTrainForward<<<chunks*(CHUNK/16), 64*WAVES, 0, m->stream>>>(m->dev, data.X, data.T, rows, count, buf.act, buf.loss);
     float c1 = 1.0f, c2 = 1.0f;
     if (apply) {
         m->adamStep++;
         c1 = (float) (1.0/(1.0 - std::pow(0.9, (double) m->adamStep)));
         c2 = (float) (1.0/(1.0 - std::pow(0.999, (double) m->adamStep)));
     }
-    mlpUpdate<<<blocksFor(MLP_PARAMS, 256), 256, 0, m->stream>>>(m->master, m->mom1, m->mom2, buf.partials, chunks,
-            1.0f/count, lr, c1, c2, m->dev, gradOut, apply ? 1 : 0);
+    const UpdateArgs u = {m->master, m->mom1, m->mom2, 1.0f/count, lr, c1, c2, m->dev, gradOut, apply ? 1 : 0};
+    const bool split = chunks > GRAD_ONE_LAUNCH;
+    const unsigned groups = split ? blocksFor(chunks, GRAD_WAVES) : 1u;
+    mlpGradUpdate<<<dim3(GRAD_JOBS, groups), 64*GRAD_WAVES, 0, m->stream>>>(buf.act, chunks, u, split ? buf.partials : nullptr);
+    if (split)
+        mlpUpdate<<<blocksFor(MLP_PARAMS, 256), 256, 0, m->stream>>>(buf.partials, chunks, u);
     hipCheck(hipGetLastError(), "training launch");
 }
 

@@ -1,12 +1,19 @@
 """Kernels and dispatch branches at the sizes where they can go wrong, against the FP64 oracle or the path that they
 replace."""
+import os
+import sys
+
 import numpy as np
 import pytest
 
 from lbm_amd import LBMForce
+from lbm_amd.closure import MLPClosure, NUM_INPUTS
 from lbm_amd.harness import DeviceParticles
 import oracle_lib
 from parity import Setup, lockstep
+
+sys.path.insert(0, os.path.join(oracle_lib.ROOT, "oracle"))
+import mlp_oracle as mo  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
@@ -86,3 +93,20 @@ def test_row_chunks_match_the_oracle(nx, storage, tolerance):
     s.configure.append(conf)
     worst, _, _ = lockstep(s, 12, check_every=4, storage=storage)
     assert max(worst.values()) <= tolerance, worst
+
+
+@pytest.mark.parametrize("rows", [1, 16, 17, 255, 256, 257, 8192, 8193])
+def test_gradients_at_chunk_edges_match_the_oracle(rows):
+    """Minibatches at the edges of the tiles of 16 rows, the chunks of 256 and the 32 chunks up to which one launch sums and
+    updates (the tolerance of the gradients' parity test: FP16 operands, 2e-2 of a block's norm)."""
+    rng = np.random.default_rng(rows)
+    net = MLPClosure(seed=7)
+    net.setNormalization(u_scale=50.0, v_scale=20.0, out_scale=40.0, u_bound=1e3, v_bound=1e3)
+    raw = rng.normal(scale=0.02, size=(rows, NUM_INPUTS)).astype(np.float32)
+    target = rng.normal(scale=0.02, size=(rows, 3)).astype(np.float32)
+    g, loss = net.gradients(raw, target)
+    params = net.getParameters().astype(np.float64)
+    x = mo.normalize(raw.astype(np.float64), 50.0, 20.0)
+    ref = mo.backward(params, x, target.astype(np.float64)*40.0, emulate16=True)
+    assert abs(loss - mo.loss(params, x, target.astype(np.float64)*40.0, emulate16=True)) <= 1e-3*loss
+    assert np.linalg.norm(g - ref) <= 2e-2*np.linalg.norm(ref)
