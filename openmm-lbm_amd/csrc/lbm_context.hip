@@ -139,12 +139,7 @@ struct lbm_context {
     double* stageVel = nullptr;
     // Learned closure (include/lbm_amd_closure.h): the network and its per-particle buffers.
     lbm_mlp* closure = nullptr;
-    _Float16* closureX = nullptr;             // normalized inputs [n][96]
-    uint32_t* closureNode = nullptr;          // nearest node
-    double* closureU = nullptr;               // u(nearest), lattice units
-    float* closureDu = nullptr;               // network output
     uint8_t* closureOod = nullptr;            // out-of-distribution flags
-    uint8_t* closureFrame = nullptr;          // each particle's frame (reflections and axis order of its inputs)
     unsigned long long* closureCounters = nullptr;   // couplings through the network / the fallback
     double* closureField = nullptr;           // node velocities [node][3], when the particles are dense
     // Centred drag: its solver state and the other forces of the host path.
@@ -361,15 +356,12 @@ void couple(lbm_context* c, const double* dPos, const double* dVel, const double
         ClosureNorm norm = mlpClosureNorm(c->closure);
         if (c->closureField != nullptr)
             launchClosureField(c->p.storage, c->popA, c->mask, c->ucm, a, c->closureField, c->stream);
-        launchClosureFeatures(c->p.storage, c->popA, c->mask, dPos, dVel, c->particles, c->ucm, a, norm,
-                c->closureField, c->closureX, nullptr, c->closureNode, c->closureU, c->closureOod, c->closureFrame,
-                c->stream);
-        launchMlpInfer(mlpDeviceWeights(c->closure), c->closureX, c->numParticles, norm.outScale, c->closureDu,
-                c->stream);
-        launchClosureCouple(dVel, c->particles, c->mass, a, c->closureNode, c->closureU, c->closureDu, c->closureOod,
-                c->closureFrame, c->particleForce, c->reactionFixed, c->touched, c->closureCounters, c->stream);
+        launchClosureStep(c->p.storage, c->popA, c->mask, dPos, dVel, c->particles, c->mass, c->ucm, a, norm,
+                mlpDeviceWeights(c->closure), c->closureField, c->closureOod, c->particleForce, c->forceTarget,
+                c->reactionFixed, c->touched, c->closureCounters, c->stream);
         launchClosureFallback(c->p.storage, c->popA, c->mask, dPos, dVel, c->particles, c->mass, c->ucm, a,
-                c->closureOod, c->particleForce, c->reactionFixed, c->touched, partials, c->stream);
+                c->closureOod, c->particleForce, c->forceTarget, c->reactionFixed, c->touched, partials, c->stream);
+        c->forcesAdded = c->forceTarget != nullptr;
         return;
     }
     const SpreadBins* bins = nullptr;
@@ -526,8 +518,8 @@ void destroy(lbm_context* c) {
                        c->overflow, c->binCounts[0], c->binCounts[1], c->binSpilled, c->bins.beads, c->bins.anchor, c->bins.force,
                        c->bins.slotWeight, c->momentField, c->axisStencils,
                        c->ucm, c->wallPartials, c->particles, c->mass, c->particleForce, c->reactionFixed,
-                       c->touched, c->nextTouched, c->stagePos, c->stageVel, c->closureX, c->closureNode, c->closureU, c->closureDu,
-                       c->closureOod, c->closureFrame, c->closureCounters, c->closureField, c->stageForce};
+                       c->touched, c->nextTouched, c->stagePos, c->stageVel,
+                       c->closureOod, c->closureCounters, c->closureField, c->stageForce};
     for (void* b : buffers)
         if (b)
             (void) hipFree(b);
@@ -1200,8 +1192,7 @@ int lbm_closure_pairs(lbm_context* c, const double* positions, const double* vel
         uint8_t* ood = deviceAlloc<uint8_t>(n);
         uint8_t* frame = deviceAlloc<uint8_t>(n);
         float* t = deviceAlloc<float>(3*(size_t) n);
-        launchClosureFeatures(c->p.storage, c->popA, c->mask, c->stagePos, c->stageVel, c->particles, c->ucm, a, norm,
-                nullptr, X, raw, node, u, ood, frame, c->stream);
+        launchClosureFeatures(c->p.storage, c->popA, c->mask, c->stagePos, c->stageVel, c->particles, c->ucm, a, norm, X, raw, node, u, ood, frame, c->stream);
         launchClosureTargets(c->p.storage, c->popA, c->mask, c->stagePos, c->particles, c->ucm, a, u, frame, t,
                 c->stream);
         hipError_t e = hipGetLastError();
@@ -1226,20 +1217,15 @@ int lbm_set_closure(lbm_context* c, lbm_mlp* mlp) {
             if (c->p.drag_scheme != LBM_DRAG_EXPLICIT)
                 throw Error(LBM_ERROR_UNSUPPORTED, "lbm_set_closure: the closure corrects the explicit drag only");
             size_t n = (size_t) std::max(c->numParticles, 1);
-            if (c->closureX == nullptr) {
-                c->closureX = deviceAlloc<_Float16>(n*MLP_IN_PAD);
-                c->closureNode = deviceAlloc<uint32_t>(n);
-                c->closureU = deviceAlloc<double>(3*n);
-                c->closureDu = deviceAlloc<float>(3*n);
-                c->closureOod = deviceAlloc<uint8_t>(n);
-                c->closureFrame = deviceAlloc<uint8_t>(n);
-                const size_t counters = 2*(size_t) closureCoupleBlocks(c->numParticles);
-                c->closureCounters = deviceAlloc<unsigned long long>(counters);
-                HIP_CHECK(hipMemsetAsync(c->closureCounters, 0, counters*sizeof(unsigned long long), c->stream));
-            }
             // Dense particles (more neighbourhood nodes than lattice nodes): one velocity pass over the lattice.
             if (c->closureField == nullptr && 27*(int64_t) c->numParticles >= (int64_t) c->g.n)
                 c->closureField = deviceAlloc<double>(3*(size_t) c->g.n);
+            if (c->closureOod == nullptr) {
+                c->closureOod = deviceAlloc<uint8_t>(n);
+                const size_t counters = 2*(size_t) closureStepBlocks(c->numParticles, c->closureField != nullptr);
+                c->closureCounters = deviceAlloc<unsigned long long>(counters);
+                HIP_CHECK(hipMemsetAsync(c->closureCounters, 0, counters*sizeof(unsigned long long), c->stream));
+            }
         }
         HIP_CHECK(hipStreamSynchronize(c->stream));
         c->closure = mlp;
@@ -1253,7 +1239,8 @@ int lbm_closure_stats(lbm_context* c, int64_t* network, int64_t* fallback) {
         unsigned long long counts[2] = {0, 0};
         if (c->closureCounters != nullptr) {
             // Two counts per work-group of the closure coupling, summed here.
-            std::vector<unsigned long long> blocks(2*(size_t) closureCoupleBlocks(c->numParticles));
+            std::vector<unsigned long long> blocks(2*(size_t) closureStepBlocks(c->numParticles,
+                    c->closureField != nullptr));
             const size_t bytes = blocks.size()*sizeof(unsigned long long);
             HIP_CHECK(hipMemcpyAsync(blocks.data(), c->closureCounters, bytes, hipMemcpyDeviceToHost, c->stream));
             HIP_CHECK(hipMemsetAsync(c->closureCounters, 0, bytes, c->stream));

@@ -636,10 +636,10 @@ __device__ __forceinline__ void coupleGroup(const S* __restrict__ src, const uin
         const double* x, const double* vel, uint32_t index, double m, bool active, int lane,
         const double* __restrict__ ucm, const ParticleArgs& a, double* forceOut,
         unsigned long long* __restrict__ reactionFixed, uint32_t* __restrict__ touched, double wallAcc[3],
-        const double* noise = nullptr) {
+        const double* noise = nullptr, double* systemForce = nullptr) {
     double u[3];
     StencilSlot sl = interpolateGroup<S, LANES>(src, mask, x, active, lane, ucm, a, u);
-    finishGroup<LANES>(sl, u, vel, index, m, active, lane, a, forceOut, reactionFixed, touched, wallAcc, noise);
+    finishGroup<LANES>(sl, u, vel, index, m, active, lane, a, forceOut, reactionFixed, touched, wallAcc, noise, systemForce);
 }
 
 }  // namespace lbm

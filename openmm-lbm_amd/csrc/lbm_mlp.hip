@@ -34,9 +34,6 @@ using namespace lbm;
 
 namespace {
 
-typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-typedef float float4_t __attribute__((ext_vector_type(4)));
-
 constexpr int WAVES = 4;                 // waves per work-group of the network kernels
 constexpr int CHUNK = 256;               // particles per partial sum of the weight gradients
 constexpr int GRAD_JOBS = 24 + 16 + 4;   // 16 x 16 tiles of dW1, dW2, dW3
@@ -44,25 +41,9 @@ constexpr int GRAD_WAVES = 8;            // chunks that a work-group of the weig
 // Chunks up to which one work-group per tile takes them all and updates the parameters (minibatches of up to 8,192 rows).
 constexpr int GRAD_ONE_LAUNCH = 32;
 
-__device__ __forceinline__ float4_t mfma16(half4_t a, half4_t b, float4_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0);
-}
-
-__device__ __forceinline__ float siluf(float z) {
-    return z/(1.0f + __expf(-z));
-}
-
 __device__ __forceinline__ float dsiluf(float z) {
     float s = 1.0f/(1.0f + __expf(-z));
     return s*(1.0f + z*(1.0f - s));
-}
-
-__device__ __forceinline__ half4_t load4(const _Float16* p) {
-    return *(const half4_t*) p;
-}
-
-__device__ __forceinline__ void store4(_Float16* p, half4_t v) {
-    *(half4_t*) p = v;
 }
 
 struct ForwardWeights {
@@ -170,13 +151,6 @@ __device__ __forceinline__ void storeTransposed(_Float16* out, int units, int b,
 #pragma unroll
     for (int r = 0; r < 4; r++)
         p[r*CHUNK] = v[r];
-}
-
-/* v rounded to FP32 and then to FP16 (a product and its conversion would otherwise be fused, with one rounding, or not, as
-   the compiler sees fit). */
-__device__ __forceinline__ _Float16 toHalf(float v) {
-    asm("" : "+v"(v));
-    return (_Float16) v;
 }
 
 /*

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from lbm_amd import LBMForce
-from lbm_amd.closure import MLPClosure, NUM_INPUTS
+from lbm_amd.closure import MLPClosure, NUM_INPUTS, stats
 from lbm_amd.harness import DeviceParticles
 import oracle_lib
 from parity import Setup, lockstep
@@ -110,3 +110,41 @@ def test_gradients_at_chunk_edges_match_the_oracle(rows):
     ref = mo.backward(params, x, target.astype(np.float64)*40.0, emulate16=True)
     assert abs(loss - mo.loss(params, x, target.astype(np.float64)*40.0, emulate16=True)) <= 1e-3*loss
     assert np.linalg.norm(g - ref) <= 2e-2*np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("n,beads", [(24, 1), (24, 15), (24, 17), (24, 511), (24, 513), (32, 40000)],
+                         ids=["1", "15", "17", "511-pulled", "513-field", "40000-field-per-wave"])
+def test_closure_step_with_a_zero_network_is_the_nearest_coupling(n, beads):
+    """Every path of the closure's step (nodes pulled, from a velocity field, tiles shared by a work-group or one per wave)
+    at the edges of its tiles of 16 beads: with all parameters zero the correction is zero and the run is the nearest-node
+    coupling's, bit for bit, between walls and with bounds that no bead exceeds; beads near the walls fall back."""
+    rng = np.random.default_rng(beads)
+    pos = rng.uniform([0, 0, 4], [n, n, n - 5], size=(beads, 3))
+    vel = rng.normal(scale=0.2, size=(beads, 3))
+    results = []
+    for stencil in (LBMForce.Keys, LBMForce.NearestNode):
+        s = Setup((n, n, n), tau=0.7)
+        s.add_particles(pos, velocities=vel)
+
+        def conf(f, stencil=stencil):
+            f.setSolidNodes([i for k in (0, n - 1) for i in range(k*n*n, (k + 1)*n*n)])
+            f.setWallScheme(LBMForce.BounceBack)
+            f.setFriction(10.0)
+            f.setTemperature(300.0)
+            f.setFluidFluctuations(True)
+            f.setRandomNumberSeed(11)
+            f.setInterpolationStencil(stencil)
+        s.configure.append(conf)
+        ctx = s.build()
+        if stencil == LBMForce.Keys:
+            net = MLPClosure(seed=1)
+            net.setParameters(np.zeros(11408))
+            net.attach(ctx)
+        dp = DeviceParticles(ctx)
+        dp.step(5)
+        out = dp.pull()
+        results.append((out[0], out[1], ctx.getFluidState()))
+        if stencil == LBMForce.Keys:
+            assert stats(ctx) == (5*beads, 0)
+    for a, b in zip(*results):
+        assert np.array_equal(a, b)
