@@ -378,7 +378,7 @@ void couple(lbm_context* c, const double* dPos, const double* dVel, const double
                 c->stream);
     else if (c->axisStencils != nullptr)
         launchStencilSetup(dPos, c->particles, a, c->axisStencils, c->stream);
-    launchCouple(c->p.storage, c->popA, c->mask, dPos, dVel, c->particles, order, c->mass, c->ucm, a, c->particleForce,
+    launchCouple(c->p.storage, c->popA, c->mask, dPos, dVel, c->identityParticles ? nullptr : c->particles, order, c->mass, c->ucm, a, c->particleForce,
             c->reactionFixed, c->touched, partials, c->forceTarget, bins, c->momentField, c->axisStencils, c->stream);
     if (bins != nullptr)
         launchSpreadTiles(dPos, c->particles, c->mask, a, *bins, c->reactionFixed, c->touched, c->stream);
@@ -670,10 +670,14 @@ void create(const lbm_params* params, const int* solid, int numSolid, const int*
         try {
             if (p.drag_scheme == LBM_DRAG_CENTERED)
                 c->centred = centredCreate(numParts, p.interpolation_stencil, (uint32_t) n);
-            if (p.drag_scheme == LBM_DRAG_CENTERED ? c->dense && p.interpolation_stencil != LBM_STENCIL_NEAREST : !c->dense)
-                // Sparse particles gain DRAM locality from the node order; dense ones would contend for the same
-                // accumulators when neighbours are processed together (measured: 100,000 chain beads with Keys on
-                // 128^3 couple 6% slower in node order), so they keep the index order.
+            if (p.drag_scheme == LBM_DRAG_CENTERED ? c->dense && p.interpolation_stencil != LBM_STENCIL_NEAREST :
+                    !c->dense && numParts > 2048)
+                // Sparse particles gain DRAM locality from the node order (a step of 8,000 Keys beads in 128^3 127 -> 119
+                // us, of 3,000 in 96^3 43.0 -> 41.4); up to 2,048 it gains nothing and costs a load in the coupling's chain
+                // and the sort.  Dense particles of the explicit drag would contend for the same accumulators when
+                // neighbours are processed together (measured: 100,000 chain beads with Keys on 128^3 couple 6% slower
+                // in node order), so they keep the index order; the solver of the centred drag gathers more than it
+                // spreads and takes it.
                 c->order = coupleOrderCreate(numParts, (uint32_t) n);
         }
         catch (const std::runtime_error& e) {
@@ -1192,7 +1196,8 @@ int lbm_closure_pairs(lbm_context* c, const double* positions, const double* vel
         uint8_t* ood = deviceAlloc<uint8_t>(n);
         uint8_t* frame = deviceAlloc<uint8_t>(n);
         float* t = deviceAlloc<float>(3*(size_t) n);
-        launchClosureFeatures(c->p.storage, c->popA, c->mask, c->stagePos, c->stageVel, c->particles, c->ucm, a, norm, X, raw, node, u, ood, frame, c->stream);
+        launchClosureFeatures(c->p.storage, c->popA, c->mask, c->stagePos, c->stageVel, c->particles, c->ucm, a, norm, X,
+                raw, node, u, ood, frame, c->stream);
         launchClosureTargets(c->p.storage, c->popA, c->mask, c->stagePos, c->particles, c->ucm, a, u, frame, t,
                 c->stream);
         hipError_t e = hipGetLastError();

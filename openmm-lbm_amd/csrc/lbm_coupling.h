@@ -167,7 +167,7 @@ __device__ __forceinline__ void axisSlot(double s, int n, bool open, int sub, in
         int first = STENCIL == LBM_STENCIL_THREE_POINT ? (int) floor(s + 0.5) - 1 :
                     STENCIL == LBM_STENCIL_KEYS ? (int) floor(s) - 1 : (int) floor(s);
         bool merged = open ? (first < 0 || first + w > n) : n < w;
-        if (!merged) {
+        if (__builtin_expect(!merged, 1)) {
             int i = first + sub;
             weight = stencilKernel(STENCIL, s - (double) i);
             index = open ? i : (i < 0 ? i + n : (i >= n ? i - n : i));
@@ -196,12 +196,10 @@ struct StencilSlot {
 
 /* rho and j (with j -= rho u_cm when the removal is due) of one node from its pulled populations, FP64. */
 template <typename S>
-__device__ __forceinline__ double nodeMoments(const S* __restrict__ src, const Geometry& g, uint32_t node,
-        const double* __restrict__ ucm, int removal, double j[3]) {
-    uint32_t ni, nj, nk;
-    nodeCoords(g, node, ni, nj, nk);
+__device__ __forceinline__ double momentsAt(const S* __restrict__ src, const Geometry& g, uint32_t ni, uint32_t nj,
+        uint32_t nk, const double* __restrict__ ucm, int removal, double j[3]) {
     typename StorageTraits<S>::Real f[NQ];
-    pullNode(src, g, node, ni, nj, nk, f);
+    pullNode(src, g, 0u, ni, nj, nk, f);
     double dr = 0, jx = 0, jy = 0, jz = 0;
     staticFor<NQ>([&](auto I) {
         constexpr int q = decltype(I)::value;
@@ -221,6 +219,14 @@ __device__ __forceinline__ double nodeMoments(const S* __restrict__ src, const G
     j[1] = jy;
     j[2] = jz;
     return rho;
+}
+
+template <typename S>
+__device__ __forceinline__ double nodeMoments(const S* __restrict__ src, const Geometry& g, uint32_t node,
+        const double* __restrict__ ucm, int removal, double j[3]) {
+    uint32_t ni, nj, nk;
+    nodeCoords(g, node, ni, nj, nk);
+    return momentsAt(src, g, ni, nj, nk, ucm, removal, j);
 }
 
 /* The fluid velocity of one node as the coupling sees it (computeMoments): u = j/rho of the pulled populations, with
@@ -249,18 +255,6 @@ __device__ __forceinline__ void momentFieldNode(const S* __restrict__ src, const
     double j[3];
     double rho = nodeMoments(src, g, node, ucm, removal, j);
     field[node] = make_double4(j[0], j[1], j[2], rho);
-}
-
-/* nodeVelocity from the moment field: the same arithmetic on the same moments, so the same bits. */
-__device__ __forceinline__ void fieldVelocity(const double4* __restrict__ field, uint32_t node, double weight,
-        double u[3]) {
-    const double4 m = field[node];
-    u[0] = u[1] = u[2] = 0.0;
-    if (m.w > 0) {
-        u[0] = m.x*(weight/m.w);
-        u[1] = m.y*(weight/m.w);
-        u[2] = m.z*(weight/m.w);
-    }
 }
 
 /* v of the lane that the DPP control CTRL pairs with this one (every lane of the wavefront active). */
@@ -305,53 +299,83 @@ __device__ __forceinline__ double groupSum(double v) {
 
 /*
  * The interpolated fluid velocity u(X) of one particle by a group of LANES lanes, one lane per slot of the stencil
- * a.stencil (every lane of the group calls it, inactive ones with active = false): each lane forms w_j u_j of its node
+ * a.stencil (every lane of the wavefront calls it, inactive ones with active = false): each lane forms w_j u_j of its node
  * (zero at solid nodes, whose rho is 0 in computeMoments) and the group sums them; every lane returns the sum in u and
- * its own slot.
+ * its own slot.  x: the particle's position in memory.
+ *
+ * The group's first 3w lanes each form one slot along one axis (axisSlot) and the lanes fetch their three: a third of the
+ * FP64 instructions that every lane forming its own three took, and of their code.  What bounds this: with few particles
+ * the chain of loads and the fetch of the code (64 trilinear beads 11.6 -> 10.6 us, 110 nearest ones 8.7 -> 8.4, 3,001
+ * three-point ones 18.7 -> 16.2), with many and the nodes from the moment field the instructions (100,000 Keys beads
+ * 97 -> 74 us), with many and the nodes pulled the 128 B lines of the populations (100,000 Keys beads in 256^3 158 us).
  */
 template <typename S, int LANES>
 __device__ __forceinline__ StencilSlot interpolateGroup(const S* __restrict__ src, const uint32_t* __restrict__ mask,
-        const double* x, bool active, int lane, const double* __restrict__ ucm, const ParticleArgs& a, double u[3],
+        const double* __restrict__ x, bool active, int lane, const double* __restrict__ ucm, const ParticleArgs& a, double u[3],
         const double4* __restrict__ field = nullptr, const AxisStencil* __restrict__ pre = nullptr) {
     constexpr int STENCIL = groupStencil<LANES>();
     constexpr int w = STENCIL == LBM_STENCIL_KEYS ? 4 : STENCIL == LBM_STENCIL_THREE_POINT ? 3 :
                       STENCIL == LBM_STENCIL_TRILINEAR ? 2 : 1;
-    int slot = lane;
+    const int slot = lane;
     StencilSlot sl;
     sl.inStencil = active && slot < w*w*w;
-    sl.weight = 0.0;
-    sl.node = 0;
-    int size[3] = {(int) a.g.nx, (int) a.g.ny, (int) a.g.nz};
-    int openAxis[3] = {a.g.openX, a.g.openY, a.g.openZ};
-    if (sl.inStencil) {
-        int sub[3] = {slot % w, (slot/w) % w, slot/(w*w)};
-        int nodeIdx[3];
-        sl.weight = 1.0;
-        for (int k = 0; k < 3; k++) {
-            double wk;
-            if (pre != nullptr) {
-                // The particle's stencil as stencilSetup formed it: the same axisSlot values.
-                nodeIdx[k] = pre->index[k][sub[k]];
-                wk = pre->weight[k][sub[k]];
-            }
-            else
-                axisSlot<STENCIL>(wrapCoordinate(x[k], a.dx, size[k]), size[k], openAxis[k] != 0, sub[k], nodeIdx[k],
-                        wk);
-            sl.weight *= wk;
-        }
-        sl.node = (uint32_t) (nodeIdx[0] + (int) a.g.nx*(nodeIdx[1] + (int) a.g.ny*nodeIdx[2]));
+    const int nx = (int) a.g.nx, ny = (int) a.g.ny, nz = (int) a.g.nz;
+    const int openX = a.g.openX, openY = a.g.openY, openZ = a.g.openZ;
+    int idx[3];
+    if constexpr (LANES == 1) {
+        sl.weight = active ? 1.0 : 0.0;
+        idx[0] = nearestIndex(wrapCoordinate(x[0], a.dx, nx), nx);
+        idx[1] = nearestIndex(wrapCoordinate(x[1], a.dx, ny), ny);
+        idx[2] = nearestIndex(wrapCoordinate(x[2], a.dx, nz), nz);
     }
+    else {
+        const int sub[3] = {slot % w, (slot/w) % w, min(slot/(w*w), w - 1)};
+        double wk[3];
+        if (pre != nullptr) {
+            // The particle's stencil as stencilSetup formed it: the same axisSlot values.
+            for (int k = 0; k < 3; k++) {
+                idx[k] = pre->index[k][sub[k]];
+                wk[k] = pre->weight[k][sub[k]];
+            }
+        }
+        else {
+            // Selected among values, not among the fields of `a`: of a copy that a kernel changed, that would be a choice of
+            // addresses, which puts the copy in scratch memory.
+            const int axis = lane < w ? 0 : (lane < 2*w ? 1 : 2);
+            const int n = axis == 0 ? nx : (axis == 1 ? ny : nz);
+            const int open = axis == 0 ? openX : (axis == 1 ? openY : openZ);
+            int axisIndex;
+            double axisWeight;
+            axisSlot<STENCIL>(wrapCoordinate(x[axis], a.dx, n), n, open != 0, min(lane - axis*w, w - 1), axisIndex,
+                    axisWeight);
+            for (int k = 0; k < 3; k++) {
+                idx[k] = __shfl(axisIndex, k*w + sub[k], LANES);
+                wk[k] = __shfl(axisWeight, k*w + sub[k], LANES);
+            }
+        }
+        sl.weight = sl.inStencil ? wk[0]*wk[1]*wk[2] : 0.0;
+    }
+    sl.node = sl.inStencil ? (uint32_t) (idx[0] + nx*(idx[1] + ny*idx[2])) : 0u;
     sl.solid = sl.inStencil && solidAt(mask, sl.node);
     double ux = 0, uy = 0, uz = 0;
     if (sl.inStencil && !sl.solid) {
-        double un[3];
-        if (field != nullptr)
-            fieldVelocity(field, sl.node, sl.weight, un);
+        double j[3], rho;
+        if (field != nullptr) {
+            // The same moments, formed by momentField: the same bits.
+            const double4 m = field[sl.node];
+            j[0] = m.x;
+            j[1] = m.y;
+            j[2] = m.z;
+            rho = m.w;
+        }
         else
-            nodeVelocity(src, a.g, sl.node, ucm, a.removal, sl.weight, un);
-        ux = un[0];
-        uy = un[1];
-        uz = un[2];
+            rho = momentsAt(src, a.g, (uint32_t) idx[0], (uint32_t) idx[1], (uint32_t) idx[2], ucm, a.removal, j);
+        if (rho > 0) {
+            const double scale = sl.weight/rho;
+            ux = j[0]*scale;
+            uy = j[1]*scale;
+            uz = j[2]*scale;
+        }
     }
     u[0] = groupSum<LANES>(ux);
     u[1] = groupSum<LANES>(uy);
@@ -417,6 +441,60 @@ __device__ __forceinline__ void dragForce(const double* vel, const double u[3], 
     }
 }
 
+/* Component lane (its first three lanes) of a particle's velocity, for groupForce; a lone lane loads them there. */
+template <int LANES>
+__device__ __forceinline__ double groupVelocity(const double* __restrict__ vel, int lane) {
+    return LANES == 1 ? 0.0 : vel[lane < 3 ? lane : 2];
+}
+
+/*
+ * The drag force f of a group's particle, in every lane, in the terms of dragForce; the force (kJ/mol/nm) is written to
+ * forceOut and, when given, added to systemForce (atomically, in case a particle were coupled twice).  The group's first
+ * three lanes form a component each and the others fetch them.  velocity: groupVelocity; noise: the particle's normals
+ * when already drawn (particleNoise), else nullptr.  Every lane of the wavefront calls it.
+ */
+template <int LANES>
+__device__ __forceinline__ void groupForce(const double u[3], const double* vel, double velocity, uint32_t index, double m,
+        bool active, int lane, const ParticleArgs& a, double* forceOut, const double* noise, double* systemForce, double f[3]) {
+    if constexpr (LANES == 1) {
+        f[0] = f[1] = f[2] = 0.0;
+        if (!active)
+            return;
+        dragForce(vel, u, index, m, a, f, noise);
+        for (int k = 0; k < 3; k++) {
+            forceOut[k] = f[k]*a.forceScale;
+            if (systemForce != nullptr)
+                atomicAdd(systemForce + k, f[k]*a.forceScale);
+        }
+    }
+    else {
+        double own = 0.0;
+        if (active) {
+            const int k = lane < 3 ? lane : 2;
+            const double v = velocity/a.velocityScale;
+            own = (v - (k == 0 ? u[0] : (k == 1 ? u[1] : u[2])))*(-a.gamma*m);
+            if (a.randomForce) {
+                double xi;
+                if (noise != nullptr)
+                    xi = noise[k];
+                else {
+                    double drawn[4];
+                    particleNoise(index, a, drawn);
+                    xi = k == 0 ? drawn[0] : (k == 1 ? drawn[1] : drawn[2]);
+                }
+                own += xi*sqrt(2.0*a.gamma*m*a.kT);
+            }
+            if (lane < 3) {
+                forceOut[lane] = own*a.forceScale;
+                if (systemForce != nullptr)
+                    atomicAdd(systemForce + lane, own*a.forceScale);
+            }
+        }
+        for (int k = 0; k < 3; k++)
+            f[k] = __shfl(own, k, LANES);
+    }
+}
+
 /* The reaction -w F of one slot: on a fluid node into its fixed-point accumulators; on a solid node it leaves the
    fluid and goes to the wall (ReferenceLBMKernels.cpp:959-971).  Returns whether an accumulator received a nonzero
    value (the node is then flagged in the touched mask, which the fused pass reads and clears). */
@@ -474,7 +552,7 @@ struct StagedReactions {
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         const int first = (int) threadIdx.x & ~63, lane = (int) threadIdx.x & 63;
-#pragma unroll
+#pragma unroll 1
         for (int round = 0; round < 3; round++) {
             const int item = lane + 64*round;
             const int slot = a.reactionPlanes ? first + lane : first + item/3;
@@ -581,23 +659,12 @@ __device__ __forceinline__ void storeWallPartial(const double acc[3], double* __
    in a lattice step, the spread of the reaction, through the work-group's staging when given (every lane of the
    wavefront then calls it). */
 template <int LANES, int THREADS = BLOCK>
-__device__ __forceinline__ void finishGroup(const StencilSlot& sl, const double u[3], const double* vel, uint32_t index,
-        double m, bool active, int lane, const ParticleArgs& a, double* forceOut,
+__device__ __forceinline__ void finishGroup(const StencilSlot& sl, const double u[3], const double* vel, double velocity,
+        uint32_t index, double m, bool active, int lane, const ParticleArgs& a, double* forceOut,
         unsigned long long* __restrict__ reactionFixed, uint32_t* __restrict__ touched, double wallAcc[3],
         const double* noise, double* systemForce = nullptr, StagedReactions<THREADS>* staged = nullptr) {
-    // Every lane of the group holds u; each computes the force (identical values).
-    double f[3] = {0, 0, 0};
-    if (active) {
-        dragForce(vel, u, index, m, a, f, noise);
-        if (lane == 0)
-            for (int k = 0; k < 3; k++) {
-                forceOut[k] = f[k]*a.forceScale;
-                // The caller's force array, when given: one addition per coupled particle (atomic, in case a particle
-                // were coupled twice).
-                if (systemForce != nullptr)
-                    atomicAdd(systemForce + k, f[k]*a.forceScale);
-            }
-    }
+    double f[3];
+    groupForce<LANES>(u, vel, velocity, index, m, active, lane, a, forceOut, noise, systemForce, f);
     if (a.isStep) {
         bool flagged = false;
         if (staged != nullptr) {
@@ -638,8 +705,9 @@ __device__ __forceinline__ void coupleGroup(const S* __restrict__ src, const uin
         unsigned long long* __restrict__ reactionFixed, uint32_t* __restrict__ touched, double wallAcc[3],
         const double* noise = nullptr, double* systemForce = nullptr) {
     double u[3];
+    const double velocity = groupVelocity<LANES>(vel, lane);
     StencilSlot sl = interpolateGroup<S, LANES>(src, mask, x, active, lane, ucm, a, u);
-    finishGroup<LANES>(sl, u, vel, index, m, active, lane, a, forceOut, reactionFixed, touched, wallAcc, noise, systemForce);
+    finishGroup<LANES>(sl, u, vel, velocity, index, m, active, lane, a, forceOut, reactionFixed, touched, wallAcc, noise, systemForce);
 }
 
 }  // namespace lbm

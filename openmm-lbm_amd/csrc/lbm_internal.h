@@ -238,7 +238,7 @@ void launchReduceWall(const double* partials, int count, double* out, hipStream_
 /* The reflection writes its wall momentum to allPartials[3*ownOffset...] and clears the rest of allPartials[0, 3*count). */
 void launchReflect(const double* positions, double* velocities, const int* particles, const double* mass,
         const uint32_t* mask, const ParticleArgs& a, double* allPartials, int count, int ownOffset, hipStream_t stream);
-/* order: the coupled particles in the order to process them (a permutation of 0..numParticles-1), or nullptr;
+/* particles: the System's index of each coupled particle, or nullptr where it is the same; order: coupleOrderAt's, or nullptr;
    systemForces: the caller's force array [particle][3] (kJ/mol/nm) to add the coupling forces to, or nullptr. */
 void launchCouple(int storage, const void* src, const uint32_t* mask, const double* positions, const double* velocities,
         const int* particles, const int* order, const double* mass, const double* ucm, const ParticleArgs& a,
@@ -269,7 +269,8 @@ constexpr int COUPLE_ORDER_STEPS = 128;
 struct CoupleOrder;
 CoupleOrder* coupleOrderCreate(int numParticles, uint32_t numNodes);
 void coupleOrderDestroy(CoupleOrder* order);
-/* The order for a coupling at `step`, sorted anew from the positions when stale. */
+/* The order for a coupling at `step`, sorted anew from the positions when stale: a permutation of the coupled particles
+   0 .. numParticles - 1, followed by the System's index of each. */
 const int* coupleOrderAt(CoupleOrder* order, int64_t step, const double* positions, const int* particles,
         const ParticleArgs& a, hipStream_t stream);
 void launchAddForces(const double* particleForce, const int* particles, int count, double* forces, hipStream_t stream);

@@ -87,20 +87,12 @@ __device__ __forceinline__ uint32_t anchorTile(const double* x, const ParticleAr
  * are integers, so both ways give the same bits).
  */
 template <int LANES>
-__device__ __forceinline__ void finishGroupBinned(const StencilSlot& sl, const double u[3], const double* vel,
+__device__ __forceinline__ void finishGroupBinned(const StencilSlot& sl, const double u[3], const double* vel, double velocity,
         const double* x, uint32_t index, double m, bool active, int lane, const ParticleArgs& a, double* forceOut,
         unsigned long long* __restrict__ reactionFixed, uint32_t* __restrict__ touched, double wallAcc[3],
         const double* noise, double* systemForce, const SpreadBins& bins, const AxisStencil* pre) {
-    double f[3] = {0, 0, 0};
-    if (active) {
-        dragForce(vel, u, index, m, a, f, noise);
-        if (lane == 0)
-            for (int k = 0; k < 3; k++) {
-                forceOut[k] = f[k]*a.forceScale;
-                if (systemForce != nullptr)
-                    atomicAdd(systemForce + k, f[k]*a.forceScale);
-            }
-    }
+    double f[3];
+    groupForce<LANES>(u, vel, velocity, index, m, active, lane, a, forceOut, noise, systemForce, f);
     if (!a.isStep)
         return;
     int full = 0;
@@ -218,16 +210,19 @@ __global__ void __launch_bounds__(BLOCK) coupleParticles(const S* __restrict__ s
     // Sparse beads with FP16/BF16 populations: each XCD takes a contiguous run of the work-groups, so that beads near
     // in the processing order (sorted by node) share an L2 for the 128 B lines, 64 nodes wide, that they read
     // (coupled step of 256^3 with 20,000 Keys beads 0.401 -> 0.397 ms; no gain with FP32's 32-node lines).
-    const uint32_t group = (isReduced<S>() || BINNED) && a.xcdOrder ? xcdContiguousTile(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t group = isReduced<S>() && !BINNED && a.xcdOrder ? xcdContiguousTile(blockIdx.x, gridDim.x) : blockIdx.x;
     int rank = (int) group*GROUPS + threadIdx.x/LANES;    // position in the processing order
     bool active = rank < a.numParticles;
+    // The particle, through as few loads in a row as there are.  The order holds the System's index beside the coupled one;
+    // without an order or `particles` both are the rank.  What the drag needs is loaded with the position, not after the sum.
     int i = active && order != nullptr ? order[rank] : rank;
-    int part = active ? particles[i] : 0;
-    double m = active ? mass[i] : 0.0;
+    const int part = !active ? 0 : order != nullptr ? order[a.numParticles + rank] : particles != nullptr ? particles[i] : i;
+    const double* x = positions + 3*(size_t) part;
+    const double* vel = velocities + 3*(size_t) part;
+    const double m = active ? mass[i] : 0.0, velocity = groupVelocity<LANES>(vel, lane);
     double u[3];
     const AxisStencil* pre = stencils != nullptr && active ? stencils + i : nullptr;
-    StencilSlot sl = interpolateGroup<S, LANES>(src, mask, positions + 3*(size_t) part, active, lane, ucm, a, u, field,
-            pre);
+    StencilSlot sl = interpolateGroup<S, LANES>(src, mask, x, active, lane, ucm, a, u, field, pre);
     // The normals of the work-group's particles: formed with the stencils where those were formed beforehand (no
     // barrier here), else drawn by the work-group's first 4*GROUPS lanes, one normal each, instead of by every group:
     // a wavefront pays for the logarithm and cosine or sine once however many of its lanes need them.  Drawn after the
@@ -247,12 +242,12 @@ __global__ void __launch_bounds__(BLOCK) coupleParticles(const S* __restrict__ s
         myNoise = pre->normal;
     double wallAcc[3] = {0, 0, 0};
     if constexpr (BINNED)
-        finishGroupBinned<LANES>(sl, u, velocities + 3*(size_t) part, positions + 3*(size_t) part, (uint32_t) i, m, active,
-                lane, a, particleForce + 3*(size_t) (active ? i : 0), reactionFixed, touched, wallAcc, myNoise,
+        finishGroupBinned<LANES>(sl, u, vel, velocity, x, (uint32_t) i, m, active, lane, a,
+                particleForce + 3*(size_t) (active ? i : 0), reactionFixed, touched, wallAcc, myNoise,
                 systemForces != nullptr ? systemForces + 3*(size_t) part : nullptr, bins, pre);
     else {
         __shared__ StagedReactions<BLOCK> staged;
-        finishGroup<LANES, BLOCK>(sl, u, velocities + 3*(size_t) part, (uint32_t) i, m, active, lane, a,
+        finishGroup<LANES, BLOCK>(sl, u, vel, velocity, (uint32_t) i, m, active, lane, a,
                 particleForce + 3*(size_t) (active ? i : 0), reactionFixed, touched, wallAcc, myNoise,
                 systemForces != nullptr ? systemForces + 3*(size_t) part : nullptr, &staged);
     }
@@ -523,6 +518,8 @@ __global__ void __launch_bounds__(THREADS) coupleBatch(const ReplicaDesc* __rest
     a.step = *stepCounter;
     a.isStep = 1;
     const float* src = (a.step & 1) ? d->popB : d->popA;
+    const double* vel = velocities + 3*(size_t) pp;
+    const double m = active ? mass[pp] : 0.0, velocity = groupVelocity<LANES>(vel, lane);
     double u[3];
     StencilSlot sl = interpolateGroup<float, LANES>(src, nullptr, positions + 3*(size_t) pp, active, lane, nullptr, a, u);
     // The work-group's normals, drawn by its first 4*GROUPS lanes (as in coupleParticles).
@@ -538,8 +535,7 @@ __global__ void __launch_bounds__(THREADS) coupleBatch(const ReplicaDesc* __rest
     }
     double wallAcc[3] = {0, 0, 0};
     __shared__ StagedReactions<THREADS> staged;
-    finishGroup<LANES, THREADS>(sl, u, velocities + 3*(size_t) pp, (uint32_t) (pp - d->particleBegin),
-            active ? mass[pp] : 0.0, active, lane, a, forces + 3*(size_t) pp, d->reactionFixed,
+    finishGroup<LANES, THREADS>(sl, u, vel, velocity, (uint32_t) (pp - d->particleBegin), m, active, lane, a, forces + 3*(size_t) pp, d->reactionFixed,
             (a.step & 1) ? d->touchedB : d->touchedA, wallAcc, myNoise, nullptr, &staged);
 }
 
@@ -778,6 +774,13 @@ __global__ void __launch_bounds__(BLOCK) orderKeys(const double* __restrict__ po
     values[i] = i;
 }
 
+/* The System's index of each place of the order, after the order itself. */
+__global__ void __launch_bounds__(BLOCK) orderParticles(const int* __restrict__ particles, int count, int* __restrict__ order) {
+    int rank = blockIdx.x*BLOCK + threadIdx.x;
+    if (rank < count)
+        order[count + rank] = particles[order[rank]];
+}
+
 static void orderCheck(hipError_t e, const char* what) {
     if (e != hipSuccess)
         throw std::runtime_error(std::string("HIP error in the coupling order (") + what + "): " + hipGetErrorString(e));
@@ -802,7 +805,7 @@ CoupleOrder* coupleOrderCreate(int numParticles, uint32_t numNodes) {
         orderCheck(hipMalloc((void**) &o->keys, sizeof(uint32_t)*numParticles), "allocation");
         orderCheck(hipMalloc((void**) &o->sortedKeys, sizeof(uint32_t)*numParticles), "allocation");
         orderCheck(hipMalloc((void**) &o->values, sizeof(int)*numParticles), "allocation");
-        orderCheck(hipMalloc((void**) &o->order, sizeof(int)*numParticles), "allocation");
+        orderCheck(hipMalloc((void**) &o->order, 2*sizeof(int)*numParticles), "allocation");
         orderCheck(hipcub::DeviceRadixSort::SortPairs(nullptr, o->tempBytes, o->keys, o->sortedKeys, o->values, o->order,
                 numParticles, 0, o->sortBits, (hipStream_t) 0), "sort size");
         orderCheck(hipMalloc(&o->temp, std::max<size_t>(o->tempBytes, 1)), "allocation");
@@ -822,6 +825,7 @@ const int* coupleOrderAt(CoupleOrder* o, int64_t step, const double* positions, 
     size_t bytes = o->tempBytes;
     orderCheck(hipcub::DeviceRadixSort::SortPairs(o->temp, bytes, o->keys, o->sortedKeys, o->values, o->order, o->count,
             0, o->sortBits, stream), "sort");
+    orderParticles<<<gridFor(o->count), BLOCK, 0, stream>>>(particles, o->count, o->order);
     orderCheck(hipGetLastError(), "launch");
     o->sortedAt = step;
     o->valid = true;

@@ -148,3 +148,37 @@ def test_closure_step_with_a_zero_network_is_the_nearest_coupling(n, beads):
             assert stats(ctx) == (5*beads, 0)
     for a, b in zip(*results):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("stencil", [LBMForce.NearestNode, LBMForce.Trilinear, LBMForce.ThreePoint, LBMForce.Keys],
+                         ids=["nearest", "trilinear", "threepoint", "keys"])
+@pytest.mark.parametrize("grid,open_faces,beads", [((3, 2, 17), False, 37), ((6, 5, 7), True, 37), ((50, 48, 46), False, 4300)],
+                         ids=["narrower-than-the-stencil", "open-faces", "in-node-order"])
+def test_slots_of_a_group_are_those_formed_per_particle(grid, open_faces, beads, stencil, monkeypatch):
+    """The stencil slots that a group's lanes form for each other against those formed once per particle beforehand, bit for
+    bit: slots merged on narrow lattices and past open faces, and wrapped at periodic ones, with every other particle
+    coupled and a group left over in the last wavefront; enough particles for the node order in one case."""
+    rng = np.random.default_rng(beads + stencil)
+    s = Setup(grid, tau=0.8)
+    for i in range(beads):
+        s.add_particles(rng.uniform(0, grid), velocities=rng.normal(scale=0.5, size=(1, 3)), coupled=i % 2 == 0)
+
+    def conf(f):
+        if open_faces:
+            for face in range(6):
+                f.setFaceBoundary(face, LBMForce.Velocity)
+            f.setFaceVelocity(LBMForce.ZMax, (0.2, 0.1, 0))
+        f.setFriction(10.0)
+        f.setTemperature(300.0)
+        f.setRandomNumberSeed(5)
+        f.setInterpolationStencil(stencil)
+    s.configure.append(conf)
+    runs = []
+    for setup in ("0", "1"):
+        monkeypatch.setenv("LBM_AMD_STENCIL_SETUP", setup)
+        c = s.build(None, storage=LBMForce.FP32)
+        c.step(5)
+        runs.append((c.getFluidState(), c.positions.copy(), c.velocities.copy(), c.getForces()))
+    assert np.abs(runs[0][0]).max() > 0
+    for a, b in zip(*runs):
+        assert np.array_equal(a, b)
