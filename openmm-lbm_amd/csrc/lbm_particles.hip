@@ -275,12 +275,16 @@ __global__ void __launch_bounds__(SPREAD_THREADS) spreadTiles(ParticleArgs a, Sp
     // The bin entries are taken SPREAD_CHUNK at a time, so that the candidates' LDS stays small and four work-groups
     // share a CU; a tile's eight bins hold about 8x the mean beads per tile, one chunk in the usual case.
     constexpr int SPREAD_CHUNK = 256;
-    __shared__ unsigned long long acc[3*SPREAD_THREADS];
+    // A tile row's sums are STRIDE words from the next one's: with 32 the rows of a bead would all lie in one bank.
+    constexpr int STRIDE = SPREAD_TX + 4, PLANE = STRIDE*SPREAD_TY*SPREAD_TZ;
+    __shared__ unsigned long long acc[3*PLANE];
     __shared__ int candidates[SPREAD_CHUNK];
-    __shared__ short candidateLocal[SPREAD_CHUNK][3];
     __shared__ double candidateForce[SPREAD_CHUNK][3];
+    constexpr int ROWS = W*W;                              // stencil rows along x of a bead
+    // The rows that lie in this tile: candidate | row << 8 | tile row << 12 | (first node's x + 4) << 16.
+    __shared__ uint32_t items[SPREAD_CHUNK*ROWS];
     __shared__ int counts[8], firsts[8];
-    __shared__ int numCandidates;
+    __shared__ int numCandidates, numItems;
     const uint32_t tile = blockIdx.x;
     const uint32_t tx = tile % bins.ntx, ty = (tile/bins.ntx) % bins.nty, tz = tile/(bins.ntx*bins.nty);
     const int t = (int) threadIdx.x;
@@ -292,6 +296,8 @@ __global__ void __launch_bounds__(SPREAD_THREADS) spreadTiles(ParticleArgs a, Sp
         counts[t] = min(bins.count[from], bins.cap);
         firsts[t] = (int) from;
     }
+    // Bits of beads that spread themselves (full bins); without any, the fused pass left the word clear.
+    const bool spilled = *bins.spilled != 0;
     if (t == 0) {
         bins.nextCount[tile] = 0;
         if (tile == 0)
@@ -303,15 +309,16 @@ __global__ void __launch_bounds__(SPREAD_THREADS) spreadTiles(ParticleArgs a, Sp
         total += counts[d];
     if (total == 0)
         return;
+    const int own = t/SPREAD_TX*STRIDE + t % SPREAD_TX;
     for (int k = 0; k < 3; k++)
-        acc[k*SPREAD_THREADS + t] = 0ull;
+        acc[k*PLANE + own] = 0ull;
     const int lane = t & 63;
     for (int chunk = 0; chunk < total; chunk += SPREAD_CHUNK) {
         // The candidates of this chunk of bin entries that reach into this tile, gathered by every thread: a bead
         // binned one tile back along an axis reaches it when its first stencil node lies within W - 1 nodes of that
         // tile's end.  Each keeps its first node relative to this tile's origin (negative for the tiles behind).
         if (t == 0)
-            numCandidates = 0;
+            numCandidates = numItems = 0;
         __syncthreads();
         for (int c = chunk + t; c < min(total, chunk + SPREAD_CHUNK); c += SPREAD_THREADS) {
             int r = c, d = 0;
@@ -320,64 +327,66 @@ __global__ void __launch_bounds__(SPREAD_THREADS) spreadTiles(ParticleArgs a, Sp
                 d++;
             }
             const size_t entry = (size_t) firsts[d]*bins.cap + r;
+            // Loaded whether the bead reaches the tile or not: one wait instead of two in a row.
             const uint32_t off = bins.anchor[entry];
+            const int bead = bins.beads[entry];
+            const double force[3] = {bins.force[3*entry], bins.force[3*entry + 1], bins.force[3*entry + 2]};
             const int ox = (int) (off & 31u), oy = (int) ((off >> 5) & 3u), oz = (int) ((off >> 7) & 3u);
             const bool reaches = (!(d & 1) || ox >= SPREAD_TX - W + 1) && (!(d & 2) || oy >= SPREAD_TY - W + 1) &&
                                  (!(d & 4) || oz >= SPREAD_TZ - W + 1);
             if (reaches) {
                 const int at = atomicAdd(&numCandidates, 1);
-                candidates[at] = bins.beads[entry];
-                candidateLocal[at][0] = (short) ((d & 1) ? ox - SPREAD_TX : ox);
-                candidateLocal[at][1] = (short) ((d & 2) ? oy - SPREAD_TY : oy);
-                candidateLocal[at][2] = (short) ((d & 4) ? oz - SPREAD_TZ : oz);
+                candidates[at] = bead;
                 for (int k = 0; k < 3; k++)
-                    candidateForce[at][k] = bins.force[3*entry + k];
+                    candidateForce[at][k] = force[k];
+                // Its first node relative to the tile, and the rows from max(that, 0) on that the tile holds.
+                const int cx = (d & 1) ? ox - SPREAD_TX : ox, cy = (d & 2) ? oy - SPREAD_TY : oy;
+                const int cz = (d & 4) ? oz - SPREAD_TZ : oz;
+                const int y0 = max(cy, 0), y1 = min(cy + W, SPREAD_TY), z0 = max(cz, 0), z1 = min(cz + W, SPREAD_TZ);
+                int next = atomicAdd(&numItems, (y1 - y0)*(z1 - z0));
+                for (int z = z0; z < z1; z++)
+                    for (int y = y0; y < y1; y++)
+                        items[next++] = (uint32_t) (at | (y - cy + W*(z - cz)) << 8 | (y + SPREAD_TY*z) << 12 |
+                                                    (cx + 4) << 16);
             }
         }
         __syncthreads();
-        // One item per (candidate, stencil row along x); each thread loads the weights of UNROLL rows before it adds
-        // any, so that their loads overlap.
-        constexpr int ROWS = W*W;
-        const int items = numCandidates*ROWS;
-        constexpr int UNROLL = 2;
-        for (int base = t; base < items; base += SPREAD_THREADS*UNROLL) {
-            int rowLocal[UNROLL], x0[UNROLL], cand[UNROLL];
-            double weight[UNROLL][W];
+        // One lane per slot of the listed rows; each thread loads UNROLL weights before it adds any, so that their loads
+        // overlap.  The rows are listed because only 5 in 16 of a Keys bead's lie in one of the tiles that it reaches: lanes
+        // left idle by the others paid for the FP64 conversions all the same.  With the padded rows of the sums and an
+        // entry's loads in one wait, 100,000 Keys chain beads in 128^3 73.5 -> 54 us, bound by the waits of a tile's
+        // phases (256 threads per tile 67 us, 1,024 threads 69, 512 entries at a time, two work-groups per CU, 80).
+        constexpr int UNROLL = 4;
+        const int slots = numItems*W;
+        for (int base = t; base < slots; base += SPREAD_THREADS*UNROLL) {
+            int at[UNROLL], cand[UNROLL];
+            double weight[UNROLL];
 #pragma unroll
             for (int u = 0; u < UNROLL; u++) {
-                const int item = base + u*SPREAD_THREADS;
-                rowLocal[u] = -1;
-                if (item < items) {
-                    const int c = item/ROWS, row = item % ROWS;
-                    const int ly = candidateLocal[c][1] + row % W, lz = candidateLocal[c][2] + row/W;
-                    if (ly >= 0 && ly < SPREAD_TY && lz >= 0 && lz < SPREAD_TZ) {
-                        const double* w = bins.slotWeight + (size_t) candidates[c]*LANES + W*row;
-#pragma unroll
-                        for (int sx = 0; sx < W; sx++)
-                            weight[u][sx] = w[sx];
-                        rowLocal[u] = SPREAD_TX*(ly + SPREAD_TY*lz);
-                        x0[u] = candidateLocal[c][0];
+                const int slot = base + u*SPREAD_THREADS;
+                at[u] = -1;
+                if (slot < slots) {
+                    const uint32_t item = items[slot/W];
+                    const int sx = slot % W, c = (int) (item & 255u), row = (int) ((item >> 8) & 15u);
+                    const int lx = (int) (item >> 16) - 4 + sx;
+                    if (lx >= 0 && lx < SPREAD_TX) {
+                        weight[u] = bins.slotWeight[(size_t) candidates[c]*LANES + W*row + sx];
+                        at[u] = STRIDE*(int) ((item >> 12) & 15u) + lx;
                         cand[u] = c;
                     }
                 }
             }
 #pragma unroll
             for (int u = 0; u < UNROLL; u++) {
-                if (rowLocal[u] < 0)
+                if (at[u] < 0)
                     continue;
-#pragma unroll
-                for (int sx = 0; sx < W; sx++) {
-                    const int lx = x0[u] + sx;
-                    if (lx < 0 || lx >= SPREAD_TX)
+                for (int k = 0; k < 3; k++) {
+                    double r = -weight[u]*candidateForce[cand[u]][k];
+                    if (!reactionInRange(r, a.overflow))
                         continue;
-                    for (int k = 0; k < 3; k++) {
-                        double r = -weight[u][sx]*candidateForce[cand[u]][k];
-                        if (!reactionInRange(r, a.overflow))
-                            continue;
-                        long long fixed = llrint(r*FIXED_SCALE);
-                        if (fixed != 0)
-                            atomicAdd(&acc[k*SPREAD_THREADS + rowLocal[u] + lx], (unsigned long long) fixed);
-                    }
+                    long long fixed = llrint(r*FIXED_SCALE);
+                    if (fixed != 0)
+                        atomicAdd(&acc[k*PLANE + at[u]], (unsigned long long) fixed);
                 }
             }
         }
@@ -386,12 +395,10 @@ __global__ void __launch_bounds__(SPREAD_THREADS) spreadTiles(ParticleArgs a, Sp
     const int lo[3] = {(int) tx*SPREAD_TX, (int) ty*SPREAD_TY, (int) tz*SPREAD_TZ};
     const int lx = t % SPREAD_TX, ly = (t/SPREAD_TX) % SPREAD_TY, lz = t/(SPREAD_TX*SPREAD_TY);
     const uint32_t node = (uint32_t) (lo[0] + lx) + a.g.nx*((uint32_t) (lo[1] + ly) + a.g.ny*(uint32_t) (lo[2] + lz));
-    const unsigned long long v[3] = {acc[t], acc[SPREAD_THREADS + t], acc[2*SPREAD_THREADS + t]};
+    const unsigned long long v[3] = {acc[own], acc[PLANE + own], acc[2*PLANE + own]};
     const bool any = (v[0] | v[1] | v[2]) != 0ull && !solidAt(mask, node);
     const uint64_t ballot = __ballot(any);
     const uint32_t rowBits = (uint32_t) (ballot >> (lane & 32));
-    // Bits of beads that spread themselves (full bins); without any, the fused pass left the word clear.
-    const bool spilled = *bins.spilled != 0;
     uint32_t old = 0;
     if (spilled && lx == 0 && rowBits != 0u)
         old = touched[node >> 5];
