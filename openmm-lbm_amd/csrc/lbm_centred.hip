@@ -24,6 +24,10 @@
  *    one at a time, so the iterations and results are those of a check after every iteration without a round trip
  *    to the host for each.
  *
+ *    Where the lattice is periodic and the particles have few neighbours (CgRows) the matrix is formed instead, once per
+ *    solve: row k holds K_kl of the particles l whose stencils share a node with k's, 11 on average for 56,320 Keys
+ *    particles in 120^3 against 64 slots, and a product reads its row and its neighbours' entries, no node sums.
+ *
  * The reaction goes into the same fixed-point accumulators as the explicit drag (consumed by the fused pass; with the
  * split, stored where no other slot reaches the node, since those accumulators are zero, and added atomically where
  * several do), and into the wall partial sums at solid nodes.
@@ -44,9 +48,11 @@ constexpr int CG_MAX_ITERATIONS = 1000;
 /* Device scalars of the conjugate gradients. */
 enum Scalar {
     RZ = 0, RZ_NEW = 3, RR = 6, NORM = 9, DAD = 12, ALPHA = 15, BETA = 18, SCALE = 21, INV_SCALE = 22,
+    RZ_SLOT = RZ_NEW - RZ,   // with matrix rows r.z of iteration t is at RZ + RZ_SLOT (t mod 2)
     DONE = 23,        // 1 once the residual is within tolerance: the remaining iterations' kernels return at once
     ITERS = 24,       // iterations run in this solve
-    NUM_SCALARS = 25
+    OVERFLOWED = 25,  // the host's copy of CgRows::overflow
+    NUM_SCALARS = 26
 };
 
 void check(hipError_t e, const char* what) {
@@ -199,6 +205,7 @@ struct CgArgs {
     double* r;
     double* z;
     double* d;
+    int stride;              // of z and d from one particle to the next
     double* Ad;
     uint32_t* slotNode;
     double* slotW;
@@ -217,6 +224,32 @@ struct CgArgs {
     int split;
     uint32_t* seen;
     uint32_t* shared;
+};
+
+/*
+ * The matrix of the solve by rows.  The particles are binned by the node their stencil starts at in cells of 4 x 4 x 4
+ * nodes (the last cell of an axis takes the remainder, up to 7 nodes), so that those whose stencils reach a particle's lie in
+ * the 27 cells around its own.  A row's entries are in the order of their particle, whatever the order in which the bins
+ * were filled, so a solve is reproducible.  More than CELL_CAP particles in a cell or ROW_CAP in a row raise
+ * `overflow`; the solve is then repeated with the spread.
+ */
+constexpr int CELL_CAP = 64, ROW_CAP = 128;
+constexpr double ROWS_MEAN_NEIGHBOURS = 64.0;      // half of ROW_CAP
+constexpr int ROWS_RETRY = 128;                    // solves by the spread after an overflow
+struct CellEntry {
+    int particle, rank;
+    uint32_t offset;         // of its first stencil node within the cell, x | y << 3 | z << 6
+};
+struct CgRows {
+    int cells[3] = {0, 0, 0};
+    int* cellCount = nullptr;        // cleared by cgInit
+    CellEntry* cell = nullptr;       // [cell][CELL_CAP]
+    uint32_t* home = nullptr;        // [rank][4]: the particle's cell along each axis, and its offset there
+    double* axisWeight = nullptr;    // [rank][3][3w - 2]: the weights along each axis between w - 1 zeros on either side
+    int* rowCount = nullptr;         // [rank]
+    int* rowParticle = nullptr;      // [rank][ROW_CAP]
+    double* rowValue = nullptr;
+    int* overflow = nullptr;
 };
 
 /* Whether a slot's node takes part in the spread of a product: every node without the split, else the shared ones. */
@@ -245,7 +278,7 @@ __global__ void __launch_bounds__(BLOCK) cgSetup(const S* __restrict__ src, cons
         const double* __restrict__ positions, const double* __restrict__ velocities,
         const double* __restrict__ otherForces, const int* __restrict__ particles, const double* __restrict__ mass,
         const double* __restrict__ ucm, ParticleArgs a, double gx, double gy, double gz, CgArgs c,
-        const double4* __restrict__ field) {
+        const double4* __restrict__ field, CgRows rows) {
     constexpr int GROUPS = BLOCK/LANES;
     const double h = 0.5, aa = a.gamma*h;
     int lane = threadIdx.x % LANES;
@@ -254,22 +287,52 @@ __global__ void __launch_bounds__(BLOCK) cgSetup(const S* __restrict__ src, cons
     const int i = active ? particleAt(c, rank) : 0;
     int part = active ? particles[i] : 0;
     const double* x = positions + 3*(size_t) part;
-    // The stencil of the lanes (groupStencil): each lane evaluates its own slot's kernel weight per axis.
+    // The stencil of the lanes (groupStencil), its slots along the axes formed by the group's first 3 w lanes as in
+    // interpolateGroup.
     constexpr int STENCIL = groupStencil<LANES>();
     constexpr int w = STENCIL == LBM_STENCIL_KEYS ? 4 : STENCIL == LBM_STENCIL_THREE_POINT ? 3 : 2;
     bool inStencil = active && lane < c.slots;
     double ux = 0, uy = 0, uz = 0, self = 0;
-    if (inStencil) {
-        int size[3] = {(int) a.g.nx, (int) a.g.ny, (int) a.g.nz};
-        int openAxis[3] = {a.g.openX, a.g.openY, a.g.openZ};
-        int sub[3] = {lane % w, (lane/w) % w, lane/(w*w)};
-        int nodeIdx[3];
-        double weight = 1.0;
-        for (int k = 0; k < 3; k++) {
-            double wk;
-            axisSlot<STENCIL>(wrapCoordinate(x[k], a.dx, size[k]), size[k], openAxis[k] != 0, sub[k], nodeIdx[k], wk);
-            weight *= wk;
+    const int nx = (int) a.g.nx, ny = (int) a.g.ny, nz = (int) a.g.nz;
+    const int openX = a.g.openX, openY = a.g.openY, openZ = a.g.openZ;
+    int axisIndex;
+    double axisWeight;
+    {
+        const int axis = lane < w ? 0 : (lane < 2*w ? 1 : 2);
+        const int size = axis == 0 ? nx : (axis == 1 ? ny : nz);
+        const int open = axis == 0 ? openX : (axis == 1 ? openY : openZ);
+        axisSlot<STENCIL>(wrapCoordinate(x[axis], a.dx, size), size, open != 0, min(lane - axis*w, w - 1), axisIndex,
+                axisWeight);
+    }
+    const int sub[3] = {lane % w, (lane/w) % w, min(lane/(w*w), w - 1)};
+    int nodeIdx[3], first[3];
+    double weight = 1.0;
+    for (int k = 0; k < 3; k++) {
+        nodeIdx[k] = __shfl(axisIndex, k*w + sub[k], LANES);
+        first[k] = __shfl(axisIndex, k*w, LANES);
+        weight *= __shfl(axisWeight, k*w + sub[k], LANES);
+    }
+    if (rows.cell != nullptr && active) {
+        if (lane < 3*w)
+            rows.axisWeight[((size_t) rank*3 + lane/w)*(3*w - 2) + w - 1 + lane % w] = axisWeight;
+        if (lane == 0) {
+            int cell[3];
+            uint32_t offset = 0;
+            for (int k = 0; k < 3; k++) {
+                cell[k] = min(first[k] >> 2, rows.cells[k] - 1);
+                offset |= (uint32_t) (first[k] - 4*cell[k]) << (3*k);
+                rows.home[4*(size_t) rank + k] = (uint32_t) cell[k];
+            }
+            rows.home[4*(size_t) rank + 3] = offset;
+            const size_t at = (size_t) cell[0] + (size_t) rows.cells[0]*(cell[1] + (size_t) rows.cells[1]*cell[2]);
+            const int entry = atomicAdd(rows.cellCount + at, 1);
+            if (entry < CELL_CAP)
+                rows.cell[at*CELL_CAP + entry] = CellEntry{i, rank, offset};
+            else
+                *rows.overflow = 1;
         }
+    }
+    if (inStencil) {
         uint32_t node = (uint32_t) (nodeIdx[0] + (int) a.g.nx*(nodeIdx[1] + (int) a.g.ny*nodeIdx[2]));
         bool solid = solidAt(mask, node);
         double winv = 0.0;
@@ -315,6 +378,134 @@ __global__ void __launch_bounds__(BLOCK) cgSetup(const S* __restrict__ src, cons
             c.rhs[3*(size_t) i + k] = b;
             c.F[3*(size_t) i + k] = b*(1.0/diag);
         }
+    }
+}
+
+/*
+ * The matrix row of each particle, one wavefront per particle, and the first product Ad = A F.  Pairs of lanes search a
+ * cell each, the particles found are sorted by index, and then a lane takes a neighbour l: K_kl = sum over k's slots of
+ * (w_k/rho) w_l, its own weights along the axes shifted by the distance of the two stencils (zero outside).  Forming the
+ * row by lanes that are neighbours takes 84 FP64 operations for up to 64 of them; by lanes that are slots it takes a
+ * sum over the wavefront for each.  56,320 Keys particles in 120^3: 96 us, bound by the chain of loads (cell, entries, weights),
+ * and a product then takes 17 us (cgRowsStep) where spread and gather took 145.
+ */
+template <int W>
+__global__ void __launch_bounds__(BLOCK) cgRows(int n, int nx, int ny, int nz, CgArgs c, CgRows rows,
+        const double* __restrict__ mass, double aa) {
+    constexpr int WAVES = BLOCK/64, SLOTS = W*W*W;
+    struct Found {
+        int particle[ROW_CAP], rank[ROW_CAP];
+        uint16_t shift[ROW_CAP];             // the distance of the stencils + 3 along each axis, 3 bits each
+        uint8_t sorted[ROW_CAP];
+    };
+    __shared__ Found all[WAVES];
+    const int lane = (int) threadIdx.x & 63;
+    const int rank = __builtin_amdgcn_readfirstlane((int) placeOf(c)*WAVES + (int) threadIdx.x/64);
+    if (rank >= n)
+        return;
+    // w/rho of the particle's slots: the same for every lane, so operands from scalar registers.
+    const auto* own = (const __attribute__((address_space(4))) double*) (uintptr_t) (c.slotWInvRho + (size_t) rank*SLOTS);
+    Found& f = all[threadIdx.x/64];
+    const int size[3] = {nx, ny, nz};
+    int origin[3] = {0, 0, 0};               // of the lane's cell, from the own cell's
+    size_t at = 0;
+    const uint4 home = *(const uint4*) (rows.home + 4*(size_t) rank);
+    const uint32_t offset = home.w;
+    int count = 0;
+    if (lane < 54) {
+        const int c27 = lane >> 1;
+        const int step[3] = {c27 % 3 - 1, c27/3 % 3 - 1, c27/9 - 1};
+        const int own[3] = {(int) home.x, (int) home.y, (int) home.z};
+        int cell[3];
+        for (int k = 0; k < 3; k++) {
+            const int last = rows.cells[k] - 1;
+            cell[k] = own[k] + step[k] < 0 ? last : (own[k] + step[k] > last ? 0 : own[k] + step[k]);
+            const int widthOfLast = size[k] - 4*last;
+            if (step[k] > 0)
+                origin[k] = own[k] == last ? widthOfLast : 4;
+            else if (step[k] < 0)
+                origin[k] = cell[k] == last ? -widthOfLast : -4;
+        }
+        at = (size_t) cell[0] + (size_t) rows.cells[0]*(cell[1] + (size_t) rows.cells[1]*cell[2]);
+        count = min(rows.cellCount[at], CELL_CAP);
+    }
+    int found = 0;
+    // Two lanes per cell, two entries each per turn, their loads in one wait.
+    for (int first = lane & 1; __ballot(first < count) != 0; first += 4) {
+        CellEntry entries[2];
+        for (int u = 0; u < 2; u++)
+            entries[u] = first + 2*u < count ? rows.cell[at*CELL_CAP + first + 2*u] : CellEntry{0, 0, 0};
+        for (int u = 0; u < 2; u++) {
+            const CellEntry entry = entries[u];
+            bool hit = first + 2*u < count;
+            int d[3];
+            for (int k = 0; k < 3; k++) {
+                d[k] = origin[k] + (int) ((entry.offset >> (3*k)) & 7u) - (int) ((offset >> (3*k)) & 7u);
+                hit = hit && d[k] > -W && d[k] < W;
+            }
+            const uint64_t hits = __ballot(hit);
+            const int place = found + (int) __popcll(hits & ((1ull << lane) - 1ull));
+            if (hit && place < ROW_CAP) {
+                f.particle[place] = entry.particle;
+                f.rank[place] = entry.rank;
+                f.shift[place] = (uint16_t) ((d[0] + 3) | (d[1] + 3) << 3 | (d[2] + 3) << 6);
+            }
+            found += (int) __popcll(hits);
+        }
+    }
+    if (found > ROW_CAP) {
+        if (lane == 0)
+            *rows.overflow = 1;
+        found = ROW_CAP;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    for (int e = lane; e < found; e += 64) {
+        const int own = f.particle[e];
+        int place = 0;
+        for (int o = 0; o < found; o++)
+            place += f.particle[o] < own ? 1 : 0;
+        f.sorted[place] = (uint8_t) e;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    double acc[3] = {0, 0, 0};
+    for (int e = lane; e < found; e += 64) {
+        const int from = f.sorted[e], l = f.particle[from];
+        const uint32_t shift = f.shift[from];
+        const double* weights = rows.axisWeight + (size_t) f.rank[from]*(3*(3*W - 2)) + W - 1;
+        double wl[3][W];
+        for (int k = 0; k < 3; k++) {
+            const int d = (int) ((shift >> (3*k)) & 7u) - 3;
+            for (int sl = 0; sl < W; sl++)
+                wl[k][sl] = weights[k*(3*W - 2) + sl - d];
+        }
+        double value = 0.0;
+        for (int z = 0; z < W; z++) {
+            double plane = 0.0;
+            for (int y = 0; y < W; y++) {
+                double row = 0.0;
+                for (int xs = 0; xs < W; xs++)
+                    row = fma(own[xs + W*(y + W*z)], wl[0][xs], row);
+                plane = fma(row, wl[1][y], plane);
+            }
+            value = fma(plane, wl[2][z], value);
+        }
+        rows.rowParticle[(size_t) rank*ROW_CAP + e] = l;
+        rows.rowValue[(size_t) rank*ROW_CAP + e] = value;
+        for (int k = 0; k < 3; k++)
+            acc[k] = fma(value, c.F[3*(size_t) l + k], acc[k]);
+    }
+    for (int k = 0; k < 3; k++)
+        acc[k] = groupSum<64>(acc[k]);
+    if (lane == 0)
+        rows.rowCount[rank] = found;
+    if (lane < 3) {
+        const size_t i = (size_t) particleAt(c, rank);
+        const double own = lane == 0 ? acc[0] : (lane == 1 ? acc[1] : acc[2]);
+        c.Ad[3*i + lane] = c.F[3*i + lane]*((1.0 + aa)/mass[i]) + own*aa;
     }
 }
 
@@ -492,7 +683,9 @@ __device__ __forceinline__ void reduceBlock(double v[8], int count, double* part
 }
 
 /* r = rhs - Ax, z = r/diag, d = z; partials: r.z, rhs.rhs, r.r (3 each -> 9 values in two reductions). */
-__global__ void __launch_bounds__(BLOCK) cgInit(int n, CgArgs c, double* partialsB) {
+__global__ void __launch_bounds__(BLOCK) cgInit(int n, CgArgs c, double* partialsB, int* cellCount, int numCells) {
+    for (int cell = blockIdx.x*BLOCK + threadIdx.x; cell < numCells; cell += gridDim.x*BLOCK)
+        cellCount[cell] = 0;
     double v[8] = {0, 0, 0, 0, 0, 0, 0, 0}, w[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     for (int i = blockIdx.x*BLOCK + threadIdx.x; i < n; i += gridDim.x*BLOCK)
         for (int k = 0; k < 3; k++) {
@@ -500,8 +693,8 @@ __global__ void __launch_bounds__(BLOCK) cgInit(int n, CgArgs c, double* partial
             double r = c.rhs[t] - c.Ad[t];
             double z = r*(1.0/c.diag[i]);
             c.r[t] = r;
-            c.z[t] = z;
-            c.d[t] = z;
+            c.z[(size_t) i*c.stride + k] = z;
+            c.d[(size_t) i*c.stride + k] = z;
             v[k] += r*z;
             v[3 + k] += c.rhs[t]*c.rhs[t];
             w[k] += r*r;
@@ -542,7 +735,7 @@ __global__ void __launch_bounds__(BLOCK) cgDot(int n, CgArgs c, const double* do
    fixed combination; work-group 0 keeps it in the scalars); F += alpha d, r -= alpha Ad, z = r/diag; partialsOut:
    r.z (new), r.r (a buffer of its own: other work-groups may still be reading c.partials). */
 __global__ void __launch_bounds__(BLOCK) cgUpdate(int n, CgArgs c, double* __restrict__ partialsOut,
-        const double* done) {
+        const double* done, int rz) {
     if (done != nullptr && *done != 0.0)
         return;
     __shared__ double sharedAlpha[3];
@@ -551,7 +744,7 @@ __global__ void __launch_bounds__(BLOCK) cgUpdate(int n, CgArgs c, double* __res
         combinePartials<3>(c.partials, dad);
         if (threadIdx.x == 0)
             for (int k = 0; k < 3; k++) {
-                sharedAlpha[k] = dad[k] > 0 ? c.scalars[RZ + k]/dad[k] : 0.0;
+                sharedAlpha[k] = dad[k] > 0 ? c.scalars[rz + k]/dad[k] : 0.0;
                 if (blockIdx.x == 0) {
                     c.scalars[DAD + k] = dad[k];
                     c.scalars[ALPHA + k] = sharedAlpha[k];
@@ -564,11 +757,11 @@ __global__ void __launch_bounds__(BLOCK) cgUpdate(int n, CgArgs c, double* __res
     for (int i = blockIdx.x*BLOCK + threadIdx.x; i < n; i += gridDim.x*BLOCK)
         for (int k = 0; k < 3; k++) {
             size_t t = 3*(size_t) i + k;
-            c.F[t] += alpha[k]*c.d[t];
+            c.F[t] += alpha[k]*c.d[(size_t) i*c.stride + k];
             double r = c.r[t] - alpha[k]*c.Ad[t];
             double z = r*(1.0/c.diag[i]);
             c.r[t] = r;
-            c.z[t] = z;
+            c.z[(size_t) i*c.stride + k] = z;
             v[k] += r*z;
             v[3 + k] += r*r;
         }
@@ -620,11 +813,132 @@ __global__ void __launch_bounds__(BLOCK) cgDirection(int n, CgArgs c, const doub
         c.partials[8*blockIdx.x] = lds[0];
 }
 
+/*
+ * One iteration's direction and product with the matrix rows, ROW_LANES lanes per particle: beta = r.z(new)/r.z(old) from
+ * the update's partial sums (formed by the first wavefront of every work-group, one fixed combination), d = z + beta d and
+ * Ad = A d with the neighbours' new d formed on the way, and d.Ad of each work-group.  A particle's z and old d are side by
+ * side, [particle][z, d], one gather for both (20.7 -> 16.8 us for 56,320 Keys particles, bound by these gathers); d goes to
+ * the other of two such arrays, since the neighbours read the old one, and the update puts the new z beside it.  Tests the
+ * residual first, as the direction after a converged iteration is not needed.  With cgUpdate, two launches per iteration
+ * where the spread takes six.
+ */
+constexpr int ROW_LANES = 8, ROW_THREADS_CG = 1024;
+__global__ void __launch_bounds__(ROW_THREADS_CG) cgRowsStep(int n, CgArgs c, CgRows rows, const double* __restrict__ old,
+        double* __restrict__ next, const double* __restrict__ mass, double aa, const double* __restrict__ partialsB,
+        int iteration) {
+    __shared__ double sharedBeta[3];
+    __shared__ int sharedDone;
+    __shared__ double sums[ROW_THREADS_CG/64][3];
+    const int t = (int) threadIdx.x;
+    if (t < 64) {
+        double v[6] = {0, 0, 0, 0, 0, 0};
+        if (iteration > 0)
+            combinePartials<6>(partialsB, v);
+        if (t == 0) {
+            bool done = c.scalars[DONE] != 0.0;
+            double beta[3] = {0, 0, 0};
+            if (!done && iteration > 0) {
+                double test[NUM_SCALARS];
+                for (int k = 0; k < 3; k++) {
+                    test[RR + k] = v[3 + k];
+                    test[NORM + k] = c.scalars[NORM + k];
+                    const double rz = c.scalars[RZ + RZ_SLOT*((iteration - 1) & 1) + k];
+                    beta[k] = rz > 0 ? v[k]/rz : 0.0;
+                }
+                done = residualConverged(test);
+                if (blockIdx.x == 0) {
+                    for (int k = 0; k < 3; k++)
+                        c.scalars[RZ + RZ_SLOT*(iteration & 1) + k] = v[k];
+                    if (done) {
+                        c.scalars[ITERS] = (double) iteration;
+                        c.scalars[DONE] = 1.0;
+                    }
+                }
+            }
+            for (int k = 0; k < 3; k++)
+                sharedBeta[k] = beta[k];
+            sharedDone = done ? 1 : 0;
+        }
+    }
+    __syncthreads();
+    if (sharedDone)
+        return;
+    const double beta[3] = {sharedBeta[0], sharedBeta[1], sharedBeta[2]};
+    const int lane = t % ROW_LANES;
+    constexpr int PARTICLES = ROW_THREADS_CG/ROW_LANES;
+    double dot = 0.0;                        // of component `lane`
+    for (int base = (int) blockIdx.x*PARTICLES; base < n; base += RED_BLOCKS*PARTICLES) {
+        const int rank = base + t/ROW_LANES;
+        double s[3] = {0, 0, 0};
+        if (rank < n) {
+            const int count = rows.rowCount[rank];
+            for (int e = lane; e < count; e += ROW_LANES) {
+                const double2* from = (const double2*) (old + 6*(size_t) rows.rowParticle[(size_t) rank*ROW_CAP + e]);
+                const double value = rows.rowValue[(size_t) rank*ROW_CAP + e];
+                const double2 a01 = from[0], a23 = from[1], a45 = from[2];
+                s[0] = fma(value, fma(beta[0], a23.y, a01.x), s[0]);
+                s[1] = fma(value, fma(beta[1], a45.x, a01.y), s[1]);
+                s[2] = fma(value, fma(beta[2], a45.y, a23.x), s[2]);
+            }
+        }
+        for (int k = 0; k < 3; k++)
+            s[k] = groupSum<ROW_LANES>(s[k]);
+        if (rank < n && lane < 3) {
+            const size_t i = (size_t) particleAt(c, rank);
+            const double d = fma(lane == 0 ? beta[0] : (lane == 1 ? beta[1] : beta[2]), old[6*i + 3 + lane], old[6*i + lane]);
+            const double Ad = d*((1.0 + aa)/mass[i]) + (lane == 0 ? s[0] : (lane == 1 ? s[1] : s[2]))*aa;
+            next[6*i + 3 + lane] = d;
+            c.Ad[3*i + lane] = Ad;
+            dot = fma(d, Ad, dot);
+        }
+    }
+    for (int off = ROW_LANES; off < 64; off *= 2)
+        dot += __shfl_xor(dot, off, 64);
+    if ((t & 63) < 3)
+        sums[t/64][t & 63] = dot;
+    __syncthreads();
+    if (t < 3) {
+        double v = 0.0;
+        for (int w = 0; w < ROW_THREADS_CG/64; w++)
+            v += sums[w][t];
+        c.partials[8*blockIdx.x + t] = v;
+    }
+}
+
+/* The state of the solve after `iterations` iterations with the matrix rows, to the device scalars and to the host's
+   (page-locked): whether it has converged, and whether the rows overflowed, in which case nothing of it counts. */
+__global__ void __launch_bounds__(64) cgRowsCheck(const double* __restrict__ partialsB, double* __restrict__ scalars,
+        const int* __restrict__ overflow, int iterations, double* __restrict__ host) {
+    double v[6];
+    combinePartials<6>(partialsB, v);
+    if (threadIdx.x != 0)
+        return;
+    bool done = scalars[DONE] != 0.0;
+    if (!done) {
+        double test[NUM_SCALARS];
+        for (int k = 0; k < 3; k++) {
+            test[RR + k] = v[3 + k];
+            test[NORM + k] = scalars[NORM + k];
+        }
+        done = residualConverged(test);
+        scalars[ITERS] = (double) iterations;
+    }
+    const bool over = *overflow != 0;
+    scalars[DONE] = done && !over ? 1.0 : 0.0;
+    host[DONE] = scalars[DONE];
+    host[ITERS] = scalars[ITERS];
+    host[OVERFLOWED] = over ? 1.0 : 0.0;
+}
+
 /* The forces and the reactions -w F of the solution, one group of LANES lanes per particle (block layout of the explicit
    coupling, so the wall partials fit the same slots). */
 template <int LANES>
 __global__ void __launch_bounds__(BLOCK) cgForces(int n, ParticleArgs a, CgArgs c, double* __restrict__ particleForce,
-        unsigned long long* __restrict__ reactionFixed, uint32_t* __restrict__ touched, double* __restrict__ partials) {
+        unsigned long long* __restrict__ reactionFixed, uint32_t* __restrict__ touched, double* __restrict__ partials,
+        const int* __restrict__ rowCount) {
+    // With matrix rows the host launches this before it knows whether the solve has converged.
+    if (rowCount != nullptr && c.scalars[DONE] == 0.0)
+        return;
     constexpr int GROUPS = BLOCK/LANES;
     int lane = threadIdx.x % LANES;
     const int rank = (int) placeOf(c)*GROUPS + threadIdx.x/LANES;
@@ -646,8 +960,10 @@ __global__ void __launch_bounds__(BLOCK) cgForces(int n, ParticleArgs a, CgArgs 
             if (w != 0.0) {
                 double r[3] = {-w*F[0], -w*F[1], -w*F[2]};
                 bool solid = c.slotSolid[sl] != 0;
-                // With the split, a fluid slot that spreads nothing is alone at its node: a store, not an atomic.
-                if (c.split && !solid && c.slotSpreads[sl] == 0 && c.slotWInvRho[sl] != 0.0)
+                // With the split, a fluid slot that spreads nothing is alone at its node, and with matrix rows so is
+                // every slot of a particle without neighbours: a store, not an atomic.
+                const bool alone = rowCount != nullptr ? rowCount[rank] == 1 : c.split && c.slotSpreads[sl] == 0;
+                if (alone && !solid && c.slotWInvRho[sl] != 0.0)
                     flagged = storeReaction(node, r, a, reactionFixed);
                 else if (solid)
                     for (int k = 0; k < 3; k++)
@@ -658,7 +974,7 @@ __global__ void __launch_bounds__(BLOCK) cgForces(int n, ParticleArgs a, CgArgs 
         }
         // Both arrays of node sums and the node bits of the split, cleared for the next solve (every word that a
         // spread or cgMarkShared set belongs to one of these slots; nothing reads them after the solve).
-        if (lane < c.slots) {
+        if (rowCount == nullptr && lane < c.slots) {
             size_t sl = (size_t) rank*c.slots + lane;
             uint32_t at = c.slotNode[sl];
             if (c.slotSpreads[sl] != 0)
@@ -704,12 +1020,19 @@ struct CentredState {
     double* hostScalars = nullptr;        // pinned: the convergence check reads the scalars
     int lastIterations = 1;               // iterations of the previous solve: enqueued before the first check
     bool planned = true;                  // false (LBM_AMD_CG_PLANNED=0): the host reads the residual after each
+    // The matrix rows and their two arrays of directions; retryRows: solves to go by the spread after an overflow.
+    CgRows rows;
+    int numCells = 0;
+    double* directions[2] = {nullptr, nullptr};      // [particle][z, d]
+    int retryRows = 0;
+    hipEvent_t checked = nullptr;
     std::vector<void*> buffers;
 };
 
-CentredState* centredCreate(int numParticles, int stencil, uint32_t numNodes) {
+CentredState* centredCreate(int numParticles, int stencil, const Geometry& g) {
     CentredState* st = new CentredState();
     try {
+        const uint32_t numNodes = g.n;
         int n = std::max(numParticles, 1);
         st->n = numParticles;
         st->stencil = stencil;
@@ -734,6 +1057,7 @@ CentredState* centredCreate(int numParticles, int stencil, uint32_t numNodes) {
         else {
             CgArgs& c = st->cg;
             c.slots = st->slots;
+            c.stride = 3;
             c.rhs = alloc<double>(3*(size_t) n);
             c.diag = alloc<double>(n);
             c.F = alloc<double>(3*(size_t) n);
@@ -774,6 +1098,42 @@ CentredState* centredCreate(int numParticles, int stencil, uint32_t numNodes) {
                            c.shared};
             check(hipHostMalloc((void**) &st->hostScalars, NUM_SCALARS*sizeof(double), hipHostMallocDefault),
                     "pinned scalars");
+            // The matrix rows: periodic axes of at least three cells (no stencil meets another from both sides), and rows
+            // that are expected at most half full, as are the cells.  There a step by the rows was the faster one at every
+            // size measured: 56,320 Keys particles in 120^3 (11 neighbours) 620 us against 1,330, 20,000 in 256^3 (0.4) 781
+            // against 938, 20,000 in 48^3 (62) 310 against 546, 2,000 trilinear ones in 128^3 148 against 193.
+            // LBM_AMD_CG_ROWS=0 or 1 forces the choice where the lattice allows it; LBM_AMD_CG_SPLIT chooses a spread.
+            const double reach = (2.0*w - 1)*(2.0*w - 1)*(2.0*w - 1);
+            const char* rowsEnv = getenv("LBM_AMD_CG_ROWS");
+            const bool periodic = !g.openX && !g.openY && !g.openZ && g.nx >= 12 && g.ny >= 12 && g.nz >= 12;
+            const bool want = rowsEnv ? rowsEnv[0] == '1' : splitEnv == nullptr &&
+                    reach*numParticles <= ROWS_MEAN_NEIGHBOURS*numNodes && numParticles <= (4 << 20) &&
+                    64.0*numParticles <= 0.5*CELL_CAP*numNodes;
+            if (periodic && want) {
+                CgRows& r = st->rows;
+                r.cells[0] = (int) g.nx/4;
+                r.cells[1] = (int) g.ny/4;
+                r.cells[2] = (int) g.nz/4;
+                st->numCells = r.cells[0]*r.cells[1]*r.cells[2];
+                r.cellCount = alloc<int>(st->numCells);
+                r.cell = alloc<CellEntry>((size_t) st->numCells*CELL_CAP);
+                r.home = alloc<uint32_t>(4*(size_t) n);
+                r.axisWeight = alloc<double>(3*(3*(size_t) w - 2)*n);
+                r.rowCount = alloc<int>(n);
+                r.rowParticle = alloc<int>((size_t) n*ROW_CAP);
+                r.rowValue = alloc<double>((size_t) n*ROW_CAP);
+                r.overflow = alloc<int>(1);
+                st->directions[0] = alloc<double>(6*(size_t) n);
+                st->directions[1] = alloc<double>(6*(size_t) n);
+                check(hipMemset(r.cellCount, 0, st->numCells*sizeof(int)), "memset");
+                check(hipMemset(r.axisWeight, 0, 3*(3*(size_t) w - 2)*n*sizeof(double)), "memset");
+                check(hipMemset(r.overflow, 0, sizeof(int)), "memset");
+                check(hipEventCreateWithFlags(&st->checked, hipEventDisableTiming), "event");
+                for (void* b : {(void*) r.cellCount, (void*) r.cell, (void*) r.home, (void*) r.axisWeight, (void*) r.rowCount,
+                                (void*) r.rowParticle, (void*) r.rowValue, (void*) r.overflow, (void*) st->directions[0],
+                                (void*) st->directions[1]})
+                    st->buffers.push_back(b);
+            }
         }
     }
     catch (...) {
@@ -789,6 +1149,8 @@ void centredDestroy(CentredState* st) {
     for (void* p : st->buffers)
         if (p)
             (void) hipFree(p);
+    if (st->checked)
+        (void) hipEventDestroy(st->checked);
     if (st->hostScalars)
         (void) hipHostFree(st->hostScalars);
     delete st;
@@ -826,6 +1188,57 @@ bool converged(CentredState* st, hipStream_t stream) {
     return residualConverged(s);
 }
 
+const char* const NOT_CONVERGED = "LBMForce: the centred drag with the interpolation stencil did not converge in 1000 "
+        "iterations of the conjugate gradients";
+
+/*
+ * The solve with the matrix rows, after cgSetup has binned the particles.  The forces (a launch that does nothing before the
+ * solve has converged) go onto the stream ahead of the host's wait for the residual, so that the device works meanwhile.
+ * Returns false if a bin or a row was too small.
+ */
+template <typename Forces>
+bool solveRows(CentredState* st, const Geometry& g, const double* mass, double aa, hipStream_t stream, Forces&& forces) {
+    CgArgs c = st->cg;
+    const CgRows& r = st->rows;
+    const int n = st->n, nx = (int) g.nx, ny = (int) g.ny, nz = (int) g.nz;
+    const unsigned waves = blocksOf(n, BLOCK/64);
+    switch (st->lanes) {
+    case 8: cgRows<2><<<waves, BLOCK, 0, stream>>>(n, nx, ny, nz, c, r, mass, aa); break;
+    case 32: cgRows<3><<<waves, BLOCK, 0, stream>>>(n, nx, ny, nz, c, r, mass, aa); break;
+    default: cgRows<4><<<waves, BLOCK, 0, stream>>>(n, nx, ny, nz, c, r, mass, aa); break;
+    }
+    c.stride = 6;
+    c.z = st->directions[0];
+    c.d = c.z + 3;
+    cgInit<<<RED_BLOCKS, BLOCK, 0, stream>>>(n, c, st->partialsB, r.cellCount, st->numCells);
+    cgFinishInit<<<1, 64, 0, stream>>>(c.partials, st->partialsB, c.scalars);
+    int iteration = 0;
+    for (int batch = st->planned ? std::max(st->lastIterations, 1) : 1;; batch = 1) {
+        for (int b = 0; b < batch; b++, iteration++) {
+            c.z = st->directions[(iteration + 1) & 1];
+            c.d = c.z + 3;
+            cgRowsStep<<<RED_BLOCKS, ROW_THREADS_CG, 0, stream>>>(n, c, r, st->directions[iteration & 1], c.z, mass, aa,
+                    st->partialsB, iteration);
+            cgUpdate<<<RED_BLOCKS, BLOCK, 0, stream>>>(n, c, st->partialsB, c.scalars + DONE, RZ + RZ_SLOT*(iteration & 1));
+        }
+        cgRowsCheck<<<1, 64, 0, stream>>>(st->partialsB, c.scalars, r.overflow, iteration, st->hostScalars);
+        check(hipEventRecord(st->checked, stream), "event");
+        forces();
+        check(hipGetLastError(), "launch");
+        check(hipEventSynchronize(st->checked), "sync");
+        if (st->hostScalars[OVERFLOWED] != 0.0) {
+            check(hipMemsetAsync(r.overflow, 0, sizeof(int), stream), "memset");
+            return false;
+        }
+        if (st->hostScalars[DONE] != 0.0)
+            break;
+        if (iteration >= CG_MAX_ITERATIONS)
+            throw std::runtime_error(NOT_CONVERGED);
+    }
+    st->lastIterations = (int) st->hostScalars[ITERS];
+    return true;
+}
+
 template <typename S>
 void centredCoupleT(CentredState* st, const S* src, const uint32_t* mask, const double* positions,
         const double* velocities, const double* otherForces, const int* particles, const double* mass,
@@ -848,20 +1261,44 @@ void centredCoupleT(CentredState* st, const S* src, const uint32_t* mask, const 
     c.order = order;
     double aa = 0.5*a.gamma;
     unsigned groups = blocksOf(n, BLOCK/st->lanes);
-    switch (st->lanes) {
-    case 8:
-        cgSetup<S, 8><<<groups, BLOCK, 0, stream>>>(src, mask, positions, velocities, otherForces, particles, mass, ucm, a,
-                g[0], g[1], g[2], c, field);
-        break;
-    case 32:
-        cgSetup<S, 32><<<groups, BLOCK, 0, stream>>>(src, mask, positions, velocities, otherForces, particles, mass, ucm, a,
-                g[0], g[1], g[2], c, field);
-        break;
-    default:
-        cgSetup<S, 64><<<groups, BLOCK, 0, stream>>>(src, mask, positions, velocities, otherForces, particles, mass, ucm, a,
-                g[0], g[1], g[2], c, field);
-        break;
+    auto setup = [&](const CgRows& rows) {
+        switch (st->lanes) {
+        case 8:
+            cgSetup<S, 8><<<groups, BLOCK, 0, stream>>>(src, mask, positions, velocities, otherForces, particles, mass, ucm, a,
+                    g[0], g[1], g[2], c, field, rows);
+            break;
+        case 32:
+            cgSetup<S, 32><<<groups, BLOCK, 0, stream>>>(src, mask, positions, velocities, otherForces, particles, mass, ucm,
+                    a, g[0], g[1], g[2], c, field, rows);
+            break;
+        default:
+            cgSetup<S, 64><<<groups, BLOCK, 0, stream>>>(src, mask, positions, velocities, otherForces, particles, mass, ucm,
+                    a, g[0], g[1], g[2], c, field, rows);
+            break;
+        }
+    };
+    auto forces = [&](const int* rowCount) {
+        switch (st->lanes) {
+        case 8:
+            cgForces<8><<<groups, BLOCK, 0, stream>>>(n, a, c, particleForce, reactionFixed, touched, partials, rowCount);
+            break;
+        case 32:
+            cgForces<32><<<groups, BLOCK, 0, stream>>>(n, a, c, particleForce, reactionFixed, touched, partials, rowCount);
+            break;
+        default:
+            cgForces<64><<<groups, BLOCK, 0, stream>>>(n, a, c, particleForce, reactionFixed, touched, partials, rowCount);
+            break;
+        }
+    };
+    if (st->rows.cell != nullptr && st->retryRows == 0) {
+        setup(st->rows);
+        if (solveRows(st, a.g, mass, aa, stream, [&] { forces(st->rows.rowCount); }))
+            return;
+        st->retryRows = ROWS_RETRY;
     }
+    else if (st->retryRows > 0)
+        st->retryRows--;
+    setup(CgRows());
     if (c.split)
         switch (st->lanes) {
         case 8: cgMarkShared<8><<<groups, BLOCK, 0, stream>>>(n, c); break;
@@ -870,7 +1307,7 @@ void centredCoupleT(CentredState* st, const S* src, const uint32_t* mask, const 
         }
     cgMaxAbs<<<RED_BLOCKS, BLOCK, 0, stream>>>(c.F, n, c.partials, nullptr);
     multiply<S>(st, c.F, c.Ad, mass, aa, nullptr, 1, true, stream);
-    cgInit<<<RED_BLOCKS, BLOCK, 0, stream>>>(n, c, st->partialsB);
+    cgInit<<<RED_BLOCKS, BLOCK, 0, stream>>>(n, c, st->partialsB, nullptr, 0);
     cgFinishInit<<<1, 64, 0, stream>>>(c.partials, st->partialsB, c.scalars);
     check(hipGetLastError(), "launch");
     // Each iteration starts with the new direction (d = z after cgInit), so that the last one computes none.  The
@@ -886,7 +1323,7 @@ void centredCoupleT(CentredState* st, const S* src, const uint32_t* mask, const 
                 cgDirection<<<RED_BLOCKS, BLOCK, 0, stream>>>(n, c, done);
             multiply<S>(st, c.d, c.Ad, mass, aa, done, iteration & 1, false, stream);
             cgDot<<<RED_BLOCKS, BLOCK, 0, stream>>>(n, c, done);
-            cgUpdate<<<RED_BLOCKS, BLOCK, 0, stream>>>(n, c, st->partialsB, done);
+            cgUpdate<<<RED_BLOCKS, BLOCK, 0, stream>>>(n, c, st->partialsB, done, RZ);
             cgFinishBeta<<<1, 64, 0, stream>>>(st->partialsB, c.scalars, done);
             check(hipGetLastError(), "launch");
         }
@@ -903,16 +1340,11 @@ void centredCoupleT(CentredState* st, const S* src, const uint32_t* mask, const 
                 check(hipMemsetAsync(c.seen, 0, bitBytes, stream), "memset");
                 check(hipMemsetAsync(c.shared, 0, bitBytes, stream), "memset");
             }
-            throw std::runtime_error("LBMForce: the centred drag with the interpolation stencil did not converge in 1000 "
-                    "iterations of the conjugate gradients");
+            throw std::runtime_error(NOT_CONVERGED);
         }
     }
     st->lastIterations = (int) st->hostScalars[ITERS];
-    switch (st->lanes) {
-    case 8: cgForces<8><<<groups, BLOCK, 0, stream>>>(n, a, c, particleForce, reactionFixed, touched, partials); break;
-    case 32: cgForces<32><<<groups, BLOCK, 0, stream>>>(n, a, c, particleForce, reactionFixed, touched, partials); break;
-    default: cgForces<64><<<groups, BLOCK, 0, stream>>>(n, a, c, particleForce, reactionFixed, touched, partials); break;
-    }
+    forces(nullptr);
     check(hipGetLastError(), "launch");
 }
 

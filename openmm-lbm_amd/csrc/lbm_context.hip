@@ -669,7 +669,7 @@ void create(const lbm_params* params, const int* solid, int numSolid, const int*
             c->stageForce = deviceAlloc<double>(3*(size_t) std::max(numSys, 1));
         try {
             if (p.drag_scheme == LBM_DRAG_CENTERED)
-                c->centred = centredCreate(numParts, p.interpolation_stencil, (uint32_t) n);
+                c->centred = centredCreate(numParts, p.interpolation_stencil, c->g);
             if (p.drag_scheme == LBM_DRAG_CENTERED ? c->dense && p.interpolation_stencil != LBM_STENCIL_NEAREST :
                     !c->dense && numParts > 2048)
                 // Sparse particles gain DRAM locality from the node order (a step of 8,000 Keys beads in 128^3 127 -> 119

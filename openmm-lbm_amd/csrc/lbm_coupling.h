@@ -267,7 +267,7 @@ __device__ __forceinline__ double pairedLane(double v) {
 }
 
 /*
- * The sum of v over each group of LANES lanes (1, 8, 32, 64), in every lane of the group: the butterfly of lane distances
+ * The sum of v over each group of LANES lanes (1, 8, 16, 32, 64), in every lane of the group: the butterfly of lane distances
  * 1, 2, 4, ... with its bits, without its trips through the LDS permute unit (two per double and distance, each waiting
  * for the one before).  Distances 1 and 2 are quad permutes; once the lanes of a quad (of 8 lanes) agree, the mirrored lane
  * holds what the lane 4 (8) away does; 16 and 32 are the row and half swaps, which give both partners' values to both.
@@ -280,8 +280,9 @@ __device__ __forceinline__ double groupSum(double v) {
         v += pairedLane<0x4E>(v);         // quad_perm [2, 3, 0, 1]
         v += pairedLane<0x141>(v);        // row_half_mirror
     }
-    if constexpr (LANES >= 32) {
+    if constexpr (LANES >= 16)
         v += pairedLane<0x140>(v);        // row_mirror
+    if constexpr (LANES >= 32) {
         const unsigned lo = (unsigned) __double2loint(v), hi = (unsigned) __double2hiint(v);
         const pair_t a = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
         const pair_t b = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
@@ -293,7 +294,7 @@ __device__ __forceinline__ double groupSum(double v) {
         const pair_t b = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
         v = __hiloint2double((int) b[0], (int) a[0]) + __hiloint2double((int) b[1], (int) a[1]);
     }
-    static_assert(LANES == 1 || LANES == 8 || LANES == 32 || LANES == 64, "group sizes of the stencils");
+    static_assert(LANES == 1 || LANES == 8 || LANES == 16 || LANES == 32 || LANES == 64, "group sizes");
     return v;
 }
 

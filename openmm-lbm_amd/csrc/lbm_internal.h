@@ -282,7 +282,7 @@ void launchParticleNodes(const double* positions, const int* particles, const Pa
    acceleration in lattice units; field: the moments of the nodes (launchMomentField) for the stencils of dense particles,
    or nullptr; order: the particles in the order to process their stencils (coupleOrderAt), or nullptr.  Throws std::runtime_error. */
 struct CentredState;
-CentredState* centredCreate(int numParticles, int stencil, uint32_t numNodes);
+CentredState* centredCreate(int numParticles, int stencil, const Geometry& g);
 void centredDestroy(CentredState* state);
 void centredCouple(CentredState* state, int storage, const void* src, const uint32_t* mask, const double* positions,
         const double* velocities, const double* otherForces, const int* particles, const double* mass,

@@ -182,3 +182,50 @@ def test_slots_of_a_group_are_those_formed_per_particle(grid, open_faces, beads,
     assert np.abs(runs[0][0]).max() > 0
     for a, b in zip(*runs):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("stencil", [LBMForce.Trilinear, LBMForce.ThreePoint, LBMForce.Keys],
+                         ids=["trilinear", "threepoint", "keys"])
+@pytest.mark.parametrize("grid,beads,crowd", [((12, 12, 12), 1, 0), ((12, 13, 15), 70, 0), ((31, 16, 23), 900, 0),
+                                              ((24, 20, 14), 40, 60), ((24, 20, 14), 40, 140)],
+                         ids=["one", "three-cells", "long-rows", "nearly-full", "overflowing"])
+def test_centred_matrix_rows_match_the_spread(grid, beads, crowd, stencil, monkeypatch):
+    """The centred drag's solve with the matrix formed by rows against the solve that spreads over the nodes: the smallest
+    lattice and those whose last cells take a remainder, particles alone and with some hundred neighbours, a cell of up to 60
+    (of 64 entries) and one of 140, after which the solve is repeated by the spread with its bits.  Both stop at a residual
+    of 1e-13 of the right-hand side; the matrix' condition is below 100 here, so the forces agree to 1e-11 of the largest.
+    Runs are reproducible, also with a check after each iteration."""
+    rng = np.random.default_rng(beads + crowd)
+    pos = rng.uniform(0, grid, size=(beads, 3))
+    pos = np.concatenate([pos, [4.5, 8.5, 4.5] + rng.uniform(-0.4, 0.4, size=(crowd, 3))])
+    vel = rng.normal(scale=0.5, size=pos.shape)
+    masses = rng.uniform(50, 200, size=len(pos))
+    s = Setup(grid, tau=0.8)
+    for x, v, m in zip(pos, vel, masses):
+        s.add_particles([x], mass=m, velocities=[v])
+
+    def conf(f):
+        f.setSolidNodes(list(range(grid[0]*grid[1])))
+        f.setWallScheme(LBMForce.BounceBack)
+        f.setFriction(10.0)
+        f.setTemperature(300.0)
+        f.setRandomNumberSeed(5)
+        f.setDragScheme(LBMForce.Centered)
+        f.setInterpolationStencil(stencil)
+    s.configure.append(conf)
+
+    def forces(rows, planned="1"):
+        monkeypatch.setenv("LBM_AMD_CG_ROWS", rows)
+        monkeypatch.setenv("LBM_AMD_CG_PLANNED", planned)
+        c = s.build(None, storage=LBMForce.FP64)
+        c.step(3)
+        return c.getForces(), c.getFluidState()
+    spread, rows = forces("0"), forces("1")
+    assert np.abs(spread[0]).max() > 0
+    assert np.abs(rows[0] - spread[0]).max() <= 1e-11*np.abs(spread[0]).max()
+    for again in (forces("1"), forces("1", planned="0")):
+        for a, b in zip(rows, again):
+            assert np.array_equal(a, b)
+    if crowd > 100:
+        for a, b in zip(rows, spread):
+            assert np.array_equal(a, b)
