@@ -931,11 +931,13 @@ __global__ void __launch_bounds__(64) cgRowsCheck(const double* __restrict__ par
 }
 
 /* The forces and the reactions -w F of the solution, one group of LANES lanes per particle (block layout of the explicit
-   coupling, so the wall partials fit the same slots). */
-template <int LANES>
+   coupling, so the wall partials fit the same slots).  BINNED: in a step each particle goes into the bin of its first
+   node's tile for spreadTiles, with the slots' weights where cgSetup left them; one whose bin is full spreads here (56,320
+   Keys particles in 120^3: 46 us and 38 us for the tiles against 118 with the atomics). */
+template <int LANES, bool BINNED>
 __global__ void __launch_bounds__(BLOCK) cgForces(int n, ParticleArgs a, CgArgs c, double* __restrict__ particleForce,
         unsigned long long* __restrict__ reactionFixed, uint32_t* __restrict__ touched, double* __restrict__ partials,
-        const int* __restrict__ rowCount) {
+        const int* __restrict__ rowCount, SpreadBins bins) {
     // With matrix rows the host launches this before it knows whether the solve has converged.
     if (rowCount != nullptr && c.scalars[DONE] == 0.0)
         return;
@@ -947,12 +949,37 @@ __global__ void __launch_bounds__(BLOCK) cgForces(int n, ParticleArgs a, CgArgs 
     bool flagged = false;
     __shared__ StagedReactions<BLOCK> staged;
     staged.clear();
+    bool atomics = true;
     if (rank < n) {
         const int i = particleAt(c, rank);
         double F[3] = {c.F[3*(size_t) i], c.F[3*(size_t) i + 1], c.F[3*(size_t) i + 2]};
         if (lane == 0)
             for (int k = 0; k < 3; k++)
                 particleForce[3*(size_t) i + k] = F[k]*a.forceScale;
+        if constexpr (BINNED) {
+            int full = 0;
+            if (a.isStep && lane == 0) {
+                uint32_t x[3];
+                nodeCoords(a.g, c.slotNode[(size_t) rank*c.slots], x[0], x[1], x[2]);
+                const uint32_t tx = tileOf(x[0], bins.ntx, bins.perNode[0]), ty = tileOf(x[1], bins.nty, bins.perNode[1]);
+                const uint32_t tz = tileOf(x[2], bins.ntz, bins.perNode[2]);
+                const uint32_t tile = tx + bins.ntx*(ty + bins.nty*tz);
+                const int slot = atomicAdd(bins.count + tile, 1);
+                if (slot < bins.cap) {
+                    const size_t entry = (size_t) tile*bins.cap + slot;
+                    bins.beads[entry] = rank;
+                    bins.anchor[entry] = (uint16_t) ((x[0] - tileStart(tx, a.g.nx, bins.perTile[0])) |
+                            (x[1] - tileStart(ty, a.g.ny, bins.perTile[1])) << 5 | (x[2] - tileStart(tz, a.g.nz, bins.perTile[2])) << 7);
+                    for (int k = 0; k < 3; k++)
+                        bins.force[3*entry + k] = F[k];
+                }
+                else {
+                    full = 1;
+                    atomicOr(bins.spilled, 1);
+                }
+            }
+            atomics = __shfl(full, 0, LANES) != 0;
+        }
         if (a.isStep && lane < c.slots) {
             size_t sl = (size_t) rank*c.slots + lane;
             double w = c.slotW[sl];
@@ -962,13 +989,13 @@ __global__ void __launch_bounds__(BLOCK) cgForces(int n, ParticleArgs a, CgArgs 
                 bool solid = c.slotSolid[sl] != 0;
                 // With the split, a fluid slot that spreads nothing is alone at its node, and with matrix rows so is
                 // every slot of a particle without neighbours: a store, not an atomic.
-                const bool alone = rowCount != nullptr ? rowCount[rank] == 1 : c.split && c.slotSpreads[sl] == 0;
+                const bool alone = BINNED ? false : rowCount != nullptr ? rowCount[rank] == 1 : c.split && c.slotSpreads[sl] == 0;
                 if (alone && !solid && c.slotWInvRho[sl] != 0.0)
                     flagged = storeReaction(node, r, a, reactionFixed);
                 else if (solid)
                     for (int k = 0; k < 3; k++)
                         wallAcc[k] = r[k];               // lattice momentum; the host converts the wall partials
-                else
+                else if (atomics)
                     flagged = staged.put(node, r, a);
             }
         }
@@ -1242,8 +1269,9 @@ bool solveRows(CentredState* st, const Geometry& g, const double* mass, double a
 template <typename S>
 void centredCoupleT(CentredState* st, const S* src, const uint32_t* mask, const double* positions,
         const double* velocities, const double* otherForces, const int* particles, const double* mass,
-        const double* ucm, const ParticleArgs& a, const double g[3], const double4* field, const int* order, double* particleForce,
-        unsigned long long* reactionFixed, uint32_t* touched, double* partials, hipStream_t stream) {
+        const double* ucm, const ParticleArgs& a, const double g[3], const double4* field, const int* order,
+        const SpreadBins* bins, double* particleForce, unsigned long long* reactionFixed, uint32_t* touched, double* partials,
+        hipStream_t stream) {
     int n = a.numParticles;
     if (n == 0)
         return;
@@ -1277,17 +1305,35 @@ void centredCoupleT(CentredState* st, const S* src, const uint32_t* mask, const 
             break;
         }
     };
+    SpreadBins spread;
+    if (bins != nullptr && a.isStep) {
+        spread = *bins;
+        spread.slotWeight = c.slotW;
+        spread.weightStride = c.slots;
+    }
     auto forces = [&](const int* rowCount) {
-        switch (st->lanes) {
-        case 8:
-            cgForces<8><<<groups, BLOCK, 0, stream>>>(n, a, c, particleForce, reactionFixed, touched, partials, rowCount);
-            break;
-        case 32:
-            cgForces<32><<<groups, BLOCK, 0, stream>>>(n, a, c, particleForce, reactionFixed, touched, partials, rowCount);
-            break;
-        default:
-            cgForces<64><<<groups, BLOCK, 0, stream>>>(n, a, c, particleForce, reactionFixed, touched, partials, rowCount);
-            break;
+        auto launch = [&](auto binned) {
+            constexpr bool B = decltype(binned)::value;
+            switch (st->lanes) {
+            case 8:
+                cgForces<8, B><<<groups, BLOCK, 0, stream>>>(n, a, c, particleForce, reactionFixed, touched, partials, rowCount,
+                        spread);
+                break;
+            case 32:
+                cgForces<32, B><<<groups, BLOCK, 0, stream>>>(n, a, c, particleForce, reactionFixed, touched, partials, rowCount,
+                        spread);
+                break;
+            default:
+                cgForces<64, B><<<groups, BLOCK, 0, stream>>>(n, a, c, particleForce, reactionFixed, touched, partials, rowCount,
+                        spread);
+                break;
+            }
+        };
+        if (spread.count == nullptr)
+            launch(std::false_type());
+        else {
+            launch(std::true_type());
+            launchSpreadTiles(mask, a, spread, reactionFixed, touched, stream);
         }
     };
     if (st->rows.cell != nullptr && st->retryRows == 0) {
@@ -1352,24 +1398,25 @@ void centredCoupleT(CentredState* st, const S* src, const uint32_t* mask, const 
 
 void centredCouple(CentredState* st, int storage, const void* src, const uint32_t* mask, const double* positions,
         const double* velocities, const double* otherForces, const int* particles, const double* mass,
-        const double* ucm, const ParticleArgs& a, const double g[3], const double4* field, const int* order, double* particleForce,
-        unsigned long long* reactionFixed, uint32_t* touched, double* partials, hipStream_t stream) {
+        const double* ucm, const ParticleArgs& a, const double g[3], const double4* field, const int* order,
+        const SpreadBins* bins, double* particleForce, unsigned long long* reactionFixed, uint32_t* touched, double* partials,
+        hipStream_t stream) {
     switch (storage) {
     case LBM_STORAGE_FP16:
         centredCoupleT<__half>(st, (const __half*) src, mask, positions, velocities, otherForces, particles, mass, ucm, a,
-                g, field, order, particleForce, reactionFixed, touched, partials, stream);
+                g, field, order, bins, particleForce, reactionFixed, touched, partials, stream);
         break;
     case LBM_STORAGE_BF16:
         centredCoupleT<__hip_bfloat16>(st, (const __hip_bfloat16*) src, mask, positions, velocities, otherForces,
-                particles, mass, ucm, a, g, field, order, particleForce, reactionFixed, touched, partials, stream);
+                particles, mass, ucm, a, g, field, order, bins, particleForce, reactionFixed, touched, partials, stream);
         break;
     case LBM_STORAGE_FP64:
         centredCoupleT<double>(st, (const double*) src, mask, positions, velocities, otherForces, particles, mass, ucm, a,
-                g, field, order, particleForce, reactionFixed, touched, partials, stream);
+                g, field, order, bins, particleForce, reactionFixed, touched, partials, stream);
         break;
     default:
         centredCoupleT<float>(st, (const float*) src, mask, positions, velocities, otherForces, particles, mass, ucm, a,
-                g, field, order, particleForce, reactionFixed, touched, partials, stream);
+                g, field, order, bins, particleForce, reactionFixed, touched, partials, stream);
         break;
     }
 }

@@ -342,13 +342,24 @@ void couple(lbm_context* c, const double* dPos, const double* dVel, const double
     catch (const std::runtime_error& e) {
         throw Error(LBM_ERROR_RUNTIME, e.what());
     }
+    const SpreadBins* bins = nullptr;
+    if (c->binned && isStep && c->closure == nullptr) {
+        c->bins.count = c->binCounts[c->binParity];
+        c->bins.nextCount = c->binCounts[c->binParity ^ 1];
+        c->bins.spilled = c->binSpilled + c->binParity;
+        c->bins.nextSpilled = c->binSpilled + (c->binParity ^ 1);
+        bins = &c->bins;
+    }
     if (c->centred != nullptr) {
         // Centred drag: the other forces (dForces, before the coupling adds to them) enter the particle velocities.
         if (c->momentField != nullptr)
             launchMomentField(c->p.storage, c->popA, c->mask, a, c->ucm, c->momentField, dPos, c->particles, nullptr,
                     c->stream);
         centredCouple(c->centred, c->p.storage, c->popA, c->mask, dPos, dVel, dForces, c->particles, c->mass, c->ucm, a,
-                c->p.body_acceleration, c->momentField, order, c->particleForce, c->reactionFixed, c->touched, partials, c->stream);
+                c->p.body_acceleration, c->momentField, order, bins, c->particleForce,
+                c->reactionFixed, c->touched, partials, c->stream);
+        if (bins != nullptr)
+            c->binParity ^= 1;           // not after a solve that failed: its bins stay empty
         return;
     }
     if (c->closure != nullptr) {
@@ -364,15 +375,6 @@ void couple(lbm_context* c, const double* dPos, const double* dVel, const double
         c->forcesAdded = c->forceTarget != nullptr;
         return;
     }
-    const SpreadBins* bins = nullptr;
-    if (c->binned && isStep) {
-        c->bins.count = c->binCounts[c->binParity];
-        c->bins.nextCount = c->binCounts[c->binParity ^ 1];
-        c->bins.spilled = c->binSpilled + c->binParity;
-        c->bins.nextSpilled = c->binSpilled + (c->binParity ^ 1);
-        c->binParity ^= 1;
-        bins = &c->bins;
-    }
     if (c->momentField != nullptr)
         launchMomentField(c->p.storage, c->popA, c->mask, a, c->ucm, c->momentField, dPos, c->particles, c->axisStencils,
                 c->stream);
@@ -380,8 +382,10 @@ void couple(lbm_context* c, const double* dPos, const double* dVel, const double
         launchStencilSetup(dPos, c->particles, a, c->axisStencils, c->stream);
     launchCouple(c->p.storage, c->popA, c->mask, dPos, dVel, c->identityParticles ? nullptr : c->particles, order, c->mass, c->ucm, a, c->particleForce,
             c->reactionFixed, c->touched, partials, c->forceTarget, bins, c->momentField, c->axisStencils, c->stream);
-    if (bins != nullptr)
-        launchSpreadTiles(dPos, c->particles, c->mask, a, *bins, c->reactionFixed, c->touched, c->stream);
+    if (bins != nullptr) {
+        launchSpreadTiles(c->mask, a, *bins, c->reactionFixed, c->touched, c->stream);
+        c->binParity ^= 1;
+    }
     c->forcesAdded = c->forceTarget != nullptr;
 }
 
@@ -683,32 +687,38 @@ void create(const lbm_params* params, const int* solid, int numSolid, const int*
         catch (const std::runtime_error& e) {
             throw Error(LBM_ERROR_RUNTIME, e.what());
         }
-        // The one-writer spread (spreadTiles) for the explicit drag on lattices of whole tiles with periodic faces.
-        // LBM_AMD_SPREAD=atomic or =tiles forces the choice where it fits; by default the tiles serve dense particles
-        // (the stencils cover more than a quarter of the lattice), whose concurrent atomics contend.
+        // The one-writer spread (spreadTiles) for the explicit drag and the centred one's stencils, with periodic faces.
+        // LBM_AMD_SPREAD=atomic or =tiles forces the choice where it fits; by default the tiles serve many particles whose
+        // slots outnumber the nodes.  A step in us by atomics and by tiles: 100,000 Keys chain beads in 124^3 372 and 260,
+        // 20,000 in 90 x 70 x 100 104 and 92, 15,000 Keys beads in 80^3 81 and 78; but with 640,000 slots (10,000 centred Keys
+        // beads in 48^3) 198 and 208, 128,000 (2,000 in 40^3) 26 and 33, and with 0.6 slots per node (20,000 in 128^3) 165
+        // and 170, 0.4 (100,000 in 256^3) 1,132 and 1,241.
         const char* spreadEnv = getenv("LBM_AMD_SPREAD");
         if (const char* xcdEnv = getenv("LBM_AMD_COUPLE_XCD"))
             c->coupleXcd = xcdEnv[0] != '0';
         bool anyOpen = c->openAxis(0) || c->openAxis(1) || c->openAxis(2);
-        bool fit = p.drag_scheme == LBM_DRAG_EXPLICIT && spreadTilesFit(p.nx, p.ny, p.nz, anyOpen);
-        bool want = spreadEnv ? std::string(spreadEnv) == "tiles" : c->dense;
-        // The moment field: by default for dense particles with the explicit drag; LBM_AMD_FIELD=0 or 1 forces it.
+        bool fit = (p.drag_scheme == LBM_DRAG_EXPLICIT || p.interpolation_stencil != LBM_STENCIL_NEAREST) &&
+                spreadTilesFit(p.nx, p.ny, p.nz, anyOpen, c->bins);
+        const uint64_t slots = (uint64_t) numParts*(uint64_t) c->numSlots;
+        bool want = spreadEnv ? std::string(spreadEnv) == "tiles" : slots >= n && slots >= 900000;
+        // The moment field and the stencils formed once per particle: by default for dense particles whose slots are worth the
+        // field's launch.  A step of the explicit drag in us without and with both: 10,000 Keys beads in 128^3 142 and 137,
+        // 15,000 in 80^3 124 and 81; but 5,000 in 50 x 47 x 61 (320,000 slots) 39 and 41, 2,000 in 40^3 24 and 26.
+        // LBM_AMD_FIELD=0 or 1 forces the field.
+        const bool many = c->dense && (p.drag_scheme == LBM_DRAG_CENTERED || slots >= 400000);
         const char* fieldEnv = getenv("LBM_AMD_FIELD");
-        bool field = fieldEnv ? fieldEnv[0] == '1' : c->dense;
+        bool field = fieldEnv ? fieldEnv[0] == '1' : many;
         if (field && (p.drag_scheme == LBM_DRAG_EXPLICIT || p.interpolation_stencil != LBM_STENCIL_NEAREST))
             c->momentField = deviceAlloc<double4>(n);
         // The stencils formed once per particle for the groups of the explicit stencil coupling, by default for dense
         // particles (100,000 Keys beads on 128^3: the coupling kernel 148 -> 110 us, the setup 11 us; for 20,000 sparse
         // beads on 256^3 the extra launch costs what it saves); LBM_AMD_STENCIL_SETUP=0 or 1 forces the choice.
         const char* setupEnv = getenv("LBM_AMD_STENCIL_SETUP");
-        bool setup = setupEnv ? setupEnv[0] == '1' : c->dense;
+        bool setup = setupEnv ? setupEnv[0] == '1' : many;
         if (p.drag_scheme == LBM_DRAG_EXPLICIT && p.interpolation_stencil != LBM_STENCIL_NEAREST && setup)
             c->axisStencils = deviceAlloc<AxisStencil>((size_t) numParts);
         if (fit && want) {
             SpreadBins& b = c->bins;
-            b.ntx = (uint32_t) (p.nx/SPREAD_TX);
-            b.nty = (uint32_t) (p.ny/SPREAD_TY);
-            b.ntz = (uint32_t) (p.nz/SPREAD_TZ);
             size_t tiles = (size_t) b.ntx*b.nty*b.ntz;
             // Room for four times the mean number of beads per tile and 16 more; a bead beyond it spreads itself with
             // the atomics.
@@ -724,7 +734,9 @@ void create(const lbm_params* params, const int* solid, int numSolid, const int*
             c->binSpilled = deviceAlloc<int>(2);
             HIP_CHECK(hipMemsetAsync(c->binSpilled, 0, 2*sizeof(int), c->stream));
             int lanes = coupleLanes(p.interpolation_stencil);
-            b.slotWeight = deviceAlloc<double>((size_t) numParts*lanes);
+            b.weightStride = lanes;
+            if (p.drag_scheme == LBM_DRAG_EXPLICIT)
+                b.slotWeight = deviceAlloc<double>((size_t) numParts*lanes);
             c->binned = true;
         }
     }

@@ -87,8 +87,9 @@ struct ParticleArgs {
 constexpr double REACTION_LIMIT = 64.0;
 
 /*
- * The bins of the one-writer spread of the particle reactions (spreadTiles): the lattice in tiles of 32 x 4 x 4 nodes
- * (x fastest; a tile row of 32 nodes is one word of the touched mask); per tile the indices of up to cap beads whose
+ * The bins of the one-writer spread of the particle reactions (spreadTiles): the lattice in tiles of up to 32 x 4 x 4 nodes
+ * (x fastest; where every tile has 32 along x, a tile row is one word of the touched mask), as few as that takes, each axis
+ * divided as evenly as whole nodes allow (tileStart); per tile the indices of up to cap beads whose
  * stencil starts in it (their anchor node), and their count.  Two count arrays alternate: the spread of one step
  * clears the one the next step fills.  force: each binned bead's coupling force, lattice units.
  */
@@ -114,9 +115,26 @@ struct SpreadBins {
     double* slotWeight = nullptr;    // [bead][slot]: the weight of each stencil slot
     int* spilled = nullptr;          // set when a bead of the step found its bin full (spread with the atomics)
     int* nextSpilled = nullptr;      // the flag of the next step, cleared by spreadTiles
+    int weightStride = 0;            // of slotWeight from one bead to the next
     int cap = 0;
     uint32_t ntx = 0, nty = 0, ntz = 0;
+    double perNode[3] = {0, 0, 0};   // 1/n and 1/tiles along each axis
+    double perTile[3] = {0, 0, 0};
 };
+
+/*
+ * The first node of tile t of `count` along an axis of n nodes, t n/count, and the tile of a node there,
+ * ((node + 1) count - 1)/n, in whole numbers.  The quotients by products: with n up to SPREAD_MAX_AXIS the numerators are below
+ * 2^26 and (numerator + 1/2)/divisor lies further from a whole number than the products round (integer divisions, six per
+ * bead, cost the coupling of 100,000 beads 8 of 77 us).
+ */
+constexpr uint32_t SPREAD_MAX_AXIS = 16384;
+__device__ __forceinline__ uint32_t tileStart(uint32_t t, uint32_t n, double perTile) {
+    return (uint32_t) (((double) (t*n) + 0.5)*perTile);
+}
+__device__ __forceinline__ uint32_t tileOf(uint32_t node, uint32_t count, double perNode) {
+    return (uint32_t) (((double) ((node + 1u)*count - 1u) + 0.5)*perNode);
+}
 
 __device__ __forceinline__ bool reactionInRange(double r, unsigned int* overflow) {
     if (fabs(r) < REACTION_LIMIT)
@@ -253,11 +271,11 @@ void launchMomentField(int storage, const void* src, const uint32_t* mask, const
 void launchStencilSetup(const double* positions, const int* particles, const ParticleArgs& a, AxisStencil* stencils,
         hipStream_t stream);
 /* The one-writer spread of the binned beads' reactions, one work-group per tile (after launchCouple with bins). */
-void launchSpreadTiles(const double* positions, const int* particles, const uint32_t* mask, const ParticleArgs& a,
-        const SpreadBins& bins, unsigned long long* reactionFixed, uint32_t* touched, hipStream_t stream);
-/* Whether the lattice suits the tile bins: every axis periodic, nx a multiple of 32 and ny, nz of 4, at least two tiles
-   along each axis. */
-bool spreadTilesFit(int nx, int ny, int nz, bool anyOpen);
+void launchSpreadTiles(const uint32_t* mask, const ParticleArgs& a, const SpreadBins& bins, unsigned long long* reactionFixed,
+        uint32_t* touched, hipStream_t stream);
+/* Whether the lattice suits the tile bins: every axis periodic and of 6 to SPREAD_MAX_AXIS nodes, so that there are two tiles or
+   more of at least 3 nodes along each (a Keys stencil reaches no further than the next tile); if so, the tiles. */
+bool spreadTilesFit(int nx, int ny, int nz, bool anyOpen, SpreadBins& bins);
 
 /*
  * The coupled particles sorted by nearest node (z slowest, descending): processed in this order, the particles of one
@@ -280,14 +298,15 @@ void launchParticleNodes(const double* positions, const int* particles, const Pa
 /* The centred drag (lbm_centred.hip): its buffers for numParticles coupled particles, and one coupling.  otherForces
    (kJ/mol/nm, all System particles, may be null) are the forces on the particles before the coupling; g is the body
    acceleration in lattice units; field: the moments of the nodes (launchMomentField) for the stencils of dense particles,
-   or nullptr; order: the particles in the order to process their stencils (coupleOrderAt), or nullptr.  Throws std::runtime_error. */
+   or nullptr; order: the particles in the order to process their stencils (coupleOrderAt), or nullptr; bins: the tile spread's,
+   for the reactions of a step, or nullptr (slotWeight unused).  Throws std::runtime_error. */
 struct CentredState;
 CentredState* centredCreate(int numParticles, int stencil, const Geometry& g);
 void centredDestroy(CentredState* state);
 void centredCouple(CentredState* state, int storage, const void* src, const uint32_t* mask, const double* positions,
         const double* velocities, const double* otherForces, const int* particles, const double* mass,
-        const double* ucm, const ParticleArgs& a, const double g[3], const double4* field, const int* order, double* particleForce,
-        unsigned long long* reactionFixed, uint32_t* touched, double* partials, hipStream_t stream);
+        const double* ucm, const ParticleArgs& a, const double g[3], const double4* field, const int* order, const SpreadBins* bins,
+        double* particleForce, unsigned long long* reactionFixed, uint32_t* touched, double* partials, hipStream_t stream);
 
 /*
  * The reflection at solid nodes that begins a step, for a caller that runs it in a kernel of its own (the device-resident

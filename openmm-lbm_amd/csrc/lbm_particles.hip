@@ -19,6 +19,7 @@
 #include "lbm_coupling.h"
 
 #include <hipcub/hipcub.hpp>
+#include <algorithm>
 #include <stdexcept>
 
 namespace lbm {
@@ -67,14 +68,13 @@ template <int STENCIL>
 __device__ __forceinline__ uint32_t anchorTile(const double* x, const ParticleArgs& a, const SpreadBins& bins,
         uint16_t* offset, const AxisStencil* pre) {
     const int size[3] = {(int) a.g.nx, (int) a.g.ny, (int) a.g.nz};
-    const int tileSize[3] = {SPREAD_TX, SPREAD_TY, SPREAD_TZ};
+    const uint32_t tiles[3] = {bins.ntx, bins.nty, bins.ntz};
     uint32_t t[3], o[3];
     for (int k = 0; k < 3; k++) {
-        // The first slot's node: on the lattices of whole tiles with periodic faces that the bins serve, no stencil is
-        // merged and it is the first node wrapped.
+        // The first slot's node: on the lattices with periodic faces that the bins serve, no stencil is merged and it is the first node wrapped.
         int first = pre != nullptr ? pre->index[k][0] : anchorIndex<STENCIL>(wrapCoordinate(x[k], a.dx, size[k]), size[k]);
-        t[k] = (uint32_t) (first/tileSize[k]);
-        o[k] = (uint32_t) (first - (int) t[k]*tileSize[k]);
+        t[k] = tileOf((uint32_t) first, tiles[k], bins.perNode[k]);
+        o[k] = (uint32_t) first - tileStart(t[k], (uint32_t) size[k], bins.perTile[k]);
     }
     *offset = (uint16_t) (o[0] | (o[1] << 5) | (o[2] << 7));
     return t[0] + bins.ntx*(t[1] + bins.nty*t[2]);
@@ -262,9 +262,9 @@ __global__ void __launch_bounds__(BLOCK) coupleParticles(const S* __restrict__ s
  * from the bead's first stencil node (its tile and anchor offset) and, where the row lies in the tile, loads its slots'
  * weights and adds the fixed-point reactions -w F of the slots inside the tile to the tile's accumulators in LDS.
  * Then each fluid node's sums are written by its own thread (a solid node's part went to the wall in the coupling),
- * and each tile row's touched-mask word by the row's first lane: no global atomics.  Weights and fixed-point values are those of the atomic spread
- * (spreadReaction), and integer sums do not depend on their order, so both give the same bits.  Lattices of whole tiles
- * with periodic faces only (spreadTilesFit): no stencil there is merged, so slot (sx, sy, sz) lies at the first node +
+ * and each tile row's touched-mask bits by the row's first lane: no global atomics on the sums.  Weights and fixed-point values are those of the atomic spread
+ * (spreadReaction), and integer sums do not depend on their order, so both give the same bits.  Lattices with periodic
+ * faces only (spreadTilesFit): no stencil there is merged, so slot (sx, sy, sz) lies at the first node +
  * (sx, sy, sz), wrapped.  The reference builds its per-node sums from a sort of the stencil slots by node
  * (lbmCoupling.cc:251-272, 1245-1266).
  */
@@ -288,6 +288,17 @@ __global__ void __launch_bounds__(SPREAD_THREADS) spreadTiles(ParticleArgs a, Sp
     const uint32_t tile = blockIdx.x;
     const uint32_t tx = tile % bins.ntx, ty = (tile/bins.ntx) % bins.nty, tz = tile/(bins.ntx*bins.nty);
     const int t = (int) threadIdx.x;
+    // The tile's origin and size, and the size of the tile before it, along each axis.
+    __shared__ int lo[3], wide[3], before[3];
+    if (t < 3) {
+        const uint32_t at = t == 0 ? tx : (t == 1 ? ty : tz), n = t == 0 ? a.g.nx : (t == 1 ? a.g.ny : a.g.nz);
+        const uint32_t tiles = t == 0 ? bins.ntx : (t == 1 ? bins.nty : bins.ntz);
+        const double perTile = t == 0 ? bins.perTile[0] : (t == 1 ? bins.perTile[1] : bins.perTile[2]);
+        const int start = (int) tileStart(at, n, perTile);
+        lo[t] = start;
+        wide[t] = (int) tileStart(at + 1, n, perTile) - start;
+        before[t] = (at > 0 ? start : (int) n) - (int) tileStart(at > 0 ? at - 1 : tiles - 1, n, perTile);
+    }
     if (t < 8) {
         uint32_t fx = (t & 1) ? (tx == 0 ? bins.ntx - 1 : tx - 1) : tx;
         uint32_t fy = (t & 2) ? (ty == 0 ? bins.nty - 1 : ty - 1) : ty;
@@ -332,17 +343,17 @@ __global__ void __launch_bounds__(SPREAD_THREADS) spreadTiles(ParticleArgs a, Sp
             const int bead = bins.beads[entry];
             const double force[3] = {bins.force[3*entry], bins.force[3*entry + 1], bins.force[3*entry + 2]};
             const int ox = (int) (off & 31u), oy = (int) ((off >> 5) & 3u), oz = (int) ((off >> 7) & 3u);
-            const bool reaches = (!(d & 1) || ox >= SPREAD_TX - W + 1) && (!(d & 2) || oy >= SPREAD_TY - W + 1) &&
-                                 (!(d & 4) || oz >= SPREAD_TZ - W + 1);
+            const bool reaches = (!(d & 1) || ox >= before[0] - W + 1) && (!(d & 2) || oy >= before[1] - W + 1) &&
+                                 (!(d & 4) || oz >= before[2] - W + 1);
             if (reaches) {
                 const int at = atomicAdd(&numCandidates, 1);
                 candidates[at] = bead;
                 for (int k = 0; k < 3; k++)
                     candidateForce[at][k] = force[k];
                 // Its first node relative to the tile, and the rows from max(that, 0) on that the tile holds.
-                const int cx = (d & 1) ? ox - SPREAD_TX : ox, cy = (d & 2) ? oy - SPREAD_TY : oy;
-                const int cz = (d & 4) ? oz - SPREAD_TZ : oz;
-                const int y0 = max(cy, 0), y1 = min(cy + W, SPREAD_TY), z0 = max(cz, 0), z1 = min(cz + W, SPREAD_TZ);
+                const int cx = (d & 1) ? ox - before[0] : ox, cy = (d & 2) ? oy - before[1] : oy;
+                const int cz = (d & 4) ? oz - before[2] : oz;
+                const int y0 = max(cy, 0), y1 = min(cy + W, wide[1]), z0 = max(cz, 0), z1 = min(cz + W, wide[2]);
                 int next = atomicAdd(&numItems, (y1 - y0)*(z1 - z0));
                 for (int z = z0; z < z1; z++)
                     for (int y = y0; y < y1; y++)
@@ -354,7 +365,7 @@ __global__ void __launch_bounds__(SPREAD_THREADS) spreadTiles(ParticleArgs a, Sp
         // One lane per slot of the listed rows; each thread loads UNROLL weights before it adds any, so that their loads
         // overlap.  The rows are listed because only 5 in 16 of a Keys bead's lie in one of the tiles that it reaches: lanes
         // left idle by the others paid for the FP64 conversions all the same.  With the padded rows of the sums and an
-        // entry's loads in one wait, 100,000 Keys chain beads in 128^3 73.5 -> 54 us, bound by the waits of a tile's
+        // entry's loads in one wait, 100,000 Keys chain beads in 128^3 73.5 -> 57 us, bound by the waits of a tile's
         // phases (256 threads per tile 67 us, 1,024 threads 69, 512 entries at a time, two work-groups per CU, 80).
         constexpr int UNROLL = 4;
         const int slots = numItems*W;
@@ -369,8 +380,8 @@ __global__ void __launch_bounds__(SPREAD_THREADS) spreadTiles(ParticleArgs a, Sp
                     const uint32_t item = items[slot/W];
                     const int sx = slot % W, c = (int) (item & 255u), row = (int) ((item >> 8) & 15u);
                     const int lx = (int) (item >> 16) - 4 + sx;
-                    if (lx >= 0 && lx < SPREAD_TX) {
-                        weight[u] = bins.slotWeight[(size_t) candidates[c]*LANES + W*row + sx];
+                    if (lx >= 0 && lx < wide[0]) {
+                        weight[u] = bins.slotWeight[(size_t) candidates[c]*bins.weightStride + W*row + sx];
                         at[u] = STRIDE*(int) ((item >> 12) & 15u) + lx;
                         cand[u] = c;
                     }
@@ -392,16 +403,22 @@ __global__ void __launch_bounds__(SPREAD_THREADS) spreadTiles(ParticleArgs a, Sp
         }
         __syncthreads();             // before the next chunk's candidates replace these
     }
-    const int lo[3] = {(int) tx*SPREAD_TX, (int) ty*SPREAD_TY, (int) tz*SPREAD_TZ};
     const int lx = t % SPREAD_TX, ly = (t/SPREAD_TX) % SPREAD_TY, lz = t/(SPREAD_TX*SPREAD_TY);
     const uint32_t node = (uint32_t) (lo[0] + lx) + a.g.nx*((uint32_t) (lo[1] + ly) + a.g.ny*(uint32_t) (lo[2] + lz));
     const unsigned long long v[3] = {acc[own], acc[PLANE + own], acc[2*PLANE + own]};
-    const bool any = (v[0] | v[1] | v[2]) != 0ull && !solidAt(mask, node);
+    const bool any = lx < wide[0] && ly < wide[1] && lz < wide[2] && (v[0] | v[1] | v[2]) != 0ull && !solidAt(mask, node);
     const uint64_t ballot = __ballot(any);
     const uint32_t rowBits = (uint32_t) (ballot >> (lane & 32));
+    // The row's bits lie in the words of its first and last node (of one word where the tiles are 32 nodes wide, and then no
+    // other tile writes it; elsewhere the words are shared and the bits are added).
+    const uint32_t bit = node & 31u;                       // the row's lane 0 holds its first node
+    const bool second = bit != 0u && (rowBits >> (32u - bit)) != 0u;
     uint32_t old = 0;
-    if (spilled && lx == 0 && rowBits != 0u)
-        old = touched[node >> 5];
+    if (spilled && lx == 0 && rowBits != 0u) {
+        old = touched[node >> 5] >> bit;
+        if (second)
+            old |= touched[(node >> 5) + 1] << (32u - bit);
+    }
     old = __shfl(old, lane & 32, 64);
     if (any) {
         const bool add = (old >> lx) & 1u;
@@ -410,8 +427,16 @@ __global__ void __launch_bounds__(SPREAD_THREADS) spreadTiles(ParticleArgs a, Sp
             reactionFixed[at] = add ? reactionFixed[at] + v[k] : v[k];
         }
     }
-    if (lx == 0 && rowBits != 0u)
-        touched[node >> 5] = old | rowBits;
+    if (lx == 0 && rowBits != 0u) {
+        if (bins.ntx*SPREAD_TX == a.g.nx)
+            touched[node >> 5] = old | rowBits;
+        else {
+            if (rowBits << bit != 0u)
+                atomicOr(touched + (node >> 5), rowBits << bit);
+            if (second)
+                atomicOr(touched + (node >> 5) + 1, rowBits >> (32u - bit));
+        }
+    }
 }
 
 /* The moment field, after SETUP work-groups that form the particles' stencils (stencilSetupLane) when STENCIL is a
@@ -480,15 +505,26 @@ void launchMomentField(int storage, const void* src, const uint32_t* mask, const
     }
 }
 
-bool spreadTilesFit(int nx, int ny, int nz, bool anyOpen) {
-    return !anyOpen && nx % SPREAD_TX == 0 && ny % SPREAD_TY == 0 && nz % SPREAD_TZ == 0 && nx >= 2*SPREAD_TX &&
-           ny >= 2*SPREAD_TY && nz >= 2*SPREAD_TZ;
+bool spreadTilesFit(int nx, int ny, int nz, bool anyOpen, SpreadBins& bins) {
+    const int n[3] = {nx, ny, nz}, tile[3] = {SPREAD_TX, SPREAD_TY, SPREAD_TZ};
+    uint32_t tiles[3];
+    for (int k = 0; k < 3; k++) {
+        if (anyOpen || n[k] < 6 || n[k] > (int) SPREAD_MAX_AXIS)
+            return false;
+        tiles[k] = (uint32_t) std::max(2, (n[k] + tile[k] - 1)/tile[k]);
+    }
+    bins.ntx = tiles[0];
+    bins.nty = tiles[1];
+    bins.ntz = tiles[2];
+    for (int k = 0; k < 3; k++) {
+        bins.perNode[k] = 1.0/n[k];
+        bins.perTile[k] = 1.0/tiles[k];
+    }
+    return true;
 }
 
-void launchSpreadTiles(const double* positions, const int* particles, const uint32_t* mask, const ParticleArgs& a,
-        const SpreadBins& bins, unsigned long long* reactionFixed, uint32_t* touched, hipStream_t stream) {
-    (void) positions;
-    (void) particles;
+void launchSpreadTiles(const uint32_t* mask, const ParticleArgs& a, const SpreadBins& bins, unsigned long long* reactionFixed,
+        uint32_t* touched, hipStream_t stream) {
     unsigned grid = bins.ntx*bins.nty*bins.ntz;
     switch (coupleLanes(a.stencil)) {
     case 64:

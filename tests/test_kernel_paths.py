@@ -229,3 +229,39 @@ def test_centred_matrix_rows_match_the_spread(grid, beads, crowd, stencil, monke
     if crowd > 100:
         for a, b in zip(rows, spread):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("stencil,centred", [(LBMForce.NearestNode, False), (LBMForce.Trilinear, True),
+                                             (LBMForce.ThreePoint, False), (LBMForce.ThreePoint, True), (LBMForce.Keys, False),
+                                             (LBMForce.Keys, True)],
+                         ids=["nearest", "trilinear-centred", "threepoint", "threepoint-centred", "keys", "keys-centred"])
+@pytest.mark.parametrize("grid,beads", [((6, 6, 6), 20), ((32, 8, 7), 300), ((33, 7, 9), 900), ((64, 9, 10), 700),
+                                        ((67, 11, 6), 1500)])
+def test_tile_spread_on_any_periodic_lattice_is_that_of_the_atomics(grid, beads, stencil, centred, monkeypatch):
+    """The one-writer spread on lattices whose tiles are narrower than 32 x 4 x 4, down to 3 nodes: rows that share words of the
+    touched mask with other tiles, beads that reach back across the periodic faces, solid nodes and a crowd that overflows its
+    bin; the reactions are the atomics', bit for bit, over steps that use both sets of bins."""
+    rng = np.random.default_rng(beads)
+    pos = np.concatenate([rng.uniform(0, grid, size=(beads, 3)), rng.uniform(2.0, 2.3, size=(150, 3))])
+    s = Setup(grid, tau=0.8)
+    s.add_particles(pos, velocities=rng.normal(scale=0.3, size=pos.shape))
+
+    def conf(f):
+        f.setSolidNodes(list(range(grid[0])))
+        f.setWallScheme(LBMForce.BounceBack)
+        f.setFriction(10.0)
+        f.setTemperature(300.0)
+        f.setFluidFluctuations(True)
+        f.setRandomNumberSeed(5)
+        f.setDragScheme(LBMForce.Centered if centred else LBMForce.Explicit)
+        f.setInterpolationStencil(stencil)
+    s.configure.append(conf)
+    runs = []
+    for spread in ("atomic", "tiles"):
+        monkeypatch.setenv("LBM_AMD_SPREAD", spread)
+        c = s.build(None, storage=LBMForce.FP32)
+        c.step(5)
+        runs.append((c.getFluidState(), c.positions.copy(), c.velocities.copy(), c.getForces()))
+    assert np.abs(runs[0][0]).max() > 0
+    for a, b in zip(*runs):
+        assert np.array_equal(a, b)
