@@ -21,6 +21,7 @@
  * Everything runs in order on one HIP stream owned by the context.
  */
 #include "lbm_mlp.h"
+#include "lbm_between.h"
 #include <algorithm>
 #include <chrono>
 #include <cmath>
@@ -162,6 +163,8 @@ struct lbm_context {
     // adds the forces of the coupled particles itself (forcesAdded then says so, and no separate addForces runs).
     double* forceTarget = nullptr;
     bool forcesAdded = false;
+    // The particle host's work between this step and the next, offered to one lbm_execute_device (lbm_internal_offer_between).
+    BetweenSteps* between = nullptr;
     // Timing of the fused pass with HIP events on the context's stream (diagnostics).
     bool profile = false;
     std::vector<std::pair<hipEvent_t, hipEvent_t>> events;
@@ -402,14 +405,29 @@ void advanceFluid(lbm_context* c, const double* dPos, const double* dVel, const 
         HIP_CHECK(hipEventCreate(&ev.second));
         HIP_CHECK(hipEventRecord(ev.first, c->stream));
     }
-    launchFused(c->p.storage, c->fusedPath, c->mask != nullptr, particles, c->fluct(), c->popA, c->popB, c->mask,
-            c->reactionFixed, c->touched, c->nextTouched, c->ucm, a, c->stream);
+    // The particles' work between this step and the next joins the pass where there are no solid nodes to reflect at, else
+    // the bounce-back, once the forces on them are complete (the centred drag adds its own after the step).
+    BetweenSteps* between = !particles || c->forcesAdded ? c->between : nullptr;
+    const bool joinPass = between != nullptr && c->mask == nullptr && c->fusedPath == FUSED_DIRECT;
+    const bool joinWalls = between != nullptr && between->reflection.mask != nullptr && c->numWall > 0 && c->numBoundary == 0;
+    if (joinPass)
+        launchFusedBetween(c->p.storage, particles, c->fluct(), c->popA, c->popB, c->reactionFixed, c->touched,
+                c->nextTouched, c->ucm, a, *between, c->stream);
+    else
+        launchFused(c->p.storage, c->fusedPath, c->mask != nullptr, particles, c->fluct(), c->popA, c->popB, c->mask,
+                c->reactionFixed, c->touched, c->nextTouched, c->ucm, a, c->stream);
     std::swap(c->touched, c->nextTouched);
     if (c->profile) {
         HIP_CHECK(hipEventRecord(ev.second, c->stream));
         c->events.push_back(ev);
     }
-    if (c->numWall > 0)
+    if (joinWalls) {
+        between->busyOffset = c->wallBounceOffset;
+        between->busyCount = c->wallBoundaryOffset - c->wallBounceOffset;
+        launchBounceBackBetween(c->p.storage, c->popB, c->wallNodes, c->wallLinks, c->numWall, c->g,
+                c->wallPartials + 3*(size_t) c->wallBounceOffset, *between, c->stream);
+    }
+    else if (c->numWall > 0)
         launchBounceBack(c->p.storage, c->popB, c->wallNodes, c->wallLinks, c->numWall, c->g,
                 c->wallPartials + 3*(size_t) c->wallBounceOffset, c->stream);
     if (c->numBoundary > 0) {
@@ -435,6 +453,8 @@ void advanceFluid(lbm_context* c, const double* dPos, const double* dVel, const 
                 c->wallPartials + 3*(size_t) c->wallBoundaryOffset, c->stream);
     }
     HIP_CHECK(hipGetLastError());
+    if (joinPass || joinWalls)
+        between->taken = true;
     std::swap(c->popA, c->popB);
     c->wallStepDone = true;
     c->stepForcesCurrent = true;
@@ -834,6 +854,10 @@ void lbm_internal_begin_reflected(lbm_context* c, int64_t step) {
     beginState(c, step);
 }
 
+void lbm_internal_offer_between(lbm_context* c, BetweenSteps* b) {
+    c->between = b;
+}
+
 #define LBM_TRY(...) \
     try { __VA_ARGS__; g_lastError.clear(); return LBM_OK; } \
     catch (const Error& e) { return fail(e); } \
@@ -889,7 +913,10 @@ int lbm_execute_device(lbm_context* c, int64_t step, int includeForces, const do
     LBM_TRY({
         struct TargetScope {
             lbm_context* c;
-            ~TargetScope() { c->forceTarget = nullptr; }
+            ~TargetScope() {
+                c->forceTarget = nullptr;
+                c->between = nullptr;
+            }
         } scope{c};
         c->forceTarget = includeForces ? forces : nullptr;
         c->forcesAdded = false;

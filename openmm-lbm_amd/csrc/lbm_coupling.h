@@ -75,11 +75,13 @@ __device__ __forceinline__ bool reflectParticle(const double x[3], double v[3], 
     return true;
 }
 
-/* Clears the wall partial sums allPartials[0, 3*count) outside this grid's own slots, one per work-group of BLOCK threads
-   from ownOffset. */
-__device__ __forceinline__ void clearOtherPartials(double* __restrict__ allPartials, int count, int ownOffset) {
-    for (int j = blockIdx.x*BLOCK + threadIdx.x; j < 3*count; j += gridDim.x*BLOCK)
-        if (j < 3*ownOffset || j >= 3*(ownOffset + (int) gridDim.x))
+/* Clears the wall partial sums allPartials[0, 3*count) outside the own slots of the launch's first `blocks` work-groups, one
+   each from ownOffset, and outside the busyCount slots from busyOffset that its other work-groups write. */
+template <int THREADS>
+__device__ __forceinline__ void clearOtherPartials(double* __restrict__ allPartials, int count, int ownOffset, int blocks,
+        int busyOffset = 0, int busyCount = 0) {
+    for (int j = blockIdx.x*THREADS + threadIdx.x; j < 3*count; j += blocks*THREADS)
+        if ((j < 3*ownOffset || j >= 3*(ownOffset + blocks)) && (j < 3*busyOffset || j >= 3*(busyOffset + busyCount)))
             allPartials[j] = 0.0;
 }
 

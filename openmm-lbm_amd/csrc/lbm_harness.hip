@@ -5,13 +5,14 @@
  *   lbm_begin_step_device -> zero forces -> extra forces (wall potential, harmonic bonds)
  *   -> lbm_execute_device (adds the coupling forces) -> leapfrog Verlet update
  *      v(t+dt/2) = v(t-dt/2) + dt F(t)/m,  x(t+dt) = x(t) + dt v(t+dt/2).
- * Between two steps of one call the update, the next step's reflection and its other forces are one launch.
+ * Between two steps of one call the update, the next step's reflection and its other forces are work-groups of a launch of
+ * the lattice step, or one launch (lbm_between.h).
  * The extra forces are those of the benchmark configurations: a repulsive wall potential
  * eps[(sigma/d1)^12 + (sigma/d2)^12] between two planes z = zlo and z = zhi (the pattern of
  * the reference's examples/cocomo/shear.py:291-310), and harmonic bonds k/2 (r - r0)^2 with the
  * minimum image (bead chains, at most two bonds per particle), summed per particle in a fixed order.
  */
-#include "lbm_coupling.h"
+#include "lbm_between.h"
 #include <stdexcept>
 #include <utility>
 #include <vector>
@@ -41,58 +42,8 @@ struct MD {
 
 thread_local std::string g_err;
 
-/* The forces of the System other than the LBMForce. */
-struct OtherForces {
-    int wall;
-    double eps, sigma, zlo, zhi;
-    const int* partners;          // [particle][2], -1: none; nullptr without bonds
-    double k, r0;
-    double box[3];
-};
-
-/* Those on particle i at x: the repulsive walls U = eps[(s/d1)^12 + (s/d2)^12] along z (when set) plus the harmonic bonds
-   to the (at most two) chain partners, in that order.  partnerAt(j, xj): the position of particle j. */
-template <typename F>
-__device__ __forceinline__ void otherForcesOn(int i, const double x[3], const OtherForces& o, F&& partnerAt, double acc[3]) {
-    acc[0] = acc[1] = acc[2] = 0;
-    if (o.wall) {
-        double z = x[2];
-        double d1 = z - o.zlo, d2 = o.zhi - z;
-        // -dU/dz = 12 eps s^12/d1^13 - 12 eps s^12/d2^13.
-        double s1 = o.sigma/d1, s2 = o.sigma/d2;
-        double s1_12 = s1*s1*s1*s1*s1*s1*s1*s1*s1*s1*s1*s1, s2_12 = s2*s2*s2*s2*s2*s2*s2*s2*s2*s2*s2*s2;
-        acc[2] = 12.0*o.eps*(s1_12/d1 - s2_12/d2);
-    }
-    if (o.partners != nullptr) {
-        double b[3] = {0, 0, 0};
-        for (int p = 0; p < 2; p++) {
-            int j = o.partners[2*i + p];
-            if (j < 0)
-                continue;
-            double d[3], xj[3];
-            partnerAt(j, xj);
-            for (int a = 0; a < 3; a++) {
-                d[a] = xj[a] - x[a];
-                d[a] -= o.box[a]*rint(d[a]/o.box[a]);
-            }
-            double r = sqrt(d[0]*d[0] + d[1]*d[1] + d[2]*d[2]);
-            double s = r > 0 ? o.k*(r - o.r0)/r : 0.0;
-            for (int a = 0; a < 3; a++)
-                b[a] += s*d[a];
-        }
-        for (int a = 0; a < 3; a++)
-            acc[a] += b[a];
-    }
-}
-
-/* One component of the leapfrog update, its roundings written out: the merged launch forms a partner's new position
-   again, and every copy has to have the same bits. */
-__device__ __forceinline__ double newVelocity(double v, double f, double invMass, double dt) {
-    return fma(dt*f, invMass, v);
-}
-__device__ __forceinline__ double newPosition(double x, double v, double dt) {
-    return fma(dt, v, x);
-}
+using lbm::OtherForces;
+using lbm::BetweenSteps;
 
 /* The other forces, written (not added) for every particle. */
 __global__ void __launch_bounds__(lbm::BLOCK) otherForces(const double* __restrict__ pos, double* __restrict__ f, int n,
@@ -101,7 +52,7 @@ __global__ void __launch_bounds__(lbm::BLOCK) otherForces(const double* __restri
     if (i >= n)
         return;
     double x[3] = {pos[3*(size_t) i], pos[3*(size_t) i + 1], pos[3*(size_t) i + 2]}, acc[3];
-    otherForcesOn(i, x, o, [&](int j, double xj[3]) {
+    lbm::otherForcesOn(i, x, o, [&](int j, double xj[3]) {
         for (int a = 0; a < 3; a++)
             xj[a] = pos[3*(size_t) j + a];
     }, acc);
@@ -116,53 +67,20 @@ __global__ void __launch_bounds__(lbm::BLOCK) verlet(double* __restrict__ pos, d
         return;
     for (int a = 0; a < 3; a++) {
         size_t k = 3*(size_t) i + a;
-        double v = newVelocity(vel[k], f[k], invMass[i], dt);
+        double v = lbm::newVelocity(vel[k], f[k], invMass[i], dt);
         vel[k] = v;
-        pos[k] = newPosition(pos[k], v, dt);
+        pos[k] = lbm::newPosition(pos[k], v, dt);
     }
 }
 
 /*
- * What lies between two lattice steps for the particles, in one launch: the leapfrog update of the step that ends, the
- * reflection at solid nodes that begins the next one (REFLECT) and its other forces.  Each of the three is bound by its
- * launch (~5 us beside a large lattice pass, 2 us beside a small one), not by its work.  A step of 64 beads in 32^3
- * 22.4 -> 20.0 us, of 3,001 beads between walls in 150 x 117 x 86 84.6 -> 80.3 us, of 100,000 chain beads in 128^3
- * 318 -> 310 us.  It reads one set of particle arrays and writes the other: a bonded particle needs its partners' new
- * positions, which it forms again from their old values.
+ * The work between two steps in a launch of its own, where no launch of the lattice step takes it.  The update, the
+ * reflection and the other forces are each bound by their launch (~5 us beside a large lattice pass, 2 us beside a small one),
+ * not by their work: in one launch, a step of 64 beads in 32^3 22.4 -> 20.0 us, of 100,000 chain beads in 128^3 318 -> 310 us.
  */
 template <bool REFLECT>
-__global__ void __launch_bounds__(lbm::BLOCK) betweenSteps(const double* __restrict__ pos, const double* __restrict__ vel,
-        const double* __restrict__ f, const double* __restrict__ invMass, int n, double dt, OtherForces o,
-        lbm::StepReflection r, double* __restrict__ posOut, double* __restrict__ velOut, double* __restrict__ fOut) {
-    if constexpr (REFLECT)
-        lbm::clearOtherPartials(r.partials, r.count, r.ownOffset);
-    const int i = blockIdx.x*lbm::BLOCK + threadIdx.x;
-    double wallAcc[3] = {0, 0, 0};
-    if (i < n) {
-        auto moved = [&](int j, double x[3], double v[3]) {
-            for (int a = 0; a < 3; a++) {
-                const size_t k = 3*(size_t) j + a;
-                v[a] = newVelocity(vel[k], f[k], invMass[j], dt);
-                x[a] = newPosition(pos[k], v[a], dt);
-            }
-        };
-        double x[3], v[3], acc[3];
-        moved(i, x, v);
-        if constexpr (REFLECT)
-            lbm::reflectParticle(x, v, r.mass[i], r.mask, r.args, wallAcc);
-        otherForcesOn(i, x, o, [&](int j, double xj[3]) {
-            double vj[3];
-            moved(j, xj, vj);
-        }, acc);
-        for (int a = 0; a < 3; a++) {
-            const size_t k = 3*(size_t) i + a;
-            posOut[k] = x[a];
-            velOut[k] = v[a];
-            fOut[k] = acc[a];
-        }
-    }
-    if constexpr (REFLECT)
-        lbm::storeWallPartial<lbm::BLOCK>(wallAcc, r.partials + 3*(size_t) r.ownOffset);
+__global__ void __launch_bounds__(lbm::BLOCK) particlesBetween(BetweenSteps b) {
+    lbm::betweenSteps<REFLECT, lbm::BLOCK>(b, (int) gridDim.x);
 }
 
 void hipCheck(hipError_t e) {
@@ -277,20 +195,33 @@ int lbm_md_step(lbm_md_system* s, lbm_context* ctx, int64_t step0, int numSteps)
             }
             otherForces<<<grid, lbm::BLOCK, 0, stream>>>(md->pos, md->force, md->n, other);
         }
+        BetweenSteps between;
+        begun = t + 1 < numSteps && lbm_internal_reflection(ctx, step + 1, md->n, between.reflection);
+        if (begun) {
+            between.pos = md->pos;
+            between.vel = md->vel;
+            between.force = md->force;
+            between.invMass = md->invMass;
+            between.n = md->n;
+            between.dt = md->dt;
+            between.other = other;
+            between.posOut = md->nextPos;
+            between.velOut = md->nextVel;
+            between.forceOut = md->nextForce;
+            lbm_internal_offer_between(ctx, &between);
+        }
         status = lbm_execute_device(ctx, step, 1, md->pos, md->vel, md->force);
         if (status != LBM_OK) {
             g_err = lbm_last_error();
             return status;
         }
-        lbm::StepReflection reflection;
-        begun = t + 1 < numSteps && lbm_internal_reflection(ctx, step + 1, md->n, reflection);
         if (begun) {
-            if (reflection.mask != nullptr)
-                betweenSteps<true><<<grid, lbm::BLOCK, 0, stream>>>(md->pos, md->vel, md->force, md->invMass, md->n, md->dt,
-                        other, reflection, md->nextPos, md->nextVel, md->nextForce);
-            else
-                betweenSteps<false><<<grid, lbm::BLOCK, 0, stream>>>(md->pos, md->vel, md->force, md->invMass, md->n,
-                        md->dt, other, reflection, md->nextPos, md->nextVel, md->nextForce);
+            if (!between.taken) {
+                if (between.reflection.mask != nullptr)
+                    particlesBetween<true><<<grid, lbm::BLOCK, 0, stream>>>(between);
+                else
+                    particlesBetween<false><<<grid, lbm::BLOCK, 0, stream>>>(between);
+            }
             std::swap(md->pos, md->nextPos);
             std::swap(md->vel, md->nextVel);
             std::swap(md->force, md->nextForce);

@@ -233,6 +233,13 @@ void launchMomentReduce(int storage, bool solids, const void* src, const uint32_
 void launchFinishReduce(const double* partials, double numFluid, double* totals, double* ucm, hipStream_t stream);
 void launchBounceBack(int storage, void* dst, const int* wallNodes, const int* wallLinks, int count, const Geometry& g,
         double* partials, hipStream_t stream);
+/* The pass (FUSED_DIRECT, no solid nodes) and the bounce-back with the particles' work between the steps (lbm_between.h). */
+struct BetweenSteps;
+void launchFusedBetween(int storage, bool reaction, bool fluct, const void* src, void* dst,
+        unsigned long long* reactionFixed, const uint32_t* touched, uint32_t* nextTouched, const double* ucm, const StepArgs& a,
+        const BetweenSteps& between, hipStream_t stream);
+void launchBounceBackBetween(int storage, void* dst, const int* wallNodes, const int* wallLinks, int count,
+        const Geometry& g, double* partials, const BetweenSteps& between, hipStream_t stream);
 void launchBoundaries(int storage, const void* src, void* dst, const BoundaryNode* nodes, const double* ucm,
         const BoundaryArgs& a, double* partials, hipStream_t stream);
 void launchGather(int storage, const void* src, double* out, const Geometry& g, hipStream_t stream);

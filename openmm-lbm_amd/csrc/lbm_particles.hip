@@ -31,7 +31,7 @@ __global__ void __launch_bounds__(BLOCK) reflectParticles(const double* __restri
         const int* __restrict__ particles, const double* __restrict__ mass, const uint32_t* __restrict__ mask,
         ParticleArgs a, double* __restrict__ allPartials, int count, int ownOffset) {
     double* partials = allPartials + 3*(size_t) ownOffset;
-    clearOtherPartials(allPartials, count, ownOffset);
+    clearOtherPartials<BLOCK>(allPartials, count, ownOffset, (int) gridDim.x);
     double acc[3] = {0, 0, 0};
     int i = blockIdx.x*BLOCK + threadIdx.x;
     if (i < a.numParticles) {

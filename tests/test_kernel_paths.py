@@ -265,3 +265,35 @@ def test_tile_spread_on_any_periodic_lattice_is_that_of_the_atomics(grid, beads,
     assert np.abs(runs[0][0]).max() > 0
     for a, b in zip(*runs):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("storage", [LBMForce.FP16, LBMForce.FP32, LBMForce.FP64], ids=["fp16", "fp32", "fp64"])
+@pytest.mark.parametrize("beads,coupled,fluct", [(255, True, False), (257, True, True), (512, True, False),
+                                                 (513, True, False), (513, False, False)])
+def test_particles_in_front_of_the_lattice_pass_are_bit_identical(beads, coupled, fluct, storage):
+    """Eight steps in one call (the particles' work between the steps in the first work-groups of the pass) against eight
+    calls of one step (launches of its own), at the edges of the work-groups of 256 and 512, and for particles that the
+    fluid does not see."""
+    rng = np.random.default_rng(beads)
+    s = Setup((20, 9, 12), tau=0.7)
+    s.add_particles(rng.uniform(0, [20, 9, 12], size=(beads, 3)), velocities=rng.normal(size=(beads, 3)), coupled=coupled)
+
+    def conf(f):
+        f.setFriction(10.0)
+        f.setTemperature(300.0 if fluct else 0.0)
+        f.setFluidFluctuations(fluct)
+        f.setBodyAcceleration((0.1, 0.05, -0.02))
+        f.setRandomNumberSeed(9)
+        f.setInterpolationStencil(LBMForce.Trilinear)
+    s.configure.append(conf)
+    results = []
+    for calls, steps in ((1, 8), (8, 1)):
+        ctx = s.build(None, storage=storage)
+        dp = DeviceParticles(ctx)
+        dp.setBonds(np.stack([np.arange(beads - 1), np.arange(1, beads)], axis=1), 100.0, 0.5)
+        for _ in range(calls):
+            dp.step(steps)
+        pos, vel = dp.pull()
+        results.append((pos, vel, ctx.getFluidState()))
+    for a, b in zip(*results):
+        assert np.array_equal(a, b)
