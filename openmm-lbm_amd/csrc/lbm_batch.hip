@@ -1,8 +1,8 @@
 /*
  * Batched replicas (include/lbm_amd_batch.h): R independent periodic lattices advanced together.
  *
- * Per step, three launches cover every replica: coupleBatch (all particles), fusedBatch (all nodes, one work-group
- * per tile of one replica, looked up in tileReplica) and verletBatch (+ the step counter).  The step index lives in
+ * Per step, two launches cover every replica: coupleBatch (all particles) and fusedBatch (the Verlet update of all
+ * particles, then all nodes, one work-group per tile of one replica, looked up in tileReplica).  The step index lives in
  * device memory and the populations alternate between the two arrays by its parity, so the launches of a step are the
  * same at every step: the batch captures STEPS_PER_GRAPH steps into a hipGraph once and replays it.
  *
@@ -26,6 +26,9 @@ using namespace lbm;
 namespace {
 
 constexpr int STEPS_PER_GRAPH = 10;
+// Work-group size of the pass until lbm_batch_autotune chooses: its 82 registers leave room for five work-groups of 256 per CU
+// but two of 512 (32 replicas of up to 96^3: 201 and 218 us; the autotuner has chosen 256 for every batch measured).
+constexpr int BATCH_THREADS = 256;
 
 struct BatchError : public std::runtime_error {
     int status;
@@ -56,7 +59,7 @@ struct lbm_batch {
     ReplicaDesc* dDesc = nullptr;
     uint16_t* tileReplica = nullptr;
     uint32_t numTiles = 0;
-    int threads = FUSED_THREADS;
+    int threads = BATCH_THREADS;
     int coupleThreads = BLOCK;              // work-group size of the coupling (particles per tile: coupleThreads/lanes)
     int xcdOrder = 3;                       // bit 0: coupling tiles in XCD-contiguous runs, bit 1: fused tiles in
                                             // runs of XCD_CHUNK per XCD
@@ -69,7 +72,7 @@ struct lbm_batch {
     double* force = nullptr;
     double* mass = nullptr;        // lattice units (per replica cell mass)
     double* invMass = nullptr;     // 1/Da
-    int64_t* stepCounter = nullptr;
+    int64_t* stepCounter = nullptr;         // [2]: the coupling's, and the pass's where there are particles
     int64_t step = 0;
     int64_t totalNodes = 0;
     hipGraphExec_t graph = nullptr;
@@ -119,7 +122,7 @@ void buildTiles(lbm_batch* b, int threads) {
 
 void launchStep(lbm_batch* b, bool timed = false) {
     launchCoupleBatch(b->stencil, b->coupleThreads, b->dDesc, b->particleTiles, b->numParticleTiles, b->pos, b->vel,
-            b->mass, b->force, b->stepCounter, (b->xcdOrder & 1) != 0, b->stream);
+            b->mass, b->force, b->stepCounter, b->stepCounter + 1, (b->xcdOrder & 1) != 0, b->stream);
     std::pair<hipEvent_t, hipEvent_t> ev{nullptr, nullptr};
     if (timed) {
         hipCheck(hipEventCreate(&ev.first), "event");
@@ -127,12 +130,14 @@ void launchStep(lbm_batch* b, bool timed = false) {
         b->events.push_back(ev);
         hipCheck(hipEventRecord(ev.first, b->stream), "event");
     }
-    launchFusedBatch(b->threads, b->fluct, b->dDesc, b->tileReplica, b->numTiles, b->stepCounter,
-            (b->xcdOrder & 2) != 0, b->stream);
+    const BatchParticles particles = {b->particleReplica, b->numParticles, b->pos, b->vel, b->force, b->invMass};
+    launchFusedBatch(b->threads, b->fluct, b->dDesc, b->tileReplica, b->numTiles,
+            b->numParticles > 0 ? b->stepCounter + 1 : b->stepCounter, b->stepCounter, particles, (b->xcdOrder & 2) != 0,
+            b->stream);
     if (timed)
         hipCheck(hipEventRecord(ev.second, b->stream), "event");
-    launchVerletBatch(b->dDesc, b->particleReplica, b->numParticles, b->pos, b->vel, b->force, b->invMass,
-            b->stepCounter, b->stream);
+    if (b->numParticles == 0)
+        launchAdvanceStep(b->stepCounter, b->stream);
 }
 
 void buildGraph(lbm_batch* b) {
@@ -310,7 +315,7 @@ void createBatch(lbm_batch* b, int R, const lbm_params* params, const int* numPa
     b->force = alloc<double>(3*np, "forces");
     b->mass = alloc<double>(np, "masses");
     b->invMass = alloc<double>(np, "masses");
-    b->stepCounter = alloc<int64_t>(1, "step counter");
+    b->stepCounter = alloc<int64_t>(2, "step counter");
     if (np > 0) {
         hipCheck(hipMemcpyAsync(b->particleReplica, particleReplica.data(), np*sizeof(uint16_t), hipMemcpyHostToDevice, b->stream), "upload");
         hipCheck(hipMemcpyAsync(b->pos, positions, 3*np*sizeof(double), hipMemcpyHostToDevice, b->stream), "upload");
@@ -318,10 +323,10 @@ void createBatch(lbm_batch* b, int R, const lbm_params* params, const int* numPa
         hipCheck(hipMemcpyAsync(b->mass, latticeMass.data(), np*sizeof(double), hipMemcpyHostToDevice, b->stream), "upload");
         hipCheck(hipMemcpyAsync(b->invMass, invMass.data(), np*sizeof(double), hipMemcpyHostToDevice, b->stream), "upload");
     }
-    hipCheck(hipMemsetAsync(b->stepCounter, 0, sizeof(int64_t), b->stream), "memset");
+    hipCheck(hipMemsetAsync(b->stepCounter, 0, 2*sizeof(int64_t), b->stream), "memset");
     hipCheck(hipStreamSynchronize(b->stream), "sync");
     buildParticleTiles(b, BLOCK);
-    buildTiles(b, FUSED_THREADS);
+    buildTiles(b, BATCH_THREADS);
     buildGraph(b);
 }
 

@@ -156,32 +156,73 @@ fusedRows(const S* __restrict__ src, S* __restrict__ dst,
             elementOf<uint32_t>(a.g, i, j, k));
 }
 
+/* *p, the same for the whole work-group and written by no kernel that runs meanwhile: by scalar loads. */
+template <typename T>
+__device__ __forceinline__ T scalarLoad(const T* p) {
+    static_assert(sizeof(T) % 4 == 0, "whole words");
+    struct Words {
+        uint32_t w[sizeof(T)/4];
+    } words;
+    const auto* from = (const __attribute__((address_space(4))) uint32_t*) (uintptr_t) p;
+#pragma unroll
+    for (size_t i = 0; i < sizeof(T)/4; i++)
+        words.w[i] = from[i];
+    return __builtin_bit_cast(T, words);
+}
+
 /*
  * The same pass over every replica of a batch in one launch: work-group b covers THREADS nodes of replica
- * tileReplica[b].  The step index comes from device memory, so one captured launch serves every step.
+ * tileReplica[b].  The step index comes from device memory, so one captured launch serves every step.  The first
+ * particleBlocks work-groups (a multiple of 8, which keeps a tile's XCD) are the leapfrog Verlet update of the particles,
+ * whose only force is the coupling's, and advance the step counter that the coupling reads; the pass reads the copy that the
+ * coupling made.  As launches of their own the two took 9.5 of the 325 us of a step of 32 replicas of up to 96^3.
  */
 template <bool FLUCT, int THREADS>
 __global__ void __launch_bounds__(THREADS) fusedBatch(const ReplicaDesc* __restrict__ table,
-        const uint16_t* __restrict__ tileReplica, const int64_t* __restrict__ stepCounter, int xcdOrder) {
+        const uint16_t* __restrict__ tileReplica, const int64_t* __restrict__ stepCounter, int64_t* __restrict__ nextCounter, BatchParticles p,
+        uint32_t particleBlocks, int xcdOrder) {
+    if (blockIdx.x < particleBlocks) {
+        if (blockIdx.x == 0 && threadIdx.x == 0)
+            *nextCounter = *stepCounter + 1;
+        const int i = blockIdx.x*THREADS + threadIdx.x;
+        if (i < p.count) {
+            const double dt = table[p.replica[i]].dt;
+            for (int k = 0; k < 3; k++) {
+                const size_t at = 3*(size_t) i + k;
+                const double v = p.velocities[at] + dt*p.forces[at]*p.invMass[i];
+                p.velocities[at] = v;
+                p.positions[at] += dt*v;
+            }
+        }
+        return;
+    }
+    const uint32_t block = blockIdx.x - particleBlocks;
     // Runs of 64 neighbouring tiles per XCD: the batched config4 pass (17.6 M nodes in 64 replicas) 0.476 -> 0.465 ms,
     // its reads' overfetch at tile borders shared in one L2 (runs of 128: 0.468 ms; of 256 or one run per XCD: none).
-    const uint32_t tile = xcdOrder ? xcdChunkedTile(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t tile = xcdOrder ? xcdChunkedTile(block, gridDim.x - particleBlocks) : block;
     const ReplicaDesc* d = table + tileReplica[tile];
-    StepArgs a = d->step;
-    a.step = *stepCounter;
+    StepArgs a = scalarLoad(&d->step);
+    a.step = scalarLoad(stepCounter);
     a.roundSeed = 0;
-    const float* src = (a.step & 1) ? d->popB : d->popA;
-    float* dst = (a.step & 1) ? d->popA : d->popB;
-    fusedNode<float, false, true, FLUCT>(src, dst, nullptr, d->reactionFixed, (a.step & 1) ? d->touchedB : d->touchedA,
-            (a.step & 1) ? d->touchedA : d->touchedB, nullptr, a, (tile - d->tileBegin)*THREADS + threadIdx.x);
+    const bool odd = (a.step & 1) != 0;
+    float* popA = scalarLoad(&d->popA);
+    float* popB = scalarLoad(&d->popB);
+    uint32_t* touchedA = scalarLoad(&d->touchedA);
+    uint32_t* touchedB = scalarLoad(&d->touchedB);
+    fusedNode<float, false, true, FLUCT>(odd ? popB : popA, odd ? popA : popB, nullptr, scalarLoad(&d->reactionFixed),
+            odd ? touchedB : touchedA, odd ? touchedA : touchedB, nullptr, a,
+            (tile - scalarLoad(&d->tileBegin))*THREADS + threadIdx.x);
 }
 
 void launchFusedBatch(int threads, bool fluct, const ReplicaDesc* table, const uint16_t* tileReplica, uint32_t numTiles,
-        const int64_t* stepCounter, bool xcdOrder, hipStream_t stream) {
+        const int64_t* stepCounter, int64_t* nextCounter, const BatchParticles& particles, bool xcdOrder, hipStream_t stream) {
+    const uint32_t particleBlocks = ((uint32_t) ((particles.count + threads - 1)/threads) + 7)/8*8;
 #define LBM_BATCH_CASE(T) \
     case T: \
-        if (fluct) fusedBatch<true, T><<<numTiles, T, 0, stream>>>(table, tileReplica, stepCounter, xcdOrder); \
-        else fusedBatch<false, T><<<numTiles, T, 0, stream>>>(table, tileReplica, stepCounter, xcdOrder); \
+        if (fluct) fusedBatch<true, T><<<particleBlocks + numTiles, T, 0, stream>>>(table, tileReplica, stepCounter, \
+                nextCounter, particles, particleBlocks, xcdOrder); \
+        else fusedBatch<false, T><<<particleBlocks + numTiles, T, 0, stream>>>(table, tileReplica, stepCounter, \
+                nextCounter, particles, particleBlocks, xcdOrder); \
         break;
     switch (threads) {
     LBM_BATCH_CASE(256)

@@ -207,14 +207,22 @@ __device__ __forceinline__ uint32_t xcdChunkedTile(uint32_t b, uint32_t n) {
 
 /* Host-side launchers (defined in lbm_fluid.hip / lbm_particles.hip); xcdOrder: coupling tiles by xcdContiguousTile,
    fused tiles by xcdChunkedTile. */
+/* The particles of a batch, for the Verlet update in the first work-groups of the pass (count 0: none). */
+struct BatchParticles {
+    const uint16_t* replica;
+    int count;
+    double* positions;
+    double* velocities;
+    const double* forces;
+    const double* invMass;
+};
 void launchFusedBatch(int threads, bool fluct, const ReplicaDesc* table, const uint16_t* tileReplica, uint32_t numTiles,
-        const int64_t* stepCounter, bool xcdOrder, hipStream_t stream);
+        const int64_t* stepCounter, int64_t* nextCounter, const BatchParticles& particles, bool xcdOrder, hipStream_t stream);
 void launchCoupleBatch(int stencil, int threads, const ReplicaDesc* table, const uint16_t* particleTiles,
         int numParticleTiles, const double* positions, const double* velocities, const double* mass, double* forces,
-        const int64_t* stepCounter, bool xcdOrder, hipStream_t stream);
+        const int64_t* stepCounter, int64_t* passCounter, bool xcdOrder, hipStream_t stream);
 int coupleLanes(int stencil);
-void launchVerletBatch(const ReplicaDesc* table, const uint16_t* particleReplica, int numParticles, double* positions,
-        double* velocities, const double* forces, const double* invMass, int64_t* stepCounter, hipStream_t stream);
+void launchAdvanceStep(int64_t* stepCounter, hipStream_t stream);
 /* Which fused-pass kernel a context runs: fusedStep with 32-bit or 64-bit offsets, or fusedRows (LDS-staged pulls). */
 enum FusedPath { FUSED_DIRECT = 0, FUSED_WIDE = 1, FUSED_ROWS = 2 };
 bool fusedRowsFit(uint32_t nx, bool wide, uint32_t rowShift);

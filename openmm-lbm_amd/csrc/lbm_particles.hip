@@ -549,7 +549,7 @@ template <int LANES, int THREADS>
 __global__ void __launch_bounds__(THREADS) coupleBatch(const ReplicaDesc* __restrict__ table,
         const uint16_t* __restrict__ particleTiles, const double* __restrict__ positions,
         const double* __restrict__ velocities, const double* __restrict__ mass, double* __restrict__ forces,
-        const int64_t* __restrict__ stepCounter, int xcdOrder) {
+        const int64_t* __restrict__ stepCounter, int64_t* __restrict__ passCounter, int xcdOrder) {
     constexpr int GROUPS = THREADS/LANES;
     int lane = threadIdx.x % LANES;
     const uint32_t tile = xcdOrder ? xcdContiguousTile(blockIdx.x, gridDim.x) : blockIdx.x;
@@ -559,6 +559,8 @@ __global__ void __launch_bounds__(THREADS) coupleBatch(const ReplicaDesc* __rest
     int pp = d->particleBegin + (active ? local : 0);
     ParticleArgs a = d->part;
     a.step = *stepCounter;
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        *passCounter = a.step;
     a.isStep = 1;
     const float* src = (a.step & 1) ? d->popB : d->popA;
     const double* vel = velocities + 3*(size_t) pp;
@@ -582,23 +584,7 @@ __global__ void __launch_bounds__(THREADS) coupleBatch(const ReplicaDesc* __rest
             (a.step & 1) ? d->touchedB : d->touchedA, wallAcc, myNoise, nullptr, &staged);
 }
 
-/* Leapfrog Verlet of the batch (the coupling force is the only force).  The step counter is advanced by advanceStep,
-   launched after this kernel on the same stream. */
-__global__ void __launch_bounds__(BLOCK) verletBatch(const ReplicaDesc* __restrict__ table,
-        const uint16_t* __restrict__ particleReplica, int numParticles, double* __restrict__ positions,
-        double* __restrict__ velocities, const double* __restrict__ forces, const double* __restrict__ invMass) {
-    int p = blockIdx.x*BLOCK + threadIdx.x;
-    if (p >= numParticles)
-        return;
-    double dt = table[particleReplica[p]].dt;
-    for (int k = 0; k < 3; k++) {
-        size_t idx = 3*(size_t) p + k;
-        double v = velocities[idx] + dt*forces[idx]*invMass[p];
-        velocities[idx] = v;
-        positions[idx] += dt*v;
-    }
-}
-
+/* The step counter of a batch without particles (else the pass's particle work-groups advance it). */
 __global__ void advanceStep(int64_t* stepCounter) {
     if (threadIdx.x == 0)
         *stepCounter += 1;
@@ -718,54 +704,50 @@ void launchCouple(int storage, const void* src, const uint32_t* mask, const doub
 template <int LANES>
 static void launchCoupleBatchT(int threads, unsigned grid, const ReplicaDesc* table, const uint16_t* particleTiles,
         const double* positions, const double* velocities, const double* mass, double* forces,
-        const int64_t* stepCounter, bool xcdOrder, hipStream_t stream) {
+        const int64_t* stepCounter, int64_t* passCounter, bool xcdOrder, hipStream_t stream) {
     switch (threads) {
     case 64:
         coupleBatch<LANES, 64><<<grid, 64, 0, stream>>>(table, particleTiles, positions, velocities, mass, forces,
-                stepCounter, xcdOrder);
+                stepCounter, passCounter, xcdOrder);
         break;
     case 128:
         coupleBatch<LANES, 128><<<grid, 128, 0, stream>>>(table, particleTiles, positions, velocities, mass, forces,
-                stepCounter, xcdOrder);
+                stepCounter, passCounter, xcdOrder);
         break;
     default:
         coupleBatch<LANES, BLOCK><<<grid, BLOCK, 0, stream>>>(table, particleTiles, positions, velocities, mass, forces,
-                stepCounter, xcdOrder);
+                stepCounter, passCounter, xcdOrder);
         break;
     }
 }
 
 void launchCoupleBatch(int stencil, int threads, const ReplicaDesc* table, const uint16_t* particleTiles,
         int numParticleTiles, const double* positions, const double* velocities, const double* mass, double* forces,
-        const int64_t* stepCounter, bool xcdOrder, hipStream_t stream) {
+        const int64_t* stepCounter, int64_t* passCounter, bool xcdOrder, hipStream_t stream) {
     if (numParticleTiles == 0)
         return;
     unsigned grid = (unsigned) numParticleTiles;
     switch (coupleLanes(stencil)) {
     case 8:
         launchCoupleBatchT<8>(threads, grid, table, particleTiles, positions, velocities, mass, forces, stepCounter,
-                xcdOrder, stream);
+                passCounter, xcdOrder, stream);
         break;
     case 32:
         launchCoupleBatchT<32>(threads, grid, table, particleTiles, positions, velocities, mass, forces, stepCounter,
-                xcdOrder, stream);
+                passCounter, xcdOrder, stream);
         break;
     case 64:
         launchCoupleBatchT<64>(threads, grid, table, particleTiles, positions, velocities, mass, forces, stepCounter,
-                xcdOrder, stream);
+                passCounter, xcdOrder, stream);
         break;
     default:
         launchCoupleBatchT<1>(threads, grid, table, particleTiles, positions, velocities, mass, forces, stepCounter,
-                xcdOrder, stream);
+                passCounter, xcdOrder, stream);
         break;
     }
 }
 
-void launchVerletBatch(const ReplicaDesc* table, const uint16_t* particleReplica, int numParticles, double* positions,
-        double* velocities, const double* forces, const double* invMass, int64_t* stepCounter, hipStream_t stream) {
-    if (numParticles > 0)
-        verletBatch<<<gridFor(numParticles), BLOCK, 0, stream>>>(table, particleReplica, numParticles, positions,
-                velocities, forces, invMass);
+void launchAdvanceStep(int64_t* stepCounter, hipStream_t stream) {
     advanceStep<<<1, 64, 0, stream>>>(stepCounter);
 }
 

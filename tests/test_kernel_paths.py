@@ -7,10 +7,12 @@ import numpy as np
 import pytest
 
 from lbm_amd import LBMForce
+from lbm_amd.batch import Batch
 from lbm_amd.closure import MLPClosure, NUM_INPUTS, stats
 from lbm_amd.harness import DeviceParticles
 import oracle_lib
 from parity import Setup, lockstep
+from test_batch import make_replica, run_single
 
 sys.path.insert(0, os.path.join(oracle_lib.ROOT, "oracle"))
 import mlp_oracle as mo  # noqa: E402
@@ -297,3 +299,18 @@ def test_particles_in_front_of_the_lattice_pass_are_bit_identical(beads, coupled
         results.append((pos, vel, ctx.getFluidState()))
     for a, b in zip(*results):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("beads", [(0, 0), (0, 1), (200, 55), (256, 1), (1900, 149)])
+def test_batch_particles_in_front_of_the_pass_match_single_replicas(beads):
+    """The Verlet update in the first work-groups of the batched pass, without particles, at the edges of a work-group of
+    256 and of the 8 that are reserved at a time (2,048 particles and one more): the single-lattice runs' bits over replayed
+    and single steps."""
+    replicas = [make_replica((13, 9, 8), 0.7, beads[0], 2.5, 11, rng_seed=1), make_replica((8, 8, 33), 0.9, beads[1], 1.5, 7, rng_seed=2)]
+    batch = Batch(replicas)
+    batch.step(23)
+    batch.synchronize()
+    particles = batch.getParticles()
+    for r, replica in enumerate(replicas):
+        for a, b in zip(run_single(replica, 23), (*batch.getFluidFields(r), *particles[r])):
+            assert np.array_equal(a, b)
