@@ -77,6 +77,7 @@ struct lbm_batch {
     int64_t totalNodes = 0;
     hipGraphExec_t graph = nullptr;
     std::vector<void*> buffers;
+    FieldStage fields;
     bool profiling = false;                                // eager steps with events around the fused pass
     std::vector<std::pair<hipEvent_t, hipEvent_t>> events;
 };
@@ -187,6 +188,7 @@ void destroyBatch(lbm_batch* b) {
         (void) hipGraphExecDestroy(b->graph);
     for (void* p : b->buffers)
         (void) hipFree(p);
+    b->fields.free();
     void* others[] = {b->dDesc, b->tileReplica, b->particleReplica, b->particleTiles, b->pos, b->vel, b->force, b->mass,
                       b->invMass,
                       b->stepCounter};
@@ -455,16 +457,19 @@ int lbm_batch_get_fluid_fields(lbm_batch* b, int r, double* density, double* vel
         const ReplicaDesc& d = b->desc[r];
         const lbm_params& p = b->params[r];
         size_t n = d.step.g.n;
-        double* dRho = alloc<double>(n, "fields");
-        double* dU = alloc<double>(3*n, "fields");
+        // 32 replicas read in turn: 5 ms of allocations, kept instead.
+        std::lock_guard<std::mutex> hold(b->fields.lock);
+        double* dRho = (double*) b->fields.get(4*n*sizeof(double));
+        if (dRho == nullptr)
+            throw BatchError(LBM_ERROR_RUNTIME, "fields: out of device memory");
+        double* dU = dRho + n;
         const float* cur = (b->step & 1) ? d.popB : d.popA;
         launchFields(LBM_STORAGE_FP32, cur, nullptr, d.step.g, FieldsLayout(), p.density, p.dx/p.dt, p.body_acceleration[0],
                 p.body_acceleration[1], p.body_acceleration[2], dRho, dU, b->stream);
         hipError_t e1 = density ? hipMemcpyAsync(density, dRho, n*sizeof(double), hipMemcpyDeviceToHost, b->stream) : hipSuccess;
         hipError_t e2 = velocity ? hipMemcpyAsync(velocity, dU, 3*n*sizeof(double), hipMemcpyDeviceToHost, b->stream) : hipSuccess;
         hipError_t e3 = hipStreamSynchronize(b->stream);
-        (void) hipFree(dRho);
-        (void) hipFree(dU);
+        (void) b->fields.done(dRho);
         hipCheck(e1, "download");
         hipCheck(e2, "download");
         hipCheck(e3, "sync");

@@ -171,6 +171,7 @@ struct lbm_context {
     // Step state (ReferenceLBMKernels.h:158-176).
     bool stepPending = false, stepForcesCurrent = false;
     int64_t stepIndex = 0;
+    FieldStage fields;
 
     bool fluct() const {
         return p.fluid_fluctuations && p.fluid_kT > 0;
@@ -544,6 +545,7 @@ void destroy(lbm_context* c) {
                        c->ucm, c->wallPartials, c->particles, c->mass, c->particleForce, c->reactionFixed,
                        c->touched, c->nextTouched, c->stagePos, c->stageVel,
                        c->closureOod, c->closureCounters, c->closureField, c->stageForce};
+    c->fields.free();
     for (void* b : buffers)
         if (b)
             (void) hipFree(b);
@@ -1017,7 +1019,10 @@ int lbm_get_fluid_fields(lbm_context* c, double* density, double* velocity, int 
             return LBM_OK;
         }
         // One staging buffer for both fields: n densities, then 3n velocities.
-        double* stage = deviceAlloc<double>(4*n);
+        std::lock_guard<std::mutex> hold(c->fields.lock);
+        double* stage = (double*) c->fields.get(4*n*sizeof(double));
+        if (stage == nullptr)
+            HIP_CHECK(hipErrorOutOfMemory);
         double* dRho = density ? stage : nullptr;
         double* dU = velocity ? stage + n : nullptr;
         try {
@@ -1033,10 +1038,10 @@ int lbm_get_fluid_fields(lbm_context* c, double* density, double* velocity, int 
         }
         catch (...) {
             (void) hipStreamSynchronize(c->stream);
-            (void) hipFree(stage);
+            (void) c->fields.done(stage);
             throw;
         }
-        HIP_CHECK(hipFree(stage));
+        HIP_CHECK(c->fields.done(stage));
     })
 }
 
