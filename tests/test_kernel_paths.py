@@ -314,3 +314,22 @@ def test_batch_particles_in_front_of_the_pass_match_single_replicas(beads):
     for r, replica in enumerate(replicas):
         for a, b in zip(run_single(replica, 23), (*batch.getFluidFields(r), *particles[r])):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("rows", [1, 5, 1506, 1507, 3013, 20000])
+def test_normalization_of_the_pairs_is_that_of_the_host(rows):
+    """The scales and bounds that training takes from its pairs, with rows at the edges of the work-groups' stride (131,072
+    values, 1,506.6 rows), against NumPy in FP64: the sums of at most 1.6 million squares agree to 1e-13, the largest
+    magnitudes exactly."""
+    rng = np.random.default_rng(rows)
+    x = rng.normal(scale=0.02, size=(rows, NUM_INPUTS)).astype(np.float32)
+    t = rng.normal(scale=0.3, size=(rows, 3)).astype(np.float32)
+    net = MLPClosure(seed=3)
+    net.train(x, t, epochs=1, batch=256, lr=1e-4, decay=0.9, seed=3)
+    got = net.getNormalization()
+    u, v = x[:, 3:84].astype(np.float64), x[:, 84:].astype(np.float64)
+    scales = [1/np.sqrt((a*a).mean()) for a in (u, v, t.astype(np.float64))]
+    want = dict(u_scale=scales[0], v_scale=scales[1], out_scale=scales[2], u_bound=np.abs(u).max()*scales[0],
+                v_bound=np.abs(v).max()*scales[1])
+    for name, value in want.items():
+        assert abs(got[name] - value) <= 1e-13*value, name
