@@ -937,7 +937,7 @@ __global__ void __launch_bounds__(64) cgRowsCheck(const double* __restrict__ par
 template <int LANES, bool BINNED>
 __global__ void __launch_bounds__(BLOCK) cgForces(int n, ParticleArgs a, CgArgs c, double* __restrict__ particleForce,
         unsigned long long* __restrict__ reactionFixed, uint32_t* __restrict__ touched, double* __restrict__ partials,
-        const int* __restrict__ rowCount, SpreadBins bins) {
+        const int* __restrict__ rowCount, SpreadBins bins, const int* __restrict__ particles, double* __restrict__ systemForce) {
     // With matrix rows the host launches this before it knows whether the solve has converged.
     if (rowCount != nullptr && c.scalars[DONE] == 0.0)
         return;
@@ -953,9 +953,13 @@ __global__ void __launch_bounds__(BLOCK) cgForces(int n, ParticleArgs a, CgArgs 
     if (rank < n) {
         const int i = particleAt(c, rank);
         double F[3] = {c.F[3*(size_t) i], c.F[3*(size_t) i + 1], c.F[3*(size_t) i + 2]};
-        if (lane == 0)
-            for (int k = 0; k < 3; k++)
-                particleForce[3*(size_t) i + k] = F[k]*a.forceScale;
+        if (lane < 3) {
+            const double f = (lane == 0 ? F[0] : (lane == 1 ? F[1] : F[2]))*a.forceScale;
+            particleForce[3*(size_t) i + lane] = f;
+            // As groupForce: atomically, in case a particle were coupled twice.
+            if (systemForce != nullptr)
+                atomicAdd(systemForce + 3*(size_t) particles[i] + lane, f);
+        }
         if constexpr (BINNED) {
             int full = 0;
             if (a.isStep && lane == 0) {
@@ -1270,8 +1274,8 @@ template <typename S>
 void centredCoupleT(CentredState* st, const S* src, const uint32_t* mask, const double* positions,
         const double* velocities, const double* otherForces, const int* particles, const double* mass,
         const double* ucm, const ParticleArgs& a, const double g[3], const double4* field, const int* order,
-        const SpreadBins* bins, double* particleForce, unsigned long long* reactionFixed, uint32_t* touched, double* partials,
-        hipStream_t stream) {
+        const SpreadBins* bins, double* particleForce, double* systemForce, unsigned long long* reactionFixed, uint32_t* touched,
+        double* partials, hipStream_t stream) {
     int n = a.numParticles;
     if (n == 0)
         return;
@@ -1317,15 +1321,15 @@ void centredCoupleT(CentredState* st, const S* src, const uint32_t* mask, const 
             switch (st->lanes) {
             case 8:
                 cgForces<8, B><<<groups, BLOCK, 0, stream>>>(n, a, c, particleForce, reactionFixed, touched, partials, rowCount,
-                        spread);
+                        spread, particles, systemForce);
                 break;
             case 32:
                 cgForces<32, B><<<groups, BLOCK, 0, stream>>>(n, a, c, particleForce, reactionFixed, touched, partials, rowCount,
-                        spread);
+                        spread, particles, systemForce);
                 break;
             default:
                 cgForces<64, B><<<groups, BLOCK, 0, stream>>>(n, a, c, particleForce, reactionFixed, touched, partials, rowCount,
-                        spread);
+                        spread, particles, systemForce);
                 break;
             }
         };
@@ -1399,24 +1403,24 @@ void centredCoupleT(CentredState* st, const S* src, const uint32_t* mask, const 
 void centredCouple(CentredState* st, int storage, const void* src, const uint32_t* mask, const double* positions,
         const double* velocities, const double* otherForces, const int* particles, const double* mass,
         const double* ucm, const ParticleArgs& a, const double g[3], const double4* field, const int* order,
-        const SpreadBins* bins, double* particleForce, unsigned long long* reactionFixed, uint32_t* touched, double* partials,
-        hipStream_t stream) {
+        const SpreadBins* bins, double* particleForce, double* systemForce, unsigned long long* reactionFixed, uint32_t* touched,
+        double* partials, hipStream_t stream) {
     switch (storage) {
     case LBM_STORAGE_FP16:
         centredCoupleT<__half>(st, (const __half*) src, mask, positions, velocities, otherForces, particles, mass, ucm, a,
-                g, field, order, bins, particleForce, reactionFixed, touched, partials, stream);
+                g, field, order, bins, particleForce, systemForce, reactionFixed, touched, partials, stream);
         break;
     case LBM_STORAGE_BF16:
         centredCoupleT<__hip_bfloat16>(st, (const __hip_bfloat16*) src, mask, positions, velocities, otherForces,
-                particles, mass, ucm, a, g, field, order, bins, particleForce, reactionFixed, touched, partials, stream);
+                particles, mass, ucm, a, g, field, order, bins, particleForce, systemForce, reactionFixed, touched, partials, stream);
         break;
     case LBM_STORAGE_FP64:
         centredCoupleT<double>(st, (const double*) src, mask, positions, velocities, otherForces, particles, mass, ucm, a,
-                g, field, order, bins, particleForce, reactionFixed, touched, partials, stream);
+                g, field, order, bins, particleForce, systemForce, reactionFixed, touched, partials, stream);
         break;
     default:
         centredCoupleT<float>(st, (const float*) src, mask, positions, velocities, otherForces, particles, mass, ucm, a,
-                g, field, order, bins, particleForce, reactionFixed, touched, partials, stream);
+                g, field, order, bins, particleForce, systemForce, reactionFixed, touched, partials, stream);
         break;
     }
 }

@@ -361,7 +361,8 @@ void couple(lbm_context* c, const double* dPos, const double* dVel, const double
                     c->stream);
         centredCouple(c->centred, c->p.storage, c->popA, c->mask, dPos, dVel, dForces, c->particles, c->mass, c->ucm, a,
                 c->p.body_acceleration, c->momentField, order, bins, c->particleForce,
-                c->reactionFixed, c->touched, partials, c->stream);
+                c->forceTarget, c->reactionFixed, c->touched, partials, c->stream);
+        c->forcesAdded = c->forceTarget != nullptr && c->p.interpolation_stencil != LBM_STENCIL_NEAREST;
         if (bins != nullptr)
             c->binParity ^= 1;           // not after a solve that failed: its bins stay empty
         return;
@@ -407,7 +408,7 @@ void advanceFluid(lbm_context* c, const double* dPos, const double* dVel, const 
         HIP_CHECK(hipEventRecord(ev.first, c->stream));
     }
     // The particles' work between this step and the next joins the pass where there are no solid nodes to reflect at, else
-    // the bounce-back, once the forces on them are complete (the centred drag adds its own after the step).
+    // the bounce-back, once the forces on them are complete (the centred drag's with the nearest node are added after the step).
     BetweenSteps* between = !particles || c->forcesAdded ? c->between : nullptr;
     const bool joinPass = between != nullptr && c->mask == nullptr && c->fusedPath == FUSED_DIRECT;
     const bool joinWalls = between != nullptr && between->reflection.mask != nullptr && c->numWall > 0 && c->numBoundary == 0;

@@ -315,14 +315,16 @@ void launchParticleNodes(const double* positions, const int* particles, const Pa
    (kJ/mol/nm, all System particles, may be null) are the forces on the particles before the coupling; g is the body
    acceleration in lattice units; field: the moments of the nodes (launchMomentField) for the stencils of dense particles,
    or nullptr; order: the particles in the order to process their stencils (coupleOrderAt), or nullptr; bins: the tile spread's,
-   for the reactions of a step, or nullptr (slotWeight unused).  Throws std::runtime_error. */
+   for the reactions of a step, or nullptr (slotWeight unused); systemForce: the caller's force array to add the forces to with a
+   stencil, or nullptr.  Throws std::runtime_error. */
 struct CentredState;
 CentredState* centredCreate(int numParticles, int stencil, const Geometry& g);
 void centredDestroy(CentredState* state);
 void centredCouple(CentredState* state, int storage, const void* src, const uint32_t* mask, const double* positions,
         const double* velocities, const double* otherForces, const int* particles, const double* mass,
         const double* ucm, const ParticleArgs& a, const double g[3], const double4* field, const int* order, const SpreadBins* bins,
-        double* particleForce, unsigned long long* reactionFixed, uint32_t* touched, double* partials, hipStream_t stream);
+        double* particleForce, double* systemForce, unsigned long long* reactionFixed, uint32_t* touched, double* partials,
+        hipStream_t stream);
 
 /*
  * The reflection at solid nodes that begins a step, for a caller that runs it in a kernel of its own (the device-resident

@@ -333,3 +333,31 @@ def test_normalization_of_the_pairs_is_that_of_the_host(rows):
                 v_bound=np.abs(v).max()*scales[1])
     for name, value in want.items():
         assert abs(got[name] - value) <= 1e-13*value, name
+
+
+@pytest.mark.parametrize("stencil,grid", [(LBMForce.NearestNode, (20, 9, 12)), (LBMForce.Keys, (20, 9, 12)), (LBMForce.Keys, (20, 14, 12))],
+                         ids=["nearest", "keys-spread", "keys-rows"])
+def test_centred_device_steps_are_those_of_the_host(stencil, grid):
+    """The centred drag's forces added to the caller's array by the solve (stencils) or after the step (nearest node), with
+    every other particle coupled: eight device-resident steps in one call, the particles' work between them in the pass or in
+    a launch of its own, against the host's steps, which add the forces themselves (the rounding of the positions and
+    velocities over eight steps: 1e-12)."""
+    rng = np.random.default_rng(3)
+    s = Setup(grid, tau=0.8)
+    for i in range(80):
+        s.add_particles(rng.uniform(0, grid), velocities=rng.normal(scale=0.3, size=(1, 3)), coupled=i % 2 == 0)
+
+    def conf(f):
+        f.setFriction(10.0)
+        f.setTemperature(300.0)
+        f.setRandomNumberSeed(9)
+        f.setDragScheme(LBMForce.Centered)
+        f.setInterpolationStencil(stencil)
+    s.configure.append(conf)
+    host, device = s.build(None, storage=LBMForce.FP64), s.build(None, storage=LBMForce.FP64)
+    host.step(8)
+    dp = DeviceParticles(device)
+    dp.step(8)
+    pos, vel = dp.pull()
+    assert np.abs(pos - host.positions).max() <= 1e-12*max(grid)
+    assert np.abs(vel - host.velocities).max() <= 1e-12*np.abs(host.velocities).max()
