@@ -246,8 +246,8 @@ struct CgRows {
     CellEntry* cell = nullptr;       // [cell][CELL_CAP]
     uint32_t* home = nullptr;        // [rank][4]: the particle's cell along each axis, and its offset there
     double* axisWeight = nullptr;    // [rank][3][3w - 2]: the weights along each axis between w - 1 zeros on either side
-    int* rowCount = nullptr;         // [rank]
-    int* rowParticle = nullptr;      // [rank][ROW_CAP]
+    int* rowCount = nullptr;         // [particle]
+    int* rowParticle = nullptr;      // [particle][ROW_CAP]
     double* rowValue = nullptr;
     int* overflow = nullptr;
 };
@@ -471,6 +471,7 @@ __global__ void __launch_bounds__(BLOCK) cgRows(int n, int nx, int ny, int nz, C
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const size_t i = (size_t) particleAt(c, rank);
     double acc[3] = {0, 0, 0};
     for (int e = lane; e < found; e += 64) {
         const int from = f.sorted[e], l = f.particle[from];
@@ -493,17 +494,16 @@ __global__ void __launch_bounds__(BLOCK) cgRows(int n, int nx, int ny, int nz, C
             }
             value = fma(plane, wl[2][z], value);
         }
-        rows.rowParticle[(size_t) rank*ROW_CAP + e] = l;
-        rows.rowValue[(size_t) rank*ROW_CAP + e] = value;
+        rows.rowParticle[i*ROW_CAP + e] = l;
+        rows.rowValue[i*ROW_CAP + e] = value;
         for (int k = 0; k < 3; k++)
             acc[k] = fma(value, c.F[3*(size_t) l + k], acc[k]);
     }
     for (int k = 0; k < 3; k++)
         acc[k] = groupSum<64>(acc[k]);
     if (lane == 0)
-        rows.rowCount[rank] = found;
+        rows.rowCount[i] = found;
     if (lane < 3) {
-        const size_t i = (size_t) particleAt(c, rank);
         const double own = lane == 0 ? acc[0] : (lane == 1 ? acc[1] : acc[2]);
         c.Ad[3*i + lane] = c.F[3*i + lane]*((1.0 + aa)/mass[i]) + own*aa;
     }
@@ -820,7 +820,9 @@ __global__ void __launch_bounds__(BLOCK) cgDirection(int n, CgArgs c, const doub
  * side, [particle][z, d], one gather for both (20.7 -> 16.8 us for 56,320 Keys particles, bound by these gathers); d goes to
  * the other of two such arrays, since the neighbours read the old one, and the update puts the new z beside it.  Tests the
  * residual first, as the direction after a converged iteration is not needed.  With cgUpdate, two launches per iteration
- * where the spread takes six.
+ * where the spread takes six.  The particles are taken by index, not by their place in the processing order, which depends
+ * on when it was last sorted: d.Ad must be the same sum in a run that was restarted (a step of 56,320 Keys particles in
+ * 120^3 508 us by place, 503 by index; of 1,000,000 in 320^3 8.38 and 8.57 ms).
  */
 constexpr int ROW_LANES = 8, ROW_THREADS_CG = 1024;
 __global__ void __launch_bounds__(ROW_THREADS_CG) cgRowsStep(int n, CgArgs c, CgRows rows, const double* __restrict__ old,
@@ -868,13 +870,13 @@ __global__ void __launch_bounds__(ROW_THREADS_CG) cgRowsStep(int n, CgArgs c, Cg
     constexpr int PARTICLES = ROW_THREADS_CG/ROW_LANES;
     double dot = 0.0;                        // of component `lane`
     for (int base = (int) blockIdx.x*PARTICLES; base < n; base += RED_BLOCKS*PARTICLES) {
-        const int rank = base + t/ROW_LANES;
+        const int i = base + t/ROW_LANES;
         double s[3] = {0, 0, 0};
-        if (rank < n) {
-            const int count = rows.rowCount[rank];
+        if (i < n) {
+            const int count = rows.rowCount[i];
             for (int e = lane; e < count; e += ROW_LANES) {
-                const double2* from = (const double2*) (old + 6*(size_t) rows.rowParticle[(size_t) rank*ROW_CAP + e]);
-                const double value = rows.rowValue[(size_t) rank*ROW_CAP + e];
+                const double2* from = (const double2*) (old + 6*(size_t) rows.rowParticle[(size_t) i*ROW_CAP + e]);
+                const double value = rows.rowValue[(size_t) i*ROW_CAP + e];
                 const double2 a01 = from[0], a23 = from[1], a45 = from[2];
                 s[0] = fma(value, fma(beta[0], a23.y, a01.x), s[0]);
                 s[1] = fma(value, fma(beta[1], a45.x, a01.y), s[1]);
@@ -883,12 +885,12 @@ __global__ void __launch_bounds__(ROW_THREADS_CG) cgRowsStep(int n, CgArgs c, Cg
         }
         for (int k = 0; k < 3; k++)
             s[k] = groupSum<ROW_LANES>(s[k]);
-        if (rank < n && lane < 3) {
-            const size_t i = (size_t) particleAt(c, rank);
-            const double d = fma(lane == 0 ? beta[0] : (lane == 1 ? beta[1] : beta[2]), old[6*i + 3 + lane], old[6*i + lane]);
+        if (i < n && lane < 3) {
+            const size_t at = 6*(size_t) i + lane;
+            const double d = fma(lane == 0 ? beta[0] : (lane == 1 ? beta[1] : beta[2]), old[at + 3], old[at]);
             const double Ad = d*((1.0 + aa)/mass[i]) + (lane == 0 ? s[0] : (lane == 1 ? s[1] : s[2]))*aa;
-            next[6*i + 3 + lane] = d;
-            c.Ad[3*i + lane] = Ad;
+            next[at + 3] = d;
+            c.Ad[3*(size_t) i + lane] = Ad;
             dot = fma(d, Ad, dot);
         }
     }
@@ -993,7 +995,7 @@ __global__ void __launch_bounds__(BLOCK) cgForces(int n, ParticleArgs a, CgArgs 
                 bool solid = c.slotSolid[sl] != 0;
                 // With the split, a fluid slot that spreads nothing is alone at its node, and with matrix rows so is
                 // every slot of a particle without neighbours: a store, not an atomic.
-                const bool alone = BINNED ? false : rowCount != nullptr ? rowCount[rank] == 1 : c.split && c.slotSpreads[sl] == 0;
+                const bool alone = BINNED ? false : rowCount != nullptr ? rowCount[particleAt(c, rank)] == 1 : c.split && c.slotSpreads[sl] == 0;
                 if (alone && !solid && c.slotWInvRho[sl] != 0.0)
                     flagged = storeReaction(node, r, a, reactionFixed);
                 else if (solid)
