@@ -231,11 +231,13 @@ struct CgArgs {
  * nodes (the last cell of an axis takes the remainder, up to 7 nodes), so that those whose stencils reach a particle's lie in
  * the 27 cells around its own.  A row's entries are in the order of their particle, whatever the order in which the bins
  * were filled, so a solve is reproducible.  More than CELL_CAP particles in a cell or ROW_CAP in a row raise
- * `overflow`; the solve is then repeated with the spread.
+ * `overflow`, which ends the solve by rows before its first iteration; the spread then takes it from what cgSetup left.
+ * Each solve tries the rows anew: which of the two it takes depends on the particles alone, never on earlier solves, so
+ * that a restarted run takes the same.  A step of 5,000 Keys particles and a crowd of 140 in 48^3, the rows' attempt
+ * included: 403 us, 367 by the spread at once, 532 before there were rows.
  */
 constexpr int CELL_CAP = 64, ROW_CAP = 128;
 constexpr double ROWS_MEAN_NEIGHBOURS = 64.0;      // half of ROW_CAP
-constexpr int ROWS_RETRY = 128;                    // solves by the spread after an overflow
 struct CellEntry {
     int particle, rank;
     uint32_t offset;         // of its first stencil node within the cell, x | y << 3 | z << 6
@@ -401,7 +403,7 @@ __global__ void __launch_bounds__(BLOCK) cgRows(int n, int nx, int ny, int nz, C
     __shared__ Found all[WAVES];
     const int lane = (int) threadIdx.x & 63;
     const int rank = __builtin_amdgcn_readfirstlane((int) placeOf(c)*WAVES + (int) threadIdx.x/64);
-    if (rank >= n)
+    if (rank >= n || *rows.overflow != 0)
         return;
     // w/rho of the particle's slots: the same for every lane, so operands from scalar registers.
     const auto* own = (const __attribute__((address_space(4))) double*) (uintptr_t) (c.slotWInvRho + (size_t) rank*SLOTS);
@@ -704,8 +706,9 @@ __global__ void __launch_bounds__(BLOCK) cgInit(int n, CgArgs c, double* partial
     reduceBlock(w, 3, partialsB);
 }
 
+/* overflow: CgRows::overflow, or nullptr; with it set no iteration runs. */
 __global__ void __launch_bounds__(64) cgFinishInit(const double* __restrict__ partials,
-        const double* __restrict__ partialsB, double* __restrict__ scalars) {
+        const double* __restrict__ partialsB, double* __restrict__ scalars, const int* __restrict__ overflow) {
     double v[6], w[3];
     combinePartials<6>(partials, v);
     combinePartials<3>(partialsB, w);
@@ -716,7 +719,7 @@ __global__ void __launch_bounds__(64) cgFinishInit(const double* __restrict__ pa
         scalars[NORM + k] = v[3 + k];
         scalars[RR + k] = w[k];
     }
-    scalars[DONE] = residualConverged(scalars) ? 1.0 : 0.0;
+    scalars[DONE] = residualConverged(scalars) || (overflow != nullptr && *overflow != 0) ? 1.0 : 0.0;
     scalars[ITERS] = 0.0;
 }
 
@@ -916,7 +919,7 @@ __global__ void __launch_bounds__(64) cgRowsCheck(const double* __restrict__ par
     if (threadIdx.x != 0)
         return;
     bool done = scalars[DONE] != 0.0;
-    if (!done) {
+    if (!done && iterations > 0) {
         double test[NUM_SCALARS];
         for (int k = 0; k < 3; k++) {
             test[RR + k] = v[3 + k];
@@ -1053,11 +1056,11 @@ struct CentredState {
     double* hostScalars = nullptr;        // pinned: the convergence check reads the scalars
     int lastIterations = 1;               // iterations of the previous solve: enqueued before the first check
     bool planned = true;                  // false (LBM_AMD_CG_PLANNED=0): the host reads the residual after each
-    // The matrix rows and their two arrays of directions; retryRows: solves to go by the spread after an overflow.
+    // The matrix rows and their two arrays of directions.
     CgRows rows;
     int numCells = 0;
     double* directions[2] = {nullptr, nullptr};      // [particle][z, d]
-    int retryRows = 0;
+    bool crowded = false;                            // the previous solve's rows overflowed: look before the iterations
     hipEvent_t checked = nullptr;
     std::vector<void*> buffers;
 };
@@ -1227,7 +1230,8 @@ const char* const NOT_CONVERGED = "LBMForce: the centred drag with the interpola
 /*
  * The solve with the matrix rows, after cgSetup has binned the particles.  The forces (a launch that does nothing before the
  * solve has converged) go onto the stream ahead of the host's wait for the residual, so that the device works meanwhile.
- * Returns false if a bin or a row was too small.
+ * Returns false if a bin or a row was too small; c.F and the slots are then as cgSetup left them.  After such a solve the
+ * host looks for that before it enqueues iterations that would do nothing.
  */
 template <typename Forces>
 bool solveRows(CentredState* st, const Geometry& g, const double* mass, double aa, hipStream_t stream, Forces&& forces) {
@@ -1244,9 +1248,10 @@ bool solveRows(CentredState* st, const Geometry& g, const double* mass, double a
     c.z = st->directions[0];
     c.d = c.z + 3;
     cgInit<<<RED_BLOCKS, BLOCK, 0, stream>>>(n, c, st->partialsB, r.cellCount, st->numCells);
-    cgFinishInit<<<1, 64, 0, stream>>>(c.partials, st->partialsB, c.scalars);
+    cgFinishInit<<<1, 64, 0, stream>>>(c.partials, st->partialsB, c.scalars, r.overflow);
     int iteration = 0;
-    for (int batch = st->planned ? std::max(st->lastIterations, 1) : 1;; batch = 1) {
+    const int planned = st->planned ? std::max(st->lastIterations, 1) : 1;
+    for (int batch = st->crowded ? 0 : planned;; batch = iteration == 0 ? planned : 1) {
         for (int b = 0; b < batch; b++, iteration++) {
             c.z = st->directions[(iteration + 1) & 1];
             c.d = c.z + 3;
@@ -1259,7 +1264,8 @@ bool solveRows(CentredState* st, const Geometry& g, const double* mass, double a
         forces();
         check(hipGetLastError(), "launch");
         check(hipEventSynchronize(st->checked), "sync");
-        if (st->hostScalars[OVERFLOWED] != 0.0) {
+        st->crowded = st->hostScalars[OVERFLOWED] != 0.0;
+        if (st->crowded) {
             check(hipMemsetAsync(r.overflow, 0, sizeof(int), stream), "memset");
             return false;
         }
@@ -1342,15 +1348,9 @@ void centredCoupleT(CentredState* st, const S* src, const uint32_t* mask, const 
             launchSpreadTiles(mask, a, spread, reactionFixed, touched, stream);
         }
     };
-    if (st->rows.cell != nullptr && st->retryRows == 0) {
-        setup(st->rows);
-        if (solveRows(st, a.g, mass, aa, stream, [&] { forces(st->rows.rowCount); }))
-            return;
-        st->retryRows = ROWS_RETRY;
-    }
-    else if (st->retryRows > 0)
-        st->retryRows--;
-    setup(CgRows());
+    setup(st->rows);
+    if (st->rows.cell != nullptr && solveRows(st, a.g, mass, aa, stream, [&] { forces(st->rows.rowCount); }))
+        return;
     if (c.split)
         switch (st->lanes) {
         case 8: cgMarkShared<8><<<groups, BLOCK, 0, stream>>>(n, c); break;
@@ -1360,7 +1360,7 @@ void centredCoupleT(CentredState* st, const S* src, const uint32_t* mask, const 
     cgMaxAbs<<<RED_BLOCKS, BLOCK, 0, stream>>>(c.F, n, c.partials, nullptr);
     multiply<S>(st, c.F, c.Ad, mass, aa, nullptr, 1, true, stream);
     cgInit<<<RED_BLOCKS, BLOCK, 0, stream>>>(n, c, st->partialsB, nullptr, 0);
-    cgFinishInit<<<1, 64, 0, stream>>>(c.partials, st->partialsB, c.scalars);
+    cgFinishInit<<<1, 64, 0, stream>>>(c.partials, st->partialsB, c.scalars, nullptr);
     check(hipGetLastError(), "launch");
     // Each iteration starts with the new direction (d = z after cgInit), so that the last one computes none.  The
     // previous solve's count of iterations is enqueued at once (those after convergence do nothing), then the host

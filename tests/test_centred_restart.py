@@ -52,3 +52,28 @@ def test_restart_with_rows_is_bit_identical(grid, beads, stencil):
         assert np.abs(first[2]).max() > 0
         for a, b in zip(first, second):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("query", [False, True], ids=["steps", "queries"])
+def test_restart_after_a_crowd_dispersed_is_bit_identical(query):
+    """A crowd of 90 particles that start their stencils in one cell of 4^3 nodes (of 64 entries), so that the solves begin by
+    the spread, and then fly on into the next cells, so that they go by the rows: a Context that never saw the crowd takes
+    the same solves as one that did."""
+    grid, crowd = (24, 16, 16), 90
+    rng = np.random.default_rng(1)
+    s = Setup(grid, tau=0.8)
+    s.add_particles(rng.uniform(0, grid, size=(60, 3)), velocities=rng.normal(scale=0.2, size=(60, 3)))
+    s.add_particles(rng.uniform([5.05, 5.05, 5.05], [8.95, 8.95, 8.95], size=(crowd, 3)),
+                    velocities=np.tile([8.0, 0.0, 0.0], (crowd, 1)))
+
+    def conf(f):
+        f.setFriction(0.5)
+        f.setTemperature(300.0)
+        f.setRandomNumberSeed(5)
+        f.setDragScheme(LBMForce.Centered)
+        f.setInterpolationStencil(LBMForce.Keys)
+    s.configure.append(conf)
+    first, second = run_restarted(s, LBMForce.FP64, 60, 36, query)
+    assert np.abs(first[2]).max() > 0
+    for a, b in zip(first, second):
+        assert np.array_equal(a, b)
