@@ -938,11 +938,14 @@ __global__ void __launch_bounds__(64) cgRowsCheck(const double* __restrict__ par
 /* The forces and the reactions -w F of the solution, one group of LANES lanes per particle (block layout of the explicit
    coupling, so the wall partials fit the same slots).  BINNED: in a step each particle goes into the bin of its first
    node's tile for spreadTiles, with the slots' weights where cgSetup left them; one whose bin is full spreads here (56,320
-   Keys particles in 120^3: 46 us and 38 us for the tiles against 118 with the atomics). */
+   Keys particles in 120^3: 46 us and 38 us for the tiles against 118 with the atomics).  wall: with a processing order, each
+   particle's wall momentum goes to wall[particle][3] for cgWall, whose sums do not depend on the order; else the work-group's
+   into partials. */
 template <int LANES, bool BINNED>
 __global__ void __launch_bounds__(BLOCK) cgForces(int n, ParticleArgs a, CgArgs c, double* __restrict__ particleForce,
         unsigned long long* __restrict__ reactionFixed, uint32_t* __restrict__ touched, double* __restrict__ partials,
-        const int* __restrict__ rowCount, SpreadBins bins, const int* __restrict__ particles, double* __restrict__ systemForce) {
+        double* __restrict__ wall, const int* __restrict__ rowCount, SpreadBins bins, const int* __restrict__ particles,
+        double* __restrict__ systemForce) {
     // With matrix rows the host launches this before it knows whether the solve has converged.
     if (rowCount != nullptr && c.scalars[DONE] == 0.0)
         return;
@@ -1029,7 +1032,30 @@ __global__ void __launch_bounds__(BLOCK) cgForces(int n, ParticleArgs a, CgArgs 
         staged.add(a, reactionFixed);
     if (a.isStep)
         markTouched<LANES == 64 ? 4 : LANES == 32 ? 3 : 2>(touched, node, flagged, lane);
-    blockPartials(wallAcc, partials);
+    if (wall == nullptr)
+        blockPartials(wallAcc, partials);
+    else
+        for (int k = 0; k < 3; k++) {
+            const double sum = groupSum<LANES>(wallAcc[k]);
+            if (rank < n && lane == 0)
+                wall[3*(size_t) particleAt(c, rank) + k] = sum;
+        }
+}
+
+/* The wall partial sums of particles that cgForces took in a processing order: by index, `group` particles to each of the
+   coupling's slots (5,000 Keys particles between walls in 64^3: 145 -> 147 us a step).  done: as cgForces, nothing before the
+   solve has converged. */
+__global__ void __launch_bounds__(BLOCK) cgWall(const double* __restrict__ wall, int n, int group, int slots,
+        double* __restrict__ partials, const double* done) {
+    if (done != nullptr && *done == 0.0)
+        return;
+    const int item = blockIdx.x*BLOCK + threadIdx.x, slot = item/3, k = item - 3*slot;
+    if (slot >= slots)
+        return;
+    double sum = 0.0;
+    for (int i = slot*group; i < n && i < (slot + 1)*group; i++)
+        sum += wall[3*(size_t) i + k];
+    partials[3*(size_t) slot + k] = sum;
 }
 
 unsigned blocksOf(size_t items, int perBlock) {
@@ -1323,20 +1349,22 @@ void centredCoupleT(CentredState* st, const S* src, const uint32_t* mask, const 
         spread.slotWeight = c.slotW;
         spread.weightStride = c.slots;
     }
+    // The particles' wall momentum, where their places in the launch depend on the order: in c.Ad, which a solve is done with.
+    double* wall = order != nullptr && partials != nullptr ? c.Ad : nullptr;
     auto forces = [&](const int* rowCount) {
         auto launch = [&](auto binned) {
             constexpr bool B = decltype(binned)::value;
             switch (st->lanes) {
             case 8:
-                cgForces<8, B><<<groups, BLOCK, 0, stream>>>(n, a, c, particleForce, reactionFixed, touched, partials, rowCount,
+                cgForces<8, B><<<groups, BLOCK, 0, stream>>>(n, a, c, particleForce, reactionFixed, touched, partials, wall, rowCount,
                         spread, particles, systemForce);
                 break;
             case 32:
-                cgForces<32, B><<<groups, BLOCK, 0, stream>>>(n, a, c, particleForce, reactionFixed, touched, partials, rowCount,
+                cgForces<32, B><<<groups, BLOCK, 0, stream>>>(n, a, c, particleForce, reactionFixed, touched, partials, wall, rowCount,
                         spread, particles, systemForce);
                 break;
             default:
-                cgForces<64, B><<<groups, BLOCK, 0, stream>>>(n, a, c, particleForce, reactionFixed, touched, partials, rowCount,
+                cgForces<64, B><<<groups, BLOCK, 0, stream>>>(n, a, c, particleForce, reactionFixed, touched, partials, wall, rowCount,
                         spread, particles, systemForce);
                 break;
             }
@@ -1347,6 +1375,9 @@ void centredCoupleT(CentredState* st, const S* src, const uint32_t* mask, const 
             launch(std::true_type());
             launchSpreadTiles(mask, a, spread, reactionFixed, touched, stream);
         }
+        if (wall != nullptr)
+            cgWall<<<blocksOf(3*(size_t) groups, BLOCK), BLOCK, 0, stream>>>(wall, n, BLOCK/st->lanes, (int) groups, partials,
+                    rowCount != nullptr ? c.scalars + DONE : nullptr);
     };
     setup(st->rows);
     if (st->rows.cell != nullptr && solveRows(st, a.g, mass, aa, stream, [&] { forces(st->rows.rowCount); }))

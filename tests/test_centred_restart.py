@@ -77,3 +77,30 @@ def test_restart_after_a_crowd_dispersed_is_bit_identical(query):
     assert np.abs(first[2]).max() > 0
     for a, b in zip(first, second):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("stencil", [LBMForce.Trilinear, LBMForce.ThreePoint, LBMForce.Keys],
+                         ids=["trilinear", "threepoint", "keys"])
+@pytest.mark.parametrize("grid,beads", [((12, 12, 12), 130), ((13, 7, 9), 301)], ids=["rows", "spread"])
+def test_restart_keeps_the_wall_force(grid, beads, stencil):
+    """Between walls: the wall force of a restarted run, with the reactions of the beads whose stencils reach the walls, is
+    bit-identical too, with the solve by rows and, on axes of fewer than 12 nodes, by the spread."""
+    rng = np.random.default_rng(beads)
+    nx, ny, nz = grid
+    s = Setup(grid, tau=0.8)
+    s.add_particles(rng.uniform(0, grid, size=(beads, 3)), velocities=rng.normal(scale=2.0, size=(beads, 3)))
+
+    def conf(f):
+        f.setSolidNodes([i for k in (0, nz - 1) for i in range(k*nx*ny, (k + 1)*nx*ny)])
+        f.setWallScheme(LBMForce.BounceBack)
+        f.setFriction(5.0)
+        f.setTemperature(300.0)
+        f.setFluidFluctuations(True)
+        f.setRandomNumberSeed(5)
+        f.setDragScheme(LBMForce.Centered)
+        f.setInterpolationStencil(stencil)
+    s.configure.append(conf)
+    first, second = run_restarted(s, LBMForce.FP64, 60, 30, False)
+    assert np.abs(first[3]).max() > 0
+    for a, b in zip(first, second):
+        assert np.array_equal(a, b)
