@@ -735,30 +735,49 @@ static FastDiv makeFastDiv(uint32_t d) {
     return f;
 }
 
-uint64_t layoutRows(Geometry& g, size_t elementSize) {
+uint64_t roomForPadding() {
+    size_t free = 0, total = 0;
+    return hipMemGetInfo(&free, &total) == hipSuccess ? free/2 : 0;
+}
+
+uint64_t layoutRows(Geometry& g, size_t elementSize, uint64_t maxPadded) {
     g.divx = makeFastDiv(g.nx);
     g.divxy = makeFastDiv(g.nxy);
     g.divy = makeFastDiv(g.ny);
-    // Chunks of 32 nodes, or of 16 with FP64 storage: a 128 B line (64 B with FP16 or BF16: chunks of 64 gain nothing
+    // Chunks of 32 nodes, or 16 with FP64 storage: a 128 B line (64 B with FP16 or BF16: chunks of 64 gain nothing
     // there and idle more lanes), from the row's start and into rows padded to whole chunks, so that every line is
     // written whole by one half-wavefront.  Where nx is no multiple of the chunk, consecutive threads on consecutive nodes
     // wrote lines in pieces from wavefronts on different XCDs.  The pass without noise, that order against this one: FP32
     // 150^3 151 -> 98.8 us, 120^3 67.0 -> 51.9, 200^3 295 -> 238, 75^3 23.1 -> 20.3; FP16 150^3 74.0 -> 56.6, 101^3
-    // 27.6 -> 21.0; FP64 150^3 247 -> 195, 101^3 79.4 -> 65.6 (chunks of 32: 69.1).  Chunks without the padding: FP32
-    // 150^3 145 us; padding without the chunks: 156.  FP32 takes chunks of 16 (64 B) where those of 32 would pad a row by
-    // more than a quarter (48^3: 10.9 us with 32, 9.8 with 16; 80^3 and 112^3, padded by less: 20.9 and 45.7 with 32, 20.8
-    // and 47.4 with 16).
-    const uint32_t by32 = (g.nx + 31u)/32u*32u;
-    g.chunkShift = elementSize == 8 || (elementSize == 4 && (by32 - g.nx)*4u > g.nx) ? 4 : 5;
-    g.chunksPerRow = ((g.nx - 1u) >> g.chunkShift) + 1u;
+    // 27.6 -> 21.0; FP64 150^3 247 -> 195, 101^3 79.4 -> 65.6 (chunks of 32: 69.1).
+    // Padding costs memory, stores and, with noise, instructions in the lanes past the rows' ends, so rows grow by a
+    // quarter at most; beyond that the chunks go unpadded, with at most one idle lane per node.  A pass without and with
+    // noise over 6 M nodes in us, consecutive nodes | chunks padded without that limit | now: FP16 nx = 33 172, 172 | 144, 183 |
+    // 153, 154; 40 140, 143 | 120, 155 | 141, 141; 100 133, 136 | 97, 126 | 113, 126; FP32 8 380, 386 | 426, 423 | 349, 352;
+    // 17 333, 352 | 282, 283 | 265, 276; 33 308, 309 | 274, 268 | 206, 211; FP64 4 872, 706 | 1315, 1318 | 769, 701; 20 476,
+    // 533 | 511, 525 | 401, 438; 36 442, 521 | 439, 451 | 357, 434.
+    const auto whole = [&](uint32_t shift) { return (((g.nx - 1u) >> shift) + 1u) << shift; };
+    const auto quarter = [&](uint32_t shift) { return (whole(shift) - g.nx)*4u <= g.nx; };
+    uint32_t shift = 5;
+    // FP64 rows of whole 64 B pieces: nothing gained by padding them to lines (40: 381 us with, 361 without).
+    if (elementSize == 8 && g.nx % 16u == 8u)
+        shift = 3;
+    // FP64 takes chunks of 16 where they are padded (unpadded ones of 16 lose to those of 32, 36: 449 and 357 us).  FP32 does
+    // (64 B) where those of 32 would pad a row too much (100: 210, 208 us, with 32 unpadded 224, 212); FP16 only where those
+    // would idle a third of their lanes (100: 126, 128 and 113, 126; but 36 150, 152 and 121, 151 to 169 from run to run).
+    else if (elementSize == 8 ? quarter(4) : elementSize == 4 ? !quarter(5) && quarter(4) : 2u*whole(5) > 3u*g.nx)
+        shift = 4;
+    while (whole(shift) > 2u*g.nx)
+        shift--;
+    g.chunkShift = shift;
+    g.chunksPerRow = ((g.nx - 1u) >> shift) + 1u;
     g.divChunks = makeFastDiv(g.chunksPerRow);
-    const uint64_t rows = (uint64_t) g.ny*g.nz;
-    const uint32_t whole = g.chunksPerRow << g.chunkShift;
     // No padding where rows are grouped in blocks, or where it would take an array that fits beyond the 4 GiB of the
     // 32-bit offsets.
-    g.padded = whole != g.nx && g.rowShift == 0 && (NQ*rows*whole*elementSize <= (1ull << 32) ||
-            NQ*rows*g.nx*elementSize > (1ull << 32)) ? 1 : 0;
-    g.qstride = (g.padded ? whole : g.nx) << g.rowShift;
+    const uint64_t rows = (uint64_t) g.ny*g.nz, padded = NQ*rows*whole(shift)*elementSize;
+    g.padded = whole(shift) != g.nx && quarter(shift) && g.rowShift == 0 && padded <= maxPadded &&
+            (padded <= (1ull << 32) || NQ*rows*g.nx*elementSize > (1ull << 32)) ? 1 : 0;
+    g.qstride = (g.padded ? whole(shift) : g.nx) << g.rowShift;
     return NQ*rows*(g.qstride >> g.rowShift);
 }
 
