@@ -726,9 +726,12 @@ void create(const lbm_params* params, const int* solid, int numSolid, const int*
         bool want = spreadEnv ? std::string(spreadEnv) == "tiles" : slots >= n && slots >= 900000;
         // The moment field and the stencils formed once per particle: by default for dense particles whose slots are worth the
         // field's launch.  A step of the explicit drag in us without and with both: 10,000 Keys beads in 128^3 142 and 137,
-        // 15,000 in 80^3 124 and 81; but 5,000 in 50 x 47 x 61 (320,000 slots) 39 and 41, 2,000 in 40^3 24 and 26.
+        // 15,000 in 80^3 124 and 81; but 5,000 in 50 x 47 x 61 (320,000 slots) 39 and 41, 2,000 in 40^3 24 and 26.  Of the centred
+        // one, which takes the field alone: 20,000 Keys beads in 128^3 (0.6 slots per node) 319 and 309, 8,000 in 80^3 (1.0) 172
+        // and 168, 40,000 trilinear ones in 64^3 (1.2; 320,000 slots) 209 and 206; but 9,000 Keys beads in 128^3 (0.27) 228 and
+        // 235, 80,000 in 256^3 (0.31) 1,352 and 1,383, 2,000 in 64^3 (128,000 slots) 115 and 116.
         // LBM_AMD_FIELD=0 or 1 forces the field.
-        const bool many = c->dense && (p.drag_scheme == LBM_DRAG_CENTERED || slots >= 400000);
+        const bool many = p.drag_scheme == LBM_DRAG_CENTERED ? 2*slots >= n && slots >= 300000 : c->dense && slots >= 400000;
         const char* fieldEnv = getenv("LBM_AMD_FIELD");
         bool field = fieldEnv ? fieldEnv[0] == '1' : many;
         if (field && (p.drag_scheme == LBM_DRAG_EXPLICIT || p.interpolation_stencil != LBM_STENCIL_NEAREST))

@@ -361,3 +361,35 @@ def test_centred_device_steps_are_those_of_the_host(stencil, grid):
     pos, vel = dp.pull()
     assert np.abs(pos - host.positions).max() <= 1e-12*max(grid)
     assert np.abs(vel - host.velocities).max() <= 1e-12*np.abs(host.velocities).max()
+
+
+@pytest.mark.parametrize("storage", [LBMForce.FP16, LBMForce.FP32, LBMForce.FP64], ids=["fp16", "fp32", "fp64"])
+@pytest.mark.parametrize("grid,beads", [((20, 14, 12), 400), ((9, 8, 7), 150)], ids=["rows", "spread"])
+def test_centred_moment_field_gives_the_pulled_moments(grid, beads, storage, monkeypatch):
+    """The centred drag's setup from the moment field against the populations pulled per stencil slot, bit for bit, between
+    walls and with the momentum removal every second step; the rule between them only weighs their times."""
+    rng = np.random.default_rng(beads)
+    nx, ny, nz = grid
+    s = Setup(grid, tau=0.8)
+    s.add_particles(rng.uniform(0, grid, size=(beads, 3)), velocities=rng.normal(scale=0.3, size=(beads, 3)))
+
+    def conf(f):
+        f.setSolidNodes([i for k in (0, nz - 1) for i in range(k*nx*ny, (k + 1)*nx*ny)])
+        f.setWallScheme(LBMForce.BounceBack)
+        f.setFriction(10.0)
+        f.setTemperature(300.0)
+        f.setFluidFluctuations(True)
+        f.setFluidMomentumRemovalFrequency(2)
+        f.setRandomNumberSeed(5)
+        f.setDragScheme(LBMForce.Centered)
+        f.setInterpolationStencil(LBMForce.Keys)
+    s.configure.append(conf)
+    runs = []
+    for field in ("0", "1"):
+        monkeypatch.setenv("LBM_AMD_FIELD", field)
+        c = s.build(None, storage=storage)
+        c.step(5)
+        runs.append((c.getFluidState(), c.positions.copy(), c.velocities.copy(), c.getWallForce(), c.getForces()))
+    assert np.abs(runs[0][0]).max() > 0
+    for a, b in zip(*runs):
+        assert np.array_equal(a, b)
