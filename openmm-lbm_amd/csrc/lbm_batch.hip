@@ -125,15 +125,21 @@ void launchStep(lbm_batch* b, bool timed = false) {
     launchCoupleBatch(b->stencil, b->coupleThreads, b->dDesc, b->particleTiles, b->numParticleTiles, b->pos, b->vel,
             b->mass, b->force, b->stepCounter, b->stepCounter + 1, (b->xcdOrder & 1) != 0, b->stream);
     std::pair<hipEvent_t, hipEvent_t> ev{nullptr, nullptr};
+    BatchParticles particles = {b->particleReplica, b->numParticles, b->pos, b->vel, b->force, b->invMass};
+    const int64_t* counter = b->numParticles > 0 ? b->stepCounter + 1 : b->stepCounter;
+    const bool xcdOrder = (b->xcdOrder & 2) != 0;
     if (timed) {
+        // The events time the lattice pass alone: the particles' work-groups in a launch of their own before it.
+        if (particles.count > 0)
+            launchFusedBatch(b->threads, b->fluct, b->dDesc, b->tileReplica, 0, counter, b->stepCounter, particles, xcdOrder,
+                    b->stream);
+        particles.count = 0;
         hipCheck(hipEventCreate(&ev.first), "event");
         hipCheck(hipEventCreate(&ev.second), "event");
         b->events.push_back(ev);
         hipCheck(hipEventRecord(ev.first, b->stream), "event");
     }
-    const BatchParticles particles = {b->particleReplica, b->numParticles, b->pos, b->vel, b->force, b->invMass};
-    launchFusedBatch(b->threads, b->fluct, b->dDesc, b->tileReplica, b->numTiles,
-            b->numParticles > 0 ? b->stepCounter + 1 : b->stepCounter, b->stepCounter, particles, (b->xcdOrder & 2) != 0,
+    launchFusedBatch(b->threads, b->fluct, b->dDesc, b->tileReplica, b->numTiles, counter, b->stepCounter, particles, xcdOrder,
             b->stream);
     if (timed)
         hipCheck(hipEventRecord(ev.second, b->stream), "event");

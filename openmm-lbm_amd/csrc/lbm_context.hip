@@ -410,7 +410,8 @@ void advanceFluid(lbm_context* c, const double* dPos, const double* dVel, const 
     // The particles' work between this step and the next joins the pass where there are no solid nodes to reflect at, else
     // the bounce-back, once the forces on them are complete (the centred drag's with the nearest node are added after the step).
     BetweenSteps* between = !particles || c->forcesAdded ? c->between : nullptr;
-    const bool joinPass = between != nullptr && c->mask == nullptr && c->fusedPath == FUSED_DIRECT;
+    // Not while the pass is timed: the events are to hold it alone.
+    const bool joinPass = between != nullptr && c->mask == nullptr && c->fusedPath == FUSED_DIRECT && !c->profile;
     const bool joinWalls = between != nullptr && between->reflection.mask != nullptr && c->numWall > 0 && c->numBoundary == 0;
     if (joinPass)
         launchFusedBetween(c->p.storage, particles, c->fluct(), c->popA, c->popB, c->reactionFixed, c->touched,
