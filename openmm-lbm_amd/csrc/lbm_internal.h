@@ -6,7 +6,7 @@
 
 #include "lbm_device.h"
 #include "../../include/lbm_amd.h"
-#include <mutex>
+#include "lbm_memory.h"
 #include <string>
 #include <vector>
 
@@ -340,40 +340,6 @@ struct StepReflection {
     const uint32_t* mask = nullptr;
     double* partials = nullptr;     // the step's wall partial sums: the kernel clears those outside its own slots
     int count = 0, ownOffset = 0;
-};
-
-/*
- * Device memory that the calls which read fields out share, one after the other: kept from call to call up to KEEP bytes and
- * freed with its owner, allocated for the call beyond.  The lock is held until the call has what it wants on the host.
- */
-struct FieldStage {
-    static constexpr size_t KEEP = 1ull << 30;
-    std::mutex lock;
-    void* kept = nullptr;
-    size_t bytes = 0;
-    /* Memory for a call that needs `need` bytes, or nullptr; give it back with done(). */
-    void* get(size_t need) {
-        if (need <= bytes)
-            return kept;
-        void* p = nullptr;
-        if (hipMalloc(&p, need) != hipSuccess)
-            return nullptr;
-        if (need <= KEEP) {
-            free();
-            kept = p;
-            bytes = need;
-        }
-        return p;
-    }
-    hipError_t done(void* p) {
-        return p == kept ? hipSuccess : hipFree(p);
-    }
-    void free() {
-        if (kept != nullptr)
-            (void) hipFree(kept);
-        kept = nullptr;
-        bytes = 0;
-    }
 };
 
 /* Nodes per axis of an interpolation stencil (LBMStencils.h:42-104). */
