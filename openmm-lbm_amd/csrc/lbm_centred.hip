@@ -1177,24 +1177,24 @@ CentredState* centredCreate(int numParticles, int stencil, const Geometry& g) {
                 r.cells[1] = (int) g.ny/4;
                 r.cells[2] = (int) g.nz/4;
                 st->numCells = r.cells[0]*r.cells[1]*r.cells[2];
-                r.cellCount = alloc<int>(st->numCells);
-                r.cell = alloc<CellEntry>((size_t) st->numCells*CELL_CAP);
-                r.home = alloc<uint32_t>(4*(size_t) n);
-                r.axisWeight = alloc<double>(3*(3*(size_t) w - 2)*n);
-                r.rowCount = alloc<int>(n);
-                r.rowParticle = alloc<int>((size_t) n*ROW_CAP);
-                r.rowValue = alloc<double>((size_t) n*ROW_CAP);
-                r.overflow = alloc<int>(1);
-                st->directions[0] = alloc<double>(6*(size_t) n);
-                st->directions[1] = alloc<double>(6*(size_t) n);
-                check(hipMemset(r.cellCount, 0, st->numCells*sizeof(int)), "memset");
-                check(hipMemset(r.axisWeight, 0, 3*(3*(size_t) w - 2)*n*sizeof(double)), "memset");
-                check(hipMemset(r.overflow, 0, sizeof(int)), "memset");
-                check(hipEventCreateWithFlags(&st->checked, hipEventDisableTiming), "event");
-                for (void* b : {(void*) r.cellCount, (void*) r.cell, (void*) r.home, (void*) r.axisWeight, (void*) r.rowCount,
-                                (void*) r.rowParticle, (void*) r.rowValue, (void*) r.overflow, (void*) st->directions[0],
-                                (void*) st->directions[1]})
-                    st->buffers.push_back(b);
+                const size_t rowEntries = (size_t) n*ROW_CAP, weights = 3*(3*(size_t) w - 2)*n;
+                // Without the memory for them the solves take the spread.
+                if (allocateOptional({{(void**) &r.cellCount, st->numCells*sizeof(int)},
+                        {(void**) &r.cell, (size_t) st->numCells*CELL_CAP*sizeof(CellEntry)},
+                        {(void**) &r.home, 4*(size_t) n*sizeof(uint32_t)}, {(void**) &r.axisWeight, weights*sizeof(double)},
+                        {(void**) &r.rowCount, n*sizeof(int)}, {(void**) &r.rowParticle, rowEntries*sizeof(int)},
+                        {(void**) &r.rowValue, rowEntries*sizeof(double)}, {(void**) &r.overflow, sizeof(int)},
+                        {(void**) &st->directions[0], 6*(size_t) n*sizeof(double)},
+                        {(void**) &st->directions[1], 6*(size_t) n*sizeof(double)}}, reservedBytes(numNodes))) {
+                    for (void* b : {(void*) r.cellCount, (void*) r.cell, (void*) r.home, (void*) r.axisWeight, (void*) r.rowCount,
+                                    (void*) r.rowParticle, (void*) r.rowValue, (void*) r.overflow, (void*) st->directions[0],
+                                    (void*) st->directions[1]})
+                        st->buffers.push_back(b);
+                    check(hipMemset(r.cellCount, 0, st->numCells*sizeof(int)), "memset");
+                    check(hipMemset(r.axisWeight, 0, weights*sizeof(double)), "memset");
+                    check(hipMemset(r.overflow, 0, sizeof(int)), "memset");
+                    check(hipEventCreateWithFlags(&st->checked, hipEventDisableTiming), "event");
+                }
             }
         }
     }

@@ -596,7 +596,7 @@ void create(const lbm_params* params, const int* solid, int numSolid, const int*
         c->g.rowShift--;
     if (n > (1ull << 30))
         throw Error(LBM_ERROR_INVALID, "LBMForce: the lattice is too large for one GPU: at most 2^30 nodes");
-    const uint64_t popBytes = layoutRows(c->g, c->elem, roomForPadding()/2)*c->elem;
+    const uint64_t popBytes = layoutRows(c->g, c->elem, spareBytes(reservedBytes(n))/2)*c->elem;
     // The fused pass addresses populations by 32-bit byte offsets while an array of them fits in 4 GiB (up to 56.5 M
     // nodes with FP32 storage), and by 64-bit indices beyond.  LBM_AMD_WIDE_ADDRESSING=1 takes the 64-bit path always.
     const char* wideEnv = getenv("LBM_AMD_WIDE_ADDRESSING");
@@ -736,14 +736,14 @@ void create(const lbm_params* params, const int* solid, int numSolid, const int*
         const char* fieldEnv = getenv("LBM_AMD_FIELD");
         bool field = fieldEnv ? fieldEnv[0] == '1' : many;
         if (field && (p.drag_scheme == LBM_DRAG_EXPLICIT || p.interpolation_stencil != LBM_STENCIL_NEAREST))
-            c->momentField = deviceAlloc<double4>(n);
+            (void) allocateOptional({{(void**) &c->momentField, n*sizeof(double4)}}, reservedBytes(n));
         // The stencils formed once per particle for the groups of the explicit stencil coupling, by default for dense
         // particles (100,000 Keys beads on 128^3: the coupling kernel 148 -> 110 us, the setup 11 us; for 20,000 sparse
         // beads on 256^3 the extra launch costs what it saves); LBM_AMD_STENCIL_SETUP=0 or 1 forces the choice.
         const char* setupEnv = getenv("LBM_AMD_STENCIL_SETUP");
         bool setup = setupEnv ? setupEnv[0] == '1' : many;
         if (p.drag_scheme == LBM_DRAG_EXPLICIT && p.interpolation_stencil != LBM_STENCIL_NEAREST && setup)
-            c->axisStencils = deviceAlloc<AxisStencil>((size_t) numParts);
+            (void) allocateOptional({{(void**) &c->axisStencils, numParts*sizeof(AxisStencil)}}, reservedBytes(n));
         if (fit && want) {
             SpreadBins& b = c->bins;
             size_t tiles = (size_t) b.ntx*b.nty*b.ntz;
@@ -751,20 +751,20 @@ void create(const lbm_params* params, const int* solid, int numSolid, const int*
             // the atomics.
             double mean = (double) numParts/(double) tiles;
             b.cap = std::min(SPREAD_MAX_CAP, ((int) std::ceil(4.0*mean) + 16 + 15)/16*16);
-            c->binCounts[0] = deviceAlloc<int>(tiles);
-            c->binCounts[1] = deviceAlloc<int>(tiles);
-            HIP_CHECK(hipMemsetAsync(c->binCounts[0], 0, tiles*sizeof(int), c->stream));
-            HIP_CHECK(hipMemsetAsync(c->binCounts[1], 0, tiles*sizeof(int), c->stream));
-            b.beads = deviceAlloc<int>(tiles*(size_t) b.cap);
-            b.anchor = deviceAlloc<uint16_t>(tiles*(size_t) b.cap);
-            b.force = deviceAlloc<double>(3*tiles*(size_t) b.cap);
-            c->binSpilled = deviceAlloc<int>(2);
-            HIP_CHECK(hipMemsetAsync(c->binSpilled, 0, 2*sizeof(int), c->stream));
             int lanes = coupleLanes(p.interpolation_stencil);
             b.weightStride = lanes;
-            if (p.drag_scheme == LBM_DRAG_EXPLICIT)
-                b.slotWeight = deviceAlloc<double>((size_t) numParts*lanes);
-            c->binned = true;
+            const size_t entries = tiles*(size_t) b.cap;
+            // The centred drag has the weights in its slots.
+            const size_t weights = p.drag_scheme == LBM_DRAG_EXPLICIT ? (size_t) numParts*lanes : 1;
+            c->binned = allocateOptional({{(void**) &c->binCounts[0], tiles*sizeof(int)}, {(void**) &c->binCounts[1], tiles*sizeof(int)},
+                    {(void**) &c->binSpilled, 2*sizeof(int)}, {(void**) &b.beads, entries*sizeof(int)},
+                    {(void**) &b.anchor, entries*sizeof(uint16_t)}, {(void**) &b.force, 3*entries*sizeof(double)},
+                    {(void**) &b.slotWeight, weights*sizeof(double)}}, reservedBytes(n));
+            if (c->binned) {
+                HIP_CHECK(hipMemsetAsync(c->binCounts[0], 0, tiles*sizeof(int), c->stream));
+                HIP_CHECK(hipMemsetAsync(c->binCounts[1], 0, tiles*sizeof(int), c->stream));
+                HIP_CHECK(hipMemsetAsync(c->binSpilled, 0, 2*sizeof(int), c->stream));
+            }
         }
     }
     // The fluid at equilibrium with the initial velocity; solid nodes hold no fluid.

@@ -735,11 +735,6 @@ static FastDiv makeFastDiv(uint32_t d) {
     return f;
 }
 
-uint64_t roomForPadding() {
-    size_t free = 0, total = 0;
-    return hipMemGetInfo(&free, &total) == hipSuccess ? free/2 : 0;
-}
-
 uint64_t layoutRows(Geometry& g, size_t elementSize, uint64_t maxPadded) {
     g.divx = makeFastDiv(g.nx);
     g.divxy = makeFastDiv(g.nxy);

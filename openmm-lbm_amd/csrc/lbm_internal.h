@@ -238,9 +238,6 @@ inline uint64_t fusedThreads(const Geometry& g) {
    rowShift are set; returns the elements of one population array.  maxPadded: the bytes that an array may take with padded
    rows; where it would take more, the rows are not padded. */
 uint64_t layoutRows(Geometry& g, size_t elementSize, uint64_t maxPadded);
-/* The bytes that all padded arrays of a lattice or batch may take, half of the device's free memory, so that what fits without
-   padding does not fail to with it. */
-uint64_t roomForPadding();
 void launchMomentReduce(int storage, bool solids, const void* src, const uint32_t* mask, const Geometry& g,
         double* partials, hipStream_t stream);
 void launchFinishReduce(const double* partials, double numFluid, double* totals, double* ucm, hipStream_t stream);

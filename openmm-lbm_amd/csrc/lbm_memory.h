@@ -1,9 +1,12 @@
 /*
- * Host-side rules of device memory: the memory that the calls which read fields out share.
+ * Host-side rules of device memory: the memory that a lattice can do without, and that which the calls that read fields out
+ * share.
  */
 #pragma once
 
 #include <hip/hip_runtime_api.h>
+#include <stdint.h>
+#include <initializer_list>
 #include <mutex>
 
 namespace lbm {
@@ -15,6 +18,46 @@ inline void* tryAllocate(size_t bytes) {
         return p;
     (void) hipGetLastError();
     return nullptr;
+}
+
+/*
+ * What stays free beside memory that a lattice of n nodes can do without (padded rows, a moment field, the tile spread's
+ * bins, matrix rows): its reaction accumulators and masks, a state of 19 FP64 values per node and the fields on their way to
+ * the host.  A lattice that fits without that memory then keeps fitting, and is read out, with it.
+ */
+inline uint64_t reservedBytes(uint64_t n) {
+    return (24 + 1 + 19*8 + 4*8)*n;
+}
+
+/* The device's free memory beyond `reserve` bytes. */
+inline uint64_t spareBytes(uint64_t reserve) {
+    size_t free = 0, total = 0;
+    return hipMemGetInfo(&free, &total) == hipSuccess && free > reserve ? free - reserve : 0;
+}
+
+/* One part of a set of arrays that are all there or not needed at all. */
+struct OptionalPart {
+    void** to;
+    size_t bytes;
+};
+
+/* All the parts, or none (nullptr): where they would take more than the spare memory, or an allocation fails. */
+inline bool allocateOptional(std::initializer_list<OptionalPart> parts, uint64_t reserve) {
+    uint64_t total = 0;
+    for (const OptionalPart& part : parts)
+        total += part.bytes;
+    bool all = total <= spareBytes(reserve);
+    for (const OptionalPart& part : parts) {
+        *part.to = all ? tryAllocate(part.bytes) : nullptr;
+        all = all && *part.to != nullptr;
+    }
+    if (!all)
+        for (const OptionalPart& part : parts) {
+            if (*part.to != nullptr)
+                (void) hipFree(*part.to);
+            *part.to = nullptr;
+        }
+    return all;
 }
 
 /*

@@ -1,5 +1,6 @@
 """The library's rules of device memory (lbm_memory.h) on a device that runs out of it, which a small program plays: its hipMalloc
-gives out no more than it is told to hold (CPU; needs a C++ compiler and HIP's headers)."""
+gives out no more than it is told to hold (CPU; needs a C++ compiler and HIP's headers); and one lattice on a GPU with little
+memory left."""
 import os
 import shutil
 import subprocess
@@ -14,10 +15,10 @@ DEVICE = r"""
 #include <cstdio>
 #include <map>
 static std::map<void*, size_t> held;
-static size_t capacity = 0, used = 0, serial = 0;
+static size_t capacity = 0, used = 0, serial = 0, fragment = ~(size_t) 0;
 static hipError_t last = hipSuccess;
 extern "C" hipError_t hipMalloc(void** p, size_t n) {
-    if (used + n > capacity)
+    if (used + n > capacity || n > fragment)
         return last = hipErrorOutOfMemory;
     *p = (void*) (0x1000 + 0x1000*++serial);
     held[*p] = n;
@@ -83,3 +84,60 @@ def test_kept_field_memory_gives_way_to_a_larger_call(tmp_path):
     stage.free();
     CHECK(used == 0);
 """)
+
+
+def test_optional_memory_leaves_the_reserve(tmp_path):
+    """All the parts of a set or none: with room for them beside the reserve, without, and where a part fails although the
+    device's figure had room for it."""
+    run(tmp_path, r"""
+    void *a = nullptr, *b = nullptr;
+    CHECK(lbm::reservedBytes(1000) == 209000);
+    capacity = 4*GB;
+    CHECK(lbm::spareBytes(3*GB) == GB && lbm::spareBytes(4*GB) == 0 && lbm::spareBytes(5*GB) == 0);
+    CHECK(lbm::allocateOptional({{&a, GB/2}, {&b, GB/2}}, 3*GB) && a && b && used == GB);
+    CHECK(hipFree(a) == hipSuccess && hipFree(b) == hipSuccess);
+    CHECK(!lbm::allocateOptional({{&a, GB/2}, {&b, GB/2 + 1}}, 3*GB) && !a && !b && used == 0);
+    capacity = GB;
+    fragment = GB/4;                                       // no block larger than this
+    CHECK(!lbm::allocateOptional({{&a, GB/8}, {&b, GB/2}}, 0) && !a && !b && used == 0);
+    CHECK(hipGetLastError() == hipSuccess);
+""")
+
+
+@pytest.mark.gpu
+def test_a_centred_solver_fits_where_it_did_without_rows():
+    """One million centred Keys particles in 200^3, which need 3.5 GB, on a device with 4.2 GB free: the 1.7 GB of the matrix
+    rows are done without, and the lattice steps and is read out."""
+    import numpy as np
+    import torch
+    from lbm_amd import LBMForce
+    from parity import Setup
+
+    n, beads = 200, 1000000
+    s = Setup((n, n, n), tau=0.7)
+    rng = np.random.default_rng(1)
+    s.masses, s.coupled = [100.0]*beads, list(range(beads))
+    s.positions, s.velocities = list(rng.uniform(0, n, size=(beads, 3))), list(np.zeros((beads, 3)))
+
+    def conf(f):
+        f.setFriction(10.0)
+        f.setTemperature(0.0)
+        f.setBodyAcceleration((1.0, 0.0, 0.0))
+        f.setDragScheme(LBMForce.Centered)
+        f.setInterpolationStencil(LBMForce.Keys)
+    s.configure.append(conf)
+    small = Setup((12, 12, 12))
+    small.configure.append(conf)
+    small.add_particles(rng.uniform(0, 12, size=(40, 3)))
+    small.build().step(1)                                  # what the first run of a kernel loads
+    torch.cuda.empty_cache()
+    fill = torch.empty(max(0, torch.cuda.mem_get_info()[0] - int(4.2e9)), dtype=torch.uint8, device="cuda")
+    try:
+        c = s.build()
+        c.step(1)
+        forces, (rho, u) = c.getForces(), c.getFluidFields()
+        assert np.isfinite(forces).all() and np.isfinite(rho).all() and u[:, 0].min() > 0
+        del c
+    finally:
+        del fill
+        torch.cuda.empty_cache()
