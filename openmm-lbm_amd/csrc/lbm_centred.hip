@@ -581,10 +581,12 @@ __device__ __forceinline__ void combinePartials(const double* __restrict__ parti
    as a third of those that three strided adds per slot made (56,320 Keys particles in 120^3: 255 -> 105 us).  The fixed-point scale, 2^(52 - e) with
    2^e >= max |x| (1 if x is zero), is formed by the first wavefront of every work-group from the largest |x| of the
    blocks in c.partials (one fixed combination, so every work-group has the same value); work-group 0 keeps it and its
-   inverse in the scalars for the gather.  The solve's first product (first = 1) records which slots spread. */
+   inverse in the scalars for the gather.  The solve's first product (first = 1) records which slots spread.
+   firstBlock: of the launch; a launch holds SPREAD_BLOCKS at most, as its threads are counted in 32 bits. */
+constexpr uint32_t SPREAD_BLOCKS = 1u << 20;
 template <int SLOTS>
 __global__ void __launch_bounds__(BLOCK) cgSpread(const double* __restrict__ x, int n, CgArgs c,
-        const double* done, int first) {
+        const double* done, int first, uint32_t firstBlock) {
     if (done != nullptr && *done != 0.0)
         return;
     __shared__ double sharedScale;
@@ -601,7 +603,7 @@ __global__ void __launch_bounds__(BLOCK) cgSpread(const double* __restrict__ x, 
         }
     }
     __syncthreads();
-    const uint64_t item = (uint64_t) placeOf(c)*BLOCK + threadIdx.x;
+    const uint64_t item = (uint64_t) (firstBlock + placeOf(c))*BLOCK + threadIdx.x;
     const uint64_t t = item/3;
     const int k = (int) (item - 3*t);
     const uint64_t rank = t/SLOTS;
@@ -1230,11 +1232,14 @@ void multiply(CentredState* st, const double* x, double* Ax, const double* mass,
     c.spread = st->sums[sums];
     c.spreadOther = st->sums[1 - sums];
     int n = st->n;
-    const unsigned spreadGroups = blocksOf(3*(size_t) n*c.slots, BLOCK);
-    switch (st->lanes) {
-    case 8: cgSpread<8><<<spreadGroups, BLOCK, 0, stream>>>(x, n, c, done, first ? 1 : 0); break;
-    case 32: cgSpread<27><<<spreadGroups, BLOCK, 0, stream>>>(x, n, c, done, first ? 1 : 0); break;
-    default: cgSpread<64><<<spreadGroups, BLOCK, 0, stream>>>(x, n, c, done, first ? 1 : 0); break;
+    const uint32_t spreadGroups = blocksOf(3*(size_t) n*c.slots, BLOCK);
+    for (uint32_t at = 0; at < spreadGroups; at += SPREAD_BLOCKS) {
+        const unsigned groups = std::min(spreadGroups - at, SPREAD_BLOCKS);
+        switch (st->lanes) {
+        case 8: cgSpread<8><<<groups, BLOCK, 0, stream>>>(x, n, c, done, first ? 1 : 0, at); break;
+        case 32: cgSpread<27><<<groups, BLOCK, 0, stream>>>(x, n, c, done, first ? 1 : 0, at); break;
+        default: cgSpread<64><<<groups, BLOCK, 0, stream>>>(x, n, c, done, first ? 1 : 0, at); break;
+        }
     }
     switch (st->lanes) {
     case 8: cgGather<8><<<blocksOf(n, BLOCK/8), BLOCK, 0, stream>>>(x, Ax, mass, n, aa, c, done); break;

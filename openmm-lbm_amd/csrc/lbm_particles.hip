@@ -513,6 +513,9 @@ bool spreadTilesFit(int nx, int ny, int nz, bool anyOpen, SpreadBins& bins) {
             return false;
         tiles[k] = (uint32_t) std::max(2, (n[k] + tile[k] - 1)/tile[k]);
     }
+    // A launch's threads are counted in 32 bits (narrow lattices have tiles of fewer nodes than threads).
+    if ((uint64_t) tiles[0]*tiles[1]*tiles[2]*SPREAD_THREADS > 0xFFFFFFFFull)
+        return false;
     bins.ntx = tiles[0];
     bins.nty = tiles[1];
     bins.ntz = tiles[2];

@@ -393,3 +393,28 @@ def test_centred_moment_field_gives_the_pulled_moments(grid, beads, storage, mon
     assert np.abs(runs[0][0]).max() > 0
     for a, b in zip(*runs):
         assert np.array_equal(a, b)
+
+
+def test_centred_spread_in_several_launches_matches_the_rows(monkeypatch):
+    """1.5 M centred Keys particles, whose spread takes two launches of at most 2^20 work-groups, against the matrix rows (both
+    stop at a residual of 1e-13 of the right-hand side: the forces agree to 1e-11 of the largest, as in the rows' test)."""
+    n, beads = 240, 1500000
+    rng = np.random.default_rng(2)
+    s = Setup((n, n, n), tau=0.8)
+    s.masses, s.coupled = [100.0]*beads, list(range(beads))
+    s.positions, s.velocities = list(rng.uniform(0, n, size=(beads, 3))), list(rng.normal(scale=0.5, size=(beads, 3)))
+
+    def conf(f):
+        f.setFriction(10.0)
+        f.setTemperature(0.0)
+        f.setDragScheme(LBMForce.Centered)
+        f.setInterpolationStencil(LBMForce.Keys)
+    s.configure.append(conf)
+    forces = []
+    for rows in ("0", "1"):
+        monkeypatch.setenv("LBM_AMD_CG_ROWS", rows)
+        c = s.build()
+        c.step(1)
+        forces.append(c.getForces())
+    assert np.abs(forces[0]).min(axis=1).max() > 0
+    assert np.abs(forces[0] - forces[1]).max() <= 1e-11*np.abs(forces[0]).max()
