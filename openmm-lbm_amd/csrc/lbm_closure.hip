@@ -12,7 +12,7 @@
  *                   scans the flags of 64 particles at a time with a fixed stride, so the wall partial sums have a fixed
  *                   order.
  *  closureField     u of every node, for closureStep where the particles are dense.
- *  closureFeatures  the same inputs for training pairs, one group of 32 lanes per particle, raw and normalized.
+ *  closureFeatures  the same inputs for training pairs, raw, one group of 32 lanes per particle.
  *  closureTargets   u_Keys(x) - u(nearest) with the stencil interpolation of the coupling, in the particle's frame
  *                   (training pairs).
  *
@@ -75,14 +75,12 @@ __device__ __forceinline__ T pick(const T v[3], int k) {
 template <typename S>
 __global__ void __launch_bounds__(BLOCK) closureFeatures(const S* __restrict__ src, const uint32_t* __restrict__ mask,
         const double* __restrict__ positions, const double* __restrict__ velocities, const int* __restrict__ particles,
-        const double* __restrict__ ucm, ParticleArgs a, ClosureNorm norm, _Float16* __restrict__ X,
-        float* __restrict__ raw, uint32_t* __restrict__ centreNode,
-        double* __restrict__ centreVelocity, uint8_t* __restrict__ ood, uint8_t* __restrict__ frame) {
+        const double* __restrict__ ucm, ParticleArgs a, float* __restrict__ raw, double* __restrict__ centreVelocity,
+        uint8_t* __restrict__ frame) {
     constexpr int GROUPS = BLOCK/FEATURE_LANES;
     int lane = threadIdx.x % FEATURE_LANES;
     int i = blockIdx.x*GROUPS + threadIdx.x/FEATURE_LANES;
     bool active = i < a.numParticles;
-    bool out = false;
     int part = active ? particles[i] : 0;
     const double* x = positions + 3*(size_t) part;
     int size[3] = {(int) a.g.nx, (int) a.g.ny, (int) a.g.nz};
@@ -109,79 +107,43 @@ __global__ void __launch_bounds__(BLOCK) closureFeatures(const S* __restrict__ s
         frame[i] = (uint8_t) code;
     const Frame fr = frameOf((unsigned) code);
     if (active) {
-        int openAxis[3] = {a.g.openX, a.g.openY, a.g.openZ};
-        _Float16* xi = X + (size_t) i*MLP_IN_PAD;
-        float* ri = raw ? raw + (size_t) i*MLP_IN : nullptr;
+        float* ri = raw + (size_t) i*MLP_IN;
         if (lane < 27) {
             int d[3] = {lane % 3 - 1, (lane/3) % 3 - 1, lane/9 - 1};
             int idx[3];
             for (int k = 0; k < 3; k++) {
                 int t = near[k] + d[k];
-                if (t < 0 || t >= size[k]) {
-                    if (openAxis[k])
-                        out = true;
+                if (t < 0 || t >= size[k])
                     t = (t + size[k]) % size[k];
-                }
                 idx[k] = t;
             }
             uint32_t node = (uint32_t) (idx[0] + (int) a.g.nx*(idx[1] + (int) a.g.ny*idx[2]));
             double u[3] = {0, 0, 0};
-            if (solidAt(mask, node))
-                out = true;
-            else
+            if (!solidAt(mask, node))
                 nodeVelocity(src, a.g, node, ucm, a.removal, 1.0, u);
-            if (lane == 13) {
-                centreNode[i] = node;
+            if (lane == 13)
                 for (int c = 0; c < 3; c++)
                     centreVelocity[3*(size_t) i + c] = u[c];
-            }
             // This node's place in the particle's frame, and its velocity there.
             int slot = 13;
             for (int k = 0, stride = 1; k < 3; k++, stride *= 3)
                 slot += stride*(fr.sign[k] < 0 ? -pick(d, fr.axis[k]) : pick(d, fr.axis[k]));
-            for (int c = 0; c < 3; c++) {
-                float r = (float) (fr.sign[c]*pick(u, fr.axis[c]));
-                float f = r*norm.uScale;
-                if (!(fabsf(f) <= norm.uBound))
-                    out = true;
-                xi[3 + 3*slot + c] = (_Float16) f;
-                if (ri)
-                    ri[3 + 3*slot + c] = r;
-            }
+            for (int c = 0; c < 3; c++)
+                ri[3 + 3*slot + c] = (float) (fr.sign[c]*pick(u, fr.axis[c]));
         }
         else if (lane == 27) {
             float r[3];
             for (int k = 0; k < 3; k++)
                 r[k] = (float) (2.0*(sw[k] - floor(sw[k] + 0.5)));
-            for (int c = 0; c < 3; c++) {
-                float q = fabsf(pick(r, fr.axis[c]));
-                xi[c] = (_Float16) q;
-                if (ri)
-                    ri[c] = q;
-            }
+            for (int c = 0; c < 3; c++)
+                ri[c] = fabsf(pick(r, fr.axis[c]));
         }
         else if (lane == 28) {
             const double* v = velocities + 3*(size_t) part;
-            for (int c = 0; c < 3; c++) {
-                float r = (float) (fr.sign[c]*pick(v, fr.axis[c])/a.velocityScale);
-                float f = r*norm.vScale;
-                if (!(fabsf(f) <= norm.vBound))
-                    out = true;
-                xi[84 + c] = (_Float16) f;
-                if (ri)
-                    ri[84 + c] = r;
-            }
-        }
-        else {
             for (int c = 0; c < 3; c++)
-                xi[MLP_IN + 3*(lane - 29) + c] = (_Float16) 0.0f;
+                ri[84 + c] = (float) (fr.sign[c]*pick(v, fr.axis[c])/a.velocityScale);
         }
     }
-    // The 32 lanes of this particle are one half of the wave's ballot.
-    unsigned long long votes = __ballot(out);
-    unsigned mine = (unsigned) (votes >> (threadIdx.x & 32));
-    if (active && lane == 0)
-        ood[i] = mine != 0u ? 1 : 0;
 }
 
 /* u = j/rho of every fluid node (zero at solid nodes), FP64, [node][3]: one coalesced pass over the populations that
@@ -534,14 +496,13 @@ unsigned gridOf(int64_t items, int perBlock) {
     }
 
 void launchClosureFeatures(int storage, const void* src, const uint32_t* mask, const double* positions,
-        const double* velocities, const int* particles, const double* ucm, const ParticleArgs& a, const ClosureNorm& norm,
-        _Float16* X, float* raw, uint32_t* centreNode, double* centreVelocity, uint8_t* ood,
-        uint8_t* frame, hipStream_t stream) {
+        const double* velocities, const int* particles, const double* ucm, const ParticleArgs& a, float* raw,
+        double* centreVelocity, uint8_t* frame, hipStream_t stream) {
     if (a.numParticles == 0)
         return;
     unsigned grid = gridOf(a.numParticles, BLOCK/FEATURE_LANES);
     LBM_CLOSURE_STORAGE(storage, (closureFeatures<S><<<grid, BLOCK, 0, stream>>>((const S*) src, mask, positions,
-            velocities, particles, ucm, a, norm, X, raw, centreNode, centreVelocity, ood, frame)))
+            velocities, particles, ucm, a, raw, centreVelocity, frame)))
 }
 
 void launchClosureField(int storage, const void* src, const uint32_t* mask, const double* ucm, const ParticleArgs& a,

@@ -1237,16 +1237,12 @@ int lbm_closure_pairs(lbm_context* c, const double* positions, const double* vel
         ParticleArgs a = particleArgs(c, c->stepIndex, false);
         if (a.removal)
             reduceMoments(c);
-        ClosureNorm norm = {1.0f, 1.0f, 1.0f, 3.0e38f, 3.0e38f};
-        _Float16* X = deviceAlloc<_Float16>((size_t) n*MLP_IN_PAD);
         float* raw = deviceAlloc<float>((size_t) n*MLP_IN);
-        uint32_t* node = deviceAlloc<uint32_t>(n);
         double* u = deviceAlloc<double>(3*(size_t) n);
-        uint8_t* ood = deviceAlloc<uint8_t>(n);
         uint8_t* frame = deviceAlloc<uint8_t>(n);
         float* t = deviceAlloc<float>(3*(size_t) n);
-        launchClosureFeatures(c->p.storage, c->popA, c->mask, c->stagePos, c->stageVel, c->particles, c->ucm, a, norm, X,
-                raw, node, u, ood, frame, c->stream);
+        launchClosureFeatures(c->p.storage, c->popA, c->mask, c->stagePos, c->stageVel, c->particles, c->ucm, a, raw,
+                u, frame, c->stream);
         launchClosureTargets(c->p.storage, c->popA, c->mask, c->stagePos, c->particles, c->ucm, a, u, frame, t,
                 c->stream);
         hipError_t e = hipGetLastError();
@@ -1255,7 +1251,7 @@ int lbm_closure_pairs(lbm_context* c, const double* positions, const double* vel
         if (e == hipSuccess)
             e = hipMemcpyAsync(targets, t, 3*(size_t) n*sizeof(float), hipMemcpyDeviceToHost, c->stream);
         (void) hipStreamSynchronize(c->stream);
-        void* scratch[] = {X, raw, node, u, ood, frame, t};
+        void* scratch[] = {raw, u, frame, t};
         for (void* b : scratch)
             (void) hipFree(b);
         HIP_CHECK(e);

@@ -87,9 +87,8 @@ void launchMlpInfer(const MlpDevice* weights, const _Float16* X, int n, float ou
  *            (closureStepBlocks(n, field != nullptr) work-groups);
  *  fallback: the stencil coupling (a.stencil) of the flagged particles, wall momentum into closureFallbackBlocks(n)
  *            partials;
- *  features and targets, for training pairs: the raw FP32 inputs [n][87] (and the normalized FP16 ones [n][96]), the frame's
- *            code, the nearest node and its FP64 velocity; u_Keys - u(nearest) in the particle's frame (a.stencil must be
- *            Keys).
+ *  features and targets, for training pairs: the raw FP32 inputs [n][87], the frame's code and the FP64 velocity of the
+ *            nearest node; u_Keys - u(nearest) in the particle's frame (a.stencil must be Keys).
  */
 void launchClosureStep(int storage, const void* src, const uint32_t* mask, const double* positions,
         const double* velocities, const int* particles, const double* mass, const double* ucm, const ParticleArgs& a,
@@ -98,9 +97,8 @@ void launchClosureStep(int storage, const void* src, const uint32_t* mask, const
         hipStream_t stream);
 int closureStepBlocks(int numParticles, bool field);
 void launchClosureFeatures(int storage, const void* src, const uint32_t* mask, const double* positions,
-        const double* velocities, const int* particles, const double* ucm, const ParticleArgs& a, const ClosureNorm& norm,
-        _Float16* X, float* raw, uint32_t* centreNode, double* centreVelocity, uint8_t* ood,
-        uint8_t* frame, hipStream_t stream);
+        const double* velocities, const int* particles, const double* ucm, const ParticleArgs& a, float* raw,
+        double* centreVelocity, uint8_t* frame, hipStream_t stream);
 /* The node velocities u = j/rho of the whole lattice, FP64 [node][3] (zero at solid nodes), for
    launchClosureStep(field = ...) when 27 x particles exceed the nodes: one coalesced pass instead of 27 scattered
    pulls per particle.  The values are those the per-particle path forms, bit for bit. */
