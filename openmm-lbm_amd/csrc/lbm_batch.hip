@@ -244,10 +244,9 @@ void createBatch(lbm_batch* b, int R, const lbm_params* params, const int* numPa
     int particleBegin = 0;
     std::vector<uint16_t> particleReplica;
     std::vector<double> latticeMass, invMass;
-    uint64_t nodes = 0;
+    PaddingRoom room{0};
     for (int r = 0; r < R; r++)
-        nodes += (uint64_t) params[r].nx*params[r].ny*params[r].nz;
-    const double room = (double) spareBytes(reservedBytes(nodes));      // of all replicas' population arrays, two each
+        room.nodes += (uint64_t) params[r].nx*params[r].ny*params[r].nz;
     for (int r = 0; r < R; r++) {
         const lbm_params& p = params[r];
         ReplicaDesc& d = b->desc[r];
@@ -259,7 +258,7 @@ void createBatch(lbm_batch* b, int R, const lbm_params* params, const int* numPa
         g.nxy = (uint32_t) (p.nx*p.ny);
         g.n = (uint32_t) ((int64_t) p.nx*p.ny*p.nz);
         g.rowShift = 0;
-        const uint64_t popCount = layoutRows(g, sizeof(float), (uint64_t) (room/2*((double) g.n/(double) nodes)));
+        const uint64_t popCount = layoutRows(g, sizeof(float), room);
         g.openX = g.openY = g.openZ = 0;
         double cellMass = p.density*p.dx*p.dx*p.dx;
         uint32_t seed = (uint32_t) p.random_number_seed;

@@ -596,7 +596,8 @@ void create(const lbm_params* params, const int* solid, int numSolid, const int*
         c->g.rowShift--;
     if (n > (1ull << 30))
         throw Error(LBM_ERROR_INVALID, "LBMForce: the lattice is too large for one GPU: at most 2^30 nodes");
-    const uint64_t popBytes = layoutRows(c->g, c->elem, spareBytes(reservedBytes(n))/2)*c->elem;
+    PaddingRoom room{n};
+    const uint64_t popBytes = layoutRows(c->g, c->elem, room)*c->elem;
     // The fused pass addresses populations by 32-bit byte offsets while an array of them fits in 4 GiB (up to 56.5 M
     // nodes with FP32 storage), and by 64-bit indices beyond.  LBM_AMD_WIDE_ADDRESSING=1 takes the 64-bit path always.
     const char* wideEnv = getenv("LBM_AMD_WIDE_ADDRESSING");

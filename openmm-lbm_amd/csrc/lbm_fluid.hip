@@ -735,7 +735,7 @@ static FastDiv makeFastDiv(uint32_t d) {
     return f;
 }
 
-uint64_t layoutRows(Geometry& g, size_t elementSize, uint64_t maxPadded) {
+uint64_t layoutRows(Geometry& g, size_t elementSize, PaddingRoom& room) {
     g.divx = makeFastDiv(g.nx);
     g.divxy = makeFastDiv(g.nxy);
     g.divy = makeFastDiv(g.ny);
@@ -770,8 +770,8 @@ uint64_t layoutRows(Geometry& g, size_t elementSize, uint64_t maxPadded) {
     // No padding where rows are grouped in blocks, or where it would take an array that fits beyond the 4 GiB of the
     // 32-bit offsets.
     const uint64_t rows = (uint64_t) g.ny*g.nz, padded = NQ*rows*whole(shift)*elementSize;
-    g.padded = whole(shift) != g.nx && quarter(shift) && g.rowShift == 0 && padded <= maxPadded &&
-            (padded <= (1ull << 32) || NQ*rows*g.nx*elementSize > (1ull << 32)) ? 1 : 0;
+    g.padded = whole(shift) != g.nx && quarter(shift) && g.rowShift == 0 &&
+            (padded <= (1ull << 32) || NQ*rows*g.nx*elementSize > (1ull << 32)) && room.holds(padded, g.n) ? 1 : 0;
     g.qstride = (g.padded ? whole(shift) : g.nx) << g.rowShift;
     return NQ*rows*(g.qstride >> g.rowShift);
 }

@@ -235,9 +235,8 @@ inline uint64_t fusedThreads(const Geometry& g) {
     return ((uint64_t) g.ny*g.nz*g.chunksPerRow) << g.chunkShift;
 }
 /* The rows' chunks and the population layout (divisions, chunkShift, qstride, padded) of a lattice whose sizes and
-   rowShift are set; returns the elements of one population array.  maxPadded: the bytes that an array may take with padded
-   rows; where it would take more, the rows are not padded. */
-uint64_t layoutRows(Geometry& g, size_t elementSize, uint64_t maxPadded);
+   rowShift are set; returns the elements of one population array.  The rows are padded only where the room holds them. */
+uint64_t layoutRows(Geometry& g, size_t elementSize, PaddingRoom& room);
 void launchMomentReduce(int storage, bool solids, const void* src, const uint32_t* mask, const Geometry& g,
         double* partials, hipStream_t stream);
 void launchFinishReduce(const double* partials, double numFluid, double* totals, double* ucm, hipStream_t stream);

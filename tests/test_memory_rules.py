@@ -15,7 +15,7 @@ DEVICE = r"""
 #include <cstdio>
 #include <map>
 static std::map<void*, size_t> held;
-static size_t capacity = 0, used = 0, serial = 0, fragment = ~(size_t) 0;
+static size_t questions = 0, capacity = 0, used = 0, serial = 0, fragment = ~(size_t) 0;
 static hipError_t last = hipSuccess;
 extern "C" hipError_t hipMalloc(void** p, size_t n) {
     if (used + n > capacity || n > fragment)
@@ -38,6 +38,7 @@ extern "C" hipError_t hipGetLastError() {
     return e;
 }
 extern "C" hipError_t hipMemGetInfo(size_t* free, size_t* total) {
+    questions++;
     *free = capacity - used;
     *total = capacity;
     return hipSuccess;
@@ -101,6 +102,18 @@ def test_optional_memory_leaves_the_reserve(tmp_path):
     fragment = GB/4;                                       // no block larger than this
     CHECK(!lbm::allocateOptional({{&a, GB/8}, {&b, GB/2}}, 0) && !a && !b && used == 0);
     CHECK(hipGetLastError() == hipSuccess);
+""")
+
+
+def test_padded_rows_share_the_room(tmp_path):
+    """Two arrays for each lattice, by their shares of the nodes, in what stays free beside the reserve of all; small arrays
+    are tried without a question, and the device is asked once."""
+    run(tmp_path, r"""
+    capacity = 2*GB + 209*1000;
+    lbm::PaddingRoom room{1000};
+    CHECK(room.holds(lbm::SMALL_BYTES, 1) && questions == 0);
+    CHECK(room.holds(GB, 1000) && !room.holds(GB + 1, 1000) && room.holds(GB/4, 250) && !room.holds(GB/4 + 1, 250));
+    CHECK(questions == 1);
 """)
 
 
