@@ -153,15 +153,21 @@ int lbm_compute_lattice_parameters(const lbm_force_settings* settings, const dou
  * LBM_AMD_FUSED_ROWS=1 makes it stage its pulls through LDS where rows hold 128 or a multiple of 256 nodes (the same
  * results; slower on MI355X, so off by default).  Other switches that change the work, never the results (each run
  * is bit-identical across them): LBM_AMD_ROW_BLOCK=1|2|4 (lattice rows per block of the population layout, default
- * 1); and, for the explicit drag, LBM_AMD_SPREAD=atomic|tiles (the reaction spread), LBM_AMD_FIELD=0|1 (stencils read a
- * lattice-wide moment field) and LBM_AMD_STENCIL_SETUP=0|1 (each particle's stencil formed once), by default tiles,
- * field and setup for dense particles (stencil slots above a quarter of the nodes) and none of them otherwise, and
- * LBM_AMD_COUPLE_XCD=0|1 (with FP16/BF16 storage, each of the 8 XCDs couples a contiguous run of the particles in
+ * 1); LBM_AMD_SPREAD=atomic|tiles (the reaction spread of the explicit drag and of the centred one with a stencil; by
+ * default tiles on lattices with periodic faces whose particles have as many stencil slots as there are nodes, and
+ * 900,000); LBM_AMD_FIELD=0|1 (the stencils of either drag read a lattice-wide moment field; by default with the explicit
+ * drag where the slots outnumber a quarter of the nodes and are 400,000, with the centred one where they are half the nodes
+ * and 300,000); for the explicit drag LBM_AMD_STENCIL_SETUP=0|1 (each particle's stencil formed once; by default with the
+ * field) and LBM_AMD_COUPLE_XCD=0|1 (with FP16/BF16 storage, each of the 8 XCDs couples a contiguous run of the particles in
  * their processing order rather than every 8th work-group's; default 1); for the
  * centred drag with a stencil, LBM_AMD_CG_PLANNED=0 makes the host read the conjugate gradients' residual after every
- * iteration instead of after the previous solve's count of them (default 1), and LBM_AMD_CG_SPLIT=0|1 spreads every
- * slot in their products or only those at nodes several slots share (default: the latter for sparse particles; the
- * results agree to the solver's tolerance, not bit for bit).
+ * iteration instead of after the previous solve's count of them (default 1).  Two switches of that solve change its results
+ * within the solver's tolerance (1e-13 of the right-hand side), not bit for bit: LBM_AMD_CG_ROWS=0|1 forms the matrix by rows
+ * or spreads its products over the nodes (rows need periodic faces and 12 nodes or more per axis; default: rows there, for up
+ * to 4 M particles with at most 64 expected neighbours each), and LBM_AMD_CG_SPLIT=0|1 spreads every slot in those products
+ * or only those at nodes several slots share (default: the latter for sparse particles; given, it also turns the rows off
+ * unless LBM_AMD_CG_ROWS=1).  Memory that a lattice can do without (padded rows, field, bins, matrix rows) is taken only
+ * where the state and the fields still find theirs beside it.
  */
 int lbm_create(const lbm_params* params, const int* solid_nodes, int num_solid, const int* particles,
         const double* particle_masses, int num_particles, int num_system_particles, lbm_context** out);
@@ -248,8 +254,8 @@ int lbm_get_fluid_totals(lbm_context* ctx, double* mass, double momentum[3]);
 int lbm_synchronize(lbm_context* ctx);
 
 /*
- * Diagnostics with no counterpart in the reference: HIP-event timing of the fused lattice pass on the
- * context's stream.  Returns the total time (ms) and the number of passes recorded since the last call,
+ * Diagnostics with no counterpart in the reference: HIP-event timing of the fused lattice pass, alone, on the
+ * context's stream (device-resident particles take launches of their own while it is on).  Returns the total time (ms) and the number of passes recorded since the last call,
  * then switches recording on (enable = 1) or off (0).  The oracle library returns LBM_ERROR_UNSUPPORTED.
  */
 int lbm_profile_fused(lbm_context* ctx, int enable, double* total_ms, int* count);

@@ -122,7 +122,7 @@ struct lbm_context {
     // Particles.
     int numParticles = 0, numSystem = 0, numSlots = 0;
     bool identityParticles = false;       // coupled particle i is particle i of the System, and all are coupled
-    bool dense = false;                   // denseCoupling(): index order, component-plane reactions
+    bool dense = false;                   // denseCoupling(): the explicit drag keeps the index order, the centred one sorts
     bool wide = false;                    // 64-bit element indices in the fused pass (populations above 4 GiB)
     bool coupleXcd = true;                // LBM_AMD_COUPLE_XCD: the coupling's particles in XCD-contiguous runs
     int fusedPath = FUSED_DIRECT;         // the fused-pass kernel (FusedPath)

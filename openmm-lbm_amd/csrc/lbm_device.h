@@ -364,7 +364,8 @@ __device__ __forceinline__ double sqrtF64(double x) {
 }
 
 /*
- * -ln(n 2^-32) for a whole number n in [1, 2^32].  n 2^-32 = m 2^e with m in [sqrt(1/2), sqrt(2)), f = m - 1 (exact) and
+ * -ln(n 2^-32) for a whole number n in [1, 2^32], put together as fdlibm's published log does, with a series and a split of
+ * ln 2 of its own.  n 2^-32 = m 2^e with m in [sqrt(1/2), sqrt(2)), f = m - 1 (exact) and
  * s = f/(2 + f): ln m = 2 atanh(s) = f - s (f - R), R = 2 (s^2/3 + s^4/5 + ...); |s| < 0.172, so the terms to s^20 leave
  * 2e-18.  ln 2 is split into a part of 32 bits, whose product with e is exact, and the rest.
  */
@@ -618,10 +619,11 @@ struct Geometry {
 
 /*
  * Population layout.  The rows (j, k) of the lattice are grouped in blocks of R = 2^rowShift consecutive rows (r = j +
- * ny k; R divides ny); a block holds its 19 populations one after the other, each as R rows of nx values.  Population
- * q of node (i, j, k) is the element ((r >> rowShift)*19 + q)*R*nx + (r & (R - 1))*nx + i.  With R = 1 each row holds
- * its 19 populations in turn, q*nx + 19*node - 18*i.  A work-group of consecutive nodes then reads and writes a few
- * contiguous runs of R*nx values per population instead of 19 planes N values apart, which the HBM serves faster (on
+ * ny k; R divides ny); a block holds its 19 populations one after the other, each as R rows of s values.  With R = 1 a row
+ * may be padded to whole chunks of the lattice pass (layoutRows), s = qstride >= nx, and population q of node (i, j, k) is
+ * the element (r*19 + q)*s + i; with R > 1 there is no padding, s = nx = qstride >> rowShift, and it is
+ * ((r >> rowShift)*19 + q)*R*s + (r & (R - 1))*s + i.  A work-group of consecutive nodes then reads and writes a few
+ * contiguous runs of R*s values per population instead of 19 planes N values apart, which the HBM serves faster (on
  * 256^3 a bare pull measured 73% of the peak instead of 69%); larger R lengthens the runs for 2-byte storage.
  */
 
