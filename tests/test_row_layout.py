@@ -1,5 +1,7 @@
 """The rows of the population layout: the memory that a lattice takes, and every chunk that the lattice pass may take of its
 rows, padded and unpadded, with each storage type."""
+import gc
+
 import numpy as np
 import pytest
 import torch
@@ -19,6 +21,7 @@ ROWS = [1, 2, 3, 5, 8, 9, 12, 13, 16, 17, 24, 25, 26, 33, 40, 48, 50, 65, 100]
 
 
 def free_memory():
+    gc.collect()                                # what earlier tests left
     torch.cuda.synchronize()
     return torch.cuda.mem_get_info()[0]
 
